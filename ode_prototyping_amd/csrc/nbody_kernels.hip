@@ -7,19 +7,15 @@
 // atomic-free gather: a workgroup owns a tile of 64 target particles (one per
 // lane) and streams the partner particles j; partner coordinates are
 // wave-uniform, so they arrive through scalar loads into SGPRs and cost no
-// VGPR bandwidth or LDS (the 32-target exact kernel, whose half-waves take
-// different partners, uses vector loads instead).
+// VGPR bandwidth or LDS (the exact kernels for smaller grids have their own
+// layouts).
 //
 //  * exact:  the reference's FP64 expression (((dx^2 + dy^2) + dz^2) + eps^2,
 //            correctly rounded sqrt, den = dist * dist_sq, three correctly
 //            rounded divisions) and, per target, the partners summed in
 //            increasing j -- the order the single-threaded pair loop adds into
-//            acc[i].  Terms are computed by all sixteen waves of a workgroup in
-//            parallel and written to LDS; three waves then fold them in order
-//            (one coordinate each), double-buffered so folding tile t-1
-//            overlaps computing tile t.  Result: bit-identical to NBodyODE
-//            with SingleThreadedExecutor.  Must be compiled with
-//            -ffp-contract=off.
+//            acc[i] (nbody_exact.hpp).  Result: bit-identical to NBodyODE with
+//            SingleThreadedExecutor.  Must be compiled with -ffp-contract=off.
 //  * fast:   FP64, r^-3 from the hardware reciprocal square root with a
 //            third-order correction (a few ulp), FMA accumulation, the j range
 //            split over 16 waves per workgroup and the partial sums combined
@@ -99,373 +95,6 @@ __device__ inline double uniform_pow2_mass(const double* __restrict__ mass, int 
   return __syncthreads_and(ok) != 0 ? mass[0] : 0.0;
 }
 
-// ------------------------------------------------------------------ exact --
-constexpr int kExactWaves = 16;
-constexpr int kExactJW = 3;  // partners per wave per tile (48-partner tiles, 144 KB LDS)
-constexpr int kExactTJ = kExactWaves * kExactJW;
-
-// The kExactJW partners one wave evaluates in one tile (wave-uniform, held
-// in SGPRs).
-struct PartnerSet {
-  double x[kExactJW], y[kExactJW], z[kExactJW], m[kExactJW];
-};
-
-// Partners jb .. jb + kExactJW - 1, all < n.
-template <bool kMass>
-__device__ __forceinline__ void load_partner_set(PartnerSet& p, uniform_ptr yu,
-                                                 uniform_ptr massu, int jb) {
-  const uniform_ptr pp = yu + 3 * jb;
-#pragma unroll
-  for (int jj = 0; jj < kExactJW; ++jj) {
-    p.x[jj] = pp[3 * jj];
-    p.y[jj] = pp[3 * jj + 1];
-    p.z[jj] = pp[3 * jj + 2];
-    p.m[jj] = kMass ? massu[jb + jj] : 1.0;
-  }
-}
-
-// The same with indices past the end clamped to n - 1: their terms are
-// computed but never folded.
-template <bool kMass>
-__device__ __forceinline__ void load_partner_set_clamped(PartnerSet& p, uniform_ptr yu,
-                                                         uniform_ptr massu, int jb, int n) {
-  if (jb + kExactJW <= n) {
-    load_partner_set<kMass>(p, yu, massu, jb);
-    return;
-  }
-#pragma unroll
-  for (int jj = 0; jj < kExactJW; ++jj) {
-    const int j = min(jb + jj, n - 1);
-    p.x[jj] = yu[3 * j];
-    p.y[jj] = yu[3 * j + 1];
-    p.z[jj] = yu[3 * j + 2];
-    p.m[jj] = kMass ? massu[j] : 1.0;
-  }
-}
-
-// This wave's kExactJW terms of one tile for its 64 targets, stored to
-// dst[jj][coordinate][lane].
-template <bool kMass, bool kShared>
-__device__ __forceinline__ void exact_tile_terms(const PartnerSet& p, double xi, double yi,
-                                                 double zi, double softening_sq,
-                                                 double (*dst)[3][64], int lane) {
-  double ax[kExactJW], ay[kExactJW], az[kExactJW];
-#pragma unroll
-  for (int jj = 0; jj < kExactJW; ++jj) {
-    const double dx = p.x[jj] - xi, dy = p.y[jj] - yi, dz = p.z[jj] - zi;
-    if (kShared)
-      exact_term_shared_rcp<kMass>(dx, dy, dz, p.m[jj], softening_sq, ax[jj], ay[jj], az[jj]);
-    else
-      exact_term_ieee<kMass>(dx, dy, dz, p.m[jj], softening_sq, ax[jj], ay[jj], az[jj]);
-  }
-#pragma unroll
-  for (int jj = 0; jj < kExactJW; ++jj) {
-    dst[jj][0][lane] = ax[jj];
-    dst[jj][1][lane] = ay[jj];
-    dst[jj][2][lane] = az[jj];
-  }
-}
-
-// Adds the terms of partners base .. base + cnt - 1 (one coordinate; src
-// points at partner 0's entry for this lane) to acc in partner order,
-// skipping the target's own index.  The skip adds +0 instead of the term:
-// acc starts at +0 and a round-to-nearest sum is -0 only if both operands
-// are, so acc is never -0 and acc + +0 is acc bit for bit -- no per-lane
-// branch.
-__device__ __forceinline__ double exact_fold(double acc, const double* src, int base, int cnt,
-                                             int i0, int i) {
-  if (cnt == kExactTJ && (base + kExactTJ <= i0 || base >= i0 + 64)) {
-#pragma unroll
-    for (int m = 0; m < kExactTJ; ++m) acc += src[m * 192];
-  } else {
-    for (int m = 0; m < cnt; ++m) {
-      const double v = src[m * 192];
-      acc += base + m != i ? v : 0.0;
-    }
-  }
-  return acc;
-}
-
-// All tiles of one workgroup; returns the folded sum of the calling lane
-// (waves 0-2: coordinate = wave).  Partner data is loaded one tile ahead
-// (scalar loads hidden behind the current tile's arithmetic).  Tiles whose
-// partners and next partners are all in range run in a loop unrolled by two
-// over two partner sets, with no bounds tests and no register copies: the
-// scalar instructions per tile stay few, since the scalar unit is shared by
-// the 16 waves that all leave the same barrier together.
-template <bool kMass, bool kShared>
-__device__ __forceinline__ double exact_tiles(double (*terms)[kExactTJ][3][64], uniform_ptr yu,
-                                              uniform_ptr massu, int n, double softening_sq,
-                                              double xi, double yi, double zi, int wave, int lane,
-                                              int i0, int i) {
-  const int n_tiles = (n + kExactTJ - 1) / kExactTJ;
-  const int n_full = n / kExactTJ;
-  const int jw = wave * kExactJW;
-  double acc = 0.0;
-  PartnerSet pa, pb;
-  // tile 0: nothing to fold yet
-  load_partner_set_clamped<kMass>(pa, yu, massu, jw, n);
-  if (n_tiles > 1) load_partner_set_clamped<kMass>(pb, yu, massu, kExactTJ + jw, n);
-  exact_tile_terms<kMass, kShared>(pa, xi, yi, zi, softening_sq, terms[0] + jw, lane);
-  __syncthreads();
-  int t = 1;
-  // Steady state: tiles t - 1 .. t + 2 are all full; tile t's partners are
-  // in pb.  Tile t is odd, so its terms go to buffer 1 and tile t + 1's to
-  // buffer 0.
-  for (; t + 2 < n_full; t += 2) {
-    if (wave < 3) acc = exact_fold(acc, &terms[0][0][wave][lane], (t - 1) * kExactTJ,
-                                   kExactTJ, i0, i);
-    load_partner_set<kMass>(pa, yu, massu, (t + 1) * kExactTJ + jw);
-    exact_tile_terms<kMass, kShared>(pb, xi, yi, zi, softening_sq, terms[1] + jw, lane);
-    __syncthreads();
-    if (wave < 3) acc = exact_fold(acc, &terms[1][0][wave][lane], t * kExactTJ, kExactTJ,
-                                   i0, i);
-    load_partner_set<kMass>(pb, yu, massu, (t + 2) * kExactTJ + jw);
-    exact_tile_terms<kMass, kShared>(pa, xi, yi, zi, softening_sq, terms[0] + jw, lane);
-    __syncthreads();
-  }
-  // The remaining tiles (partial last tile included), then the last fold.
-  for (; t <= n_tiles; ++t) {
-    if (wave < 3) {
-      const int base = (t - 1) * kExactTJ;
-      acc = exact_fold(acc, &terms[(t - 1) & 1][0][wave][lane], base, min(kExactTJ, n - base),
-                       i0, i);
-    }
-    if (t < n_tiles) {
-      pa = pb;
-      if (t + 1 < n_tiles)
-        load_partner_set_clamped<kMass>(pb, yu, massu, (t + 1) * kExactTJ + jw, n);
-      exact_tile_terms<kMass, kShared>(pa, xi, yi, zi, softening_sq, terms[t & 1] + jw, lane);
-    }
-    __syncthreads();
-  }
-  return acc;
-}
-
-template <bool kMass, bool kSharedRcp>
-__global__ __launch_bounds__(64 * kExactWaves) void k_nbody_exact(NBodyArgs a) {
-  if (prologue_skip(a)) return;
-  __shared__ double terms[2][kExactTJ][3][64];
-  const double* __restrict__ y = select_input(a);
-  const uniform_ptr yu = as_uniform(y);
-  double* __restrict__ k = a.k;
-  const uniform_ptr massu = as_uniform(a.mass);
-  const int n = a.n;
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int i0 = blockIdx.x * 64;
-  const int i = i0 + lane;
-  const bool valid_i = i < n;
-  const double xi = valid_i ? y[3 * i] : 0.0;
-  const double yi = valid_i ? y[3 * i + 1] : 0.0;
-  const double zi = valid_i ? y[3 * i + 2] : 0.0;
-  // the shared-reciprocal form is used when every position coordinate passes
-  // coord_shared_ok (one pass over the 3N coordinates per workgroup); with
-  // masses that are all one power of two, unit-mass terms and one scale of the
-  // sum (uniform_pow2_mass)
-  const bool shared_ok = kSharedRcp && all_positions_shared_ok(y, n);
-  const double m_uni = kMass && kSharedRcp && shared_ok ? uniform_pow2_mass(a.mass, n) : 0.0;
-  double acc;
-  if (kSharedRcp && shared_ok && kMass && m_uni != 0.0)
-    acc = exact_tiles<false, true>(terms, yu, massu, n, a.eps2, xi, yi, zi, wave, lane, i0, i) *
-          m_uni;
-  else if (kSharedRcp && shared_ok)
-    acc = exact_tiles<kMass, true>(terms, yu, massu, n, a.eps2, xi, yi, zi, wave, lane, i0, i);
-  else
-    acc = exact_tiles<kMass, false>(terms, yu, massu, n, a.eps2, xi, yi, zi, wave, lane, i0, i);
-  if (wave < 3 && valid_i) k[3L * n + 3 * i + wave] = acc;
-  copy_velocities(y, k, n, i0);
-}
-
-// The same exact sum with 32-target tiles: twice the workgroups, for N too
-// small to fill the chip with 64-target tiles.  Lane l evaluates target l % 32
-// against the kE32JW partners of slot l / 32 of its wave; each lane fetches
-// its slot's partners with vector loads (the two half-waves read different
-// addresses, one tile ahead), so no per-lane selection between wave-uniform
-// values is needed.  Two waves fold a tile's terms in partner order: wave 0
-// the x (lanes 0-31) and y (lanes 32-63) chains, wave 1 the z chains.  W waves
-// per workgroup: a tile has 6 W partners and the two term buffers take
-// 2 x 6W x 3 x 32 doubles (144 KB at W = 16: one workgroup per CU; 72 KB at
-// W = 8: two).
-constexpr int kE32JW = 3;  // partners per slot per tile
-// The launcher takes the instance with the power-of-two mass path from this
-// many bodies on.  Below, the second tile loop (and the register spill and
-// scratch set-up it brings) costs more per launch than the 3 products per
-// interaction it saves: 64-body solves ran 3-11 % slower with it.
-constexpr int kE32UniformMassMinN = 4096;
-template <int W>
-constexpr int e32_tj = 2 * kE32JW * W;  // partners per tile
-
-// This lane's kE32JW partners (x, y, z, m), starting at index jb.
-typedef double E32Partners[kE32JW][4];
-
-// Partners jb .. jb + kE32JW - 1, all < n.
-template <bool kMass>
-__device__ __forceinline__ void e32_load(E32Partners& q, const double* __restrict__ y,
-                                         const double* __restrict__ mass, int jb) {
-#pragma unroll
-  for (int jj = 0; jj < kE32JW; ++jj) {
-    q[jj][0] = y[3 * (jb + jj)];
-    q[jj][1] = y[3 * (jb + jj) + 1];
-    q[jj][2] = y[3 * (jb + jj) + 2];
-    q[jj][3] = kMass ? mass[jb + jj] : 1.0;
-  }
-}
-
-// The same with indices past the end clamped to n - 1 (their terms are
-// computed but never folded).
-template <bool kMass>
-__device__ __forceinline__ void e32_load_clamped(E32Partners& q, const double* __restrict__ y,
-                                                 const double* __restrict__ mass, int jb,
-                                                 int n) {
-#pragma unroll
-  for (int jj = 0; jj < kE32JW; ++jj) {
-    const int j = min(jb + jj, n - 1);
-    q[jj][0] = y[3 * j];
-    q[jj][1] = y[3 * j + 1];
-    q[jj][2] = y[3 * j + 2];
-    q[jj][3] = kMass ? mass[j] : 1.0;
-  }
-}
-
-// This lane's terms of one tile, stored to dst[m0 + jj][coordinate][tgt].
-template <bool kMass, bool kShared>
-__device__ __forceinline__ void e32_terms(const E32Partners& q, double xi, double yi, double zi,
-                                          double softening_sq, double (*dst)[3][32], int m0,
-                                          int tgt) {
-  double ax[kE32JW], ay[kE32JW], az[kE32JW];
-#pragma unroll
-  for (int jj = 0; jj < kE32JW; ++jj) {
-    const double dx = q[jj][0] - xi, dy = q[jj][1] - yi, dz = q[jj][2] - zi;
-    if (kShared)
-      exact_term_shared_rcp<kMass>(dx, dy, dz, q[jj][3], softening_sq, ax[jj], ay[jj], az[jj]);
-    else
-      exact_term_ieee<kMass>(dx, dy, dz, q[jj][3], softening_sq, ax[jj], ay[jj], az[jj]);
-  }
-#pragma unroll
-  for (int jj = 0; jj < kE32JW; ++jj) {
-    dst[m0 + jj][0][tgt] = ax[jj];
-    dst[m0 + jj][1][tgt] = ay[jj];
-    dst[m0 + jj][2][tgt] = az[jj];
-  }
-}
-
-// exact_fold for the 32-target layout (partner stride 96 doubles).
-template <int W>
-__device__ __forceinline__ double e32_fold(double acc, const double* src, int base, int cnt,
-                                           int i0, int i) {
-  constexpr int TJ = e32_tj<W>;
-  if (cnt == TJ && (base + TJ <= i0 || base >= i0 + 32)) {
-#pragma unroll
-    for (int m = 0; m < TJ; ++m) acc += src[m * 96];
-  } else {
-    for (int m = 0; m < cnt; ++m) {
-      const double v = src[m * 96];
-      acc += base + m != i ? v : 0.0;
-    }
-  }
-  return acc;
-}
-
-// All tiles of one workgroup (the structure of exact_tiles: peeled first
-// tile, a two-tile steady-state loop over two register partner sets with no
-// bounds tests, then the remaining tiles).  Returns the folded sum of the
-// calling lane (meaningful on the folding lanes).
-template <bool kMass, bool kShared, int W>
-__device__ __forceinline__ double e32_tiles(double (*terms)[e32_tj<W>][3][32],
-                                            const double* __restrict__ y,
-                                            const double* __restrict__ mass, int n,
-                                            double softening_sq, double xi, double yi, double zi,
-                                            int wave, int slot, int tgt, int i0, int i, int fc) {
-  constexpr int kE32TJ = e32_tj<W>;
-  const int n_tiles = (n + kE32TJ - 1) / kE32TJ;
-  const int n_full = n / kE32TJ;
-  const int m0 = 2 * kE32JW * wave + slot * kE32JW;  // this lane's first partner in a tile
-  double acc = 0.0;
-  E32Partners qa, qb;
-  e32_load_clamped<kMass>(qa, y, mass, m0, n);
-  if (n_tiles > 1) e32_load_clamped<kMass>(qb, y, mass, kE32TJ + m0, n);
-  e32_terms<kMass, kShared>(qa, xi, yi, zi, softening_sq, terms[0], m0, tgt);
-  __syncthreads();
-  int t = 1;
-  for (; t + 2 < n_full; t += 2) {
-    if (wave < 2)
-      acc = e32_fold<W>(acc, &terms[0][0][fc][tgt], (t - 1) * kE32TJ, kE32TJ, i0, i);
-    e32_load<kMass>(qa, y, mass, (t + 1) * kE32TJ + m0);
-    e32_terms<kMass, kShared>(qb, xi, yi, zi, softening_sq, terms[1], m0, tgt);
-    __syncthreads();
-    if (wave < 2) acc = e32_fold<W>(acc, &terms[1][0][fc][tgt], t * kE32TJ, kE32TJ, i0, i);
-    e32_load<kMass>(qb, y, mass, (t + 2) * kE32TJ + m0);
-    e32_terms<kMass, kShared>(qa, xi, yi, zi, softening_sq, terms[0], m0, tgt);
-    __syncthreads();
-  }
-  for (; t <= n_tiles; ++t) {
-    if (wave < 2) {
-      const int base = (t - 1) * kE32TJ;
-      acc = e32_fold<W>(acc, &terms[(t - 1) & 1][0][fc][tgt], base, min(kE32TJ, n - base), i0,
-                        i);
-    }
-    if (t < n_tiles) {
-      E32Partners qc;
-#pragma unroll
-      for (int jj = 0; jj < kE32JW; ++jj)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) qc[jj][c] = qb[jj][c];
-      if (t + 1 < n_tiles) e32_load_clamped<kMass>(qb, y, mass, (t + 1) * kE32TJ + m0, n);
-      e32_terms<kMass, kShared>(qc, xi, yi, zi, softening_sq, terms[t & 1], m0, tgt);
-    }
-    __syncthreads();
-  }
-  return acc;
-}
-
-// At W = 8 two workgroups share a CU: 4 waves per SIMD, <= 128 VGPRs each.
-// kUniMass: the power-of-two mass path (with kMass and kSharedRcp).
-template <bool kMass, bool kSharedRcp, int W, bool kUniMass>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4)))
-void k_nbody_exact32(NBodyArgs a) {
-  if (prologue_skip(a)) return;
-  __shared__ double terms[2][e32_tj<W>][3][32];
-  const double* __restrict__ y = select_input(a);
-  double* __restrict__ k = a.k;
-  const double* __restrict__ mass = a.mass;
-  const int n = a.n;
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int tgt = lane & 31;
-  const int slot = lane >> 5;
-  const int i0 = blockIdx.x * 32;
-  const int i = i0 + tgt;
-  const int ic = i < n ? i : n - 1;
-  const double xi = y[3 * ic], yi = y[3 * ic + 1], zi = y[3 * ic + 2];
-  // fold role: wave 0 lanes 0-31 -> x, 32-63 -> y; wave 1 lanes 0-31 -> z
-  // (wave 1 lanes 32-63 repeat the z fold and discard it)
-  const int fc = wave == 0 ? slot : 2;
-  const bool folds = (wave == 0) || (wave == 1 && slot == 0);
-  const bool shared_ok = kSharedRcp && all_positions_shared_ok(y, n);
-  // masses that are all one power of two: unit-mass terms and one exact scale
-  // of each finished sum (uniform_pow2_mass), as in k_nbody_exact
-  double m_uni = 0.0;
-  if constexpr (kUniMass && kMass && kSharedRcp)
-    m_uni = shared_ok ? uniform_pow2_mass(mass, n) : 0.0;
-  double acc;
-  if (kUniMass && kMass && kSharedRcp && shared_ok && m_uni != 0.0)
-    acc = e32_tiles<false, true, W>(terms, y, mass, n, a.eps2, xi, yi, zi, wave, slot, tgt, i0,
-                                    i, fc) *
-          m_uni;
-  else if (kSharedRcp && shared_ok)
-    acc = e32_tiles<kMass, true, W>(terms, y, mass, n, a.eps2, xi, yi, zi, wave, slot, tgt, i0,
-                                    i, fc);
-  else
-    acc = e32_tiles<kMass, false, W>(terms, y, mass, n, a.eps2, xi, yi, zi, wave, slot, tgt, i0,
-                                     i, fc);
-  if (folds && i < n) k[3L * n + 3 * i + fc] = acc;
-  // dxdt[0:3n] = x[3n:6n] for this tile's 32 particles
-  const int e = threadIdx.x;
-  const long base = 3L * i0, lim = 3L * n;
-  if (e < 96 && base + e < lim) k[base + e] = y[lim + base + e];
-}
-
 // ------------------------------------------------------------------- fast --
 constexpr int kFastWaves = 16;
 
@@ -510,6 +139,14 @@ __device__ __forceinline__ void scalar_loads_drain() {
   __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0); vector and export counters untouched
   __builtin_amdgcn_sched_barrier(0);
 }
+
+}  // namespace
+}  // namespace odehip
+
+#include "nbody_exact.hpp"
+
+namespace odehip {
+namespace {
 
 // Partners jbeg .. jend - 1 of target i in increasing j (wave-uniform scalar
 // loads); kMass: per-term masses.  kPrefetch: full sets of kFastSet partners
@@ -828,47 +465,7 @@ hipError_t launch_nbody_rhs(const NBodyArgs& a, int variant, hipStream_t s) {
   const bool guard = !(a.eps2 >= 1e-150);
   switch (variant) {
     case ODEHIP_NBODY_EXACT: {
-      // the shared-reciprocal form needs softening^2 in [2^-200, 2^100]
-      const bool shared = a.eps2 >= 0x1p-200 && a.eps2 <= 0x1p100;
-      // Both tile shapes sum every target's partners in the same order and
-      // hold one workgroup per CU (144 KB LDS each), so a launch takes
-      // ceil(workgroups / CUs) rounds.  A round of the 32-target kernel costs
-      // 0.62 of a 64-target one (MI355X sweep, N = 16384 ... 65536), so it
-      // wins while it needs at most as many rounds (N <= 8192 on 256 CUs) and
-      // where the 64-target grid's last round is half empty (e.g. N = 24576).
-      const long cus = device_cus();
-      const long r64 = ((a.n + 63) / 64 + cus - 1) / cus;
-      const long r32 = ((a.n + 31) / 32 + cus - 1) / cus;
-      if (0.62 * static_cast<double>(r32) < static_cast<double>(r64)) {
-        const unsigned b32 = static_cast<unsigned>((a.n + 31) / 32);
-        const dim3 th(64 * 16);
-        const bool uni = a.n >= kE32UniformMassMinN;
-        if (mass) {
-          if (shared && uni)
-            hipLaunchKernelGGL((k_nbody_exact32<true, true, 16, true>), dim3(b32), th, 0, s, a);
-          else if (shared)
-            hipLaunchKernelGGL((k_nbody_exact32<true, true, 16, false>), dim3(b32), th, 0, s, a);
-          else
-            hipLaunchKernelGGL((k_nbody_exact32<true, false, 16, false>), dim3(b32), th, 0, s, a);
-        } else {
-          if (shared)
-            hipLaunchKernelGGL((k_nbody_exact32<false, true, 16, false>), dim3(b32), th, 0, s, a);
-          else
-            hipLaunchKernelGGL((k_nbody_exact32<false, false, 16, false>), dim3(b32), th, 0, s, a);
-        }
-        break;
-      }
-      if (mass) {
-        if (shared)
-          hipLaunchKernelGGL((k_nbody_exact<true, true>), dim3(blocks), dim3(64 * kExactWaves), 0, s, a);
-        else
-          hipLaunchKernelGGL((k_nbody_exact<true, false>), dim3(blocks), dim3(64 * kExactWaves), 0, s, a);
-      } else {
-        if (shared)
-          hipLaunchKernelGGL((k_nbody_exact<false, true>), dim3(blocks), dim3(64 * kExactWaves), 0, s, a);
-        else
-          hipLaunchKernelGGL((k_nbody_exact<false, false>), dim3(blocks), dim3(64 * kExactWaves), 0, s, a);
-      }
+      launch_exact(a, device_cus(), s);
       break;
     }
     case ODEHIP_NBODY_FAST: {

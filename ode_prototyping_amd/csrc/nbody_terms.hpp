@@ -37,13 +37,24 @@ __device__ inline void exact_term_ieee(double dx, double dy, double dz,
 //    r = 1/2 - h g; g += g r; h += h r; twice g += (s - g^2) h); the rescale
 //    is the identity for s >= 2^-767, so the refinement alone gives the same
 //    bits.
-//  * division: the hardware sequence for n/d is d' = div_scale(d), r =
-//    rcp(d') refined by two Newton steps, q0 = n' r, rem = n' - d' q0,
-//    q = div_fmas(rem, r, q0), div_fixup.  With n and d in the range above
-//    div_scale leaves both operands unscaled (no VCC), div_fmas is a plain
-//    fma and div_fixup returns q unchanged -- so the refined reciprocal
-//    depends on d only and the three divisions by the same denominator share
-//    it: 1 rcp + 4 fma, then 3 ops per numerator instead of 11.
+//  * division: q = q0 + (n - d q0) r with q0 = n r and r = 1/d to within
+//    (1/2 + 2^-35) ulp is n/d correctly rounded: the residual is exact, so the
+//    sum before the last rounding is off by less than the distance of any
+//    quotient of two doubles from a rounding boundary (Markstein, IBM J. Res.
+//    Dev. 34 (1990), theorem 2).  The margin vanishes only where d's
+//    significand is 2 - u 2^-52 with an odd u < 2^10, whose reciprocal is
+//    within 2^-34 ulp of a tie: there r has to be the nearer double, and is
+//    not for some; at most a few numerators for each such d (fewer than 2^11
+//    of the 2^104 pairs of significands) then round the other way, as they do
+//    in the hardware's own sequence for the smallest u
+//    (tests/test_shared_reciprocal.py enumerates them).  r depends on d only,
+//    so the three divisions share it: 3 ops per numerator instead of 11.
+//  * reciprocal: d = s sqrt(s), so after the square root 2 h is 1/sqrt(s) to
+//    about 2^-46 and (2 h)^3 is 1/d to 2^-44; one Newton step squares that
+//    error, far below the rounding of r.  Three instructions in the place of
+//    v_rcp_f64 (four times the cost of one) and a Newton step: 33 full-rate
+//    instructions and one transcendental per term instead of 32 and two,
+//    about 7 % of the arithmetic, with the same bits.
 template <bool kMass>
 __device__ inline void exact_term_shared_rcp(double dx, double dy, double dz,
                                              double mj, double softening_sq,
@@ -61,10 +72,9 @@ __device__ inline void exact_term_shared_rcp(double dx, double dy, double dz,
   d = __builtin_fma(-g, g, dist_sq);
   const double dist = __builtin_fma(d, h, g);
   const double den = dist * dist_sq;
-  double r = __builtin_amdgcn_rcp(den);
-  double e = __builtin_fma(-den, r, 1.0);
-  r = __builtin_fma(r, e, r);
-  e = __builtin_fma(-den, r, 1.0);
+  const double y1 = h + h;
+  double r = (y1 * y1) * y1;
+  const double e = __builtin_fma(-den, r, 1.0);
   r = __builtin_fma(r, e, r);
   const double qx = dx * r, qy = dy * r, qz = dz * r;
   ax = __builtin_fma(__builtin_fma(-den, qx, dx), r, qx);
@@ -75,6 +85,17 @@ __device__ inline void exact_term_shared_rcp(double dx, double dy, double dz,
     ay *= mj;
     az *= mj;
   }
+}
+
+// The exact term in the form the caller established as valid.
+template <bool kMass, bool kShared>
+__device__ __forceinline__ void exact_term(double dx, double dy, double dz, double mj,
+                                           double softening_sq, double& ax, double& ay,
+                                           double& az) {
+  if constexpr (kShared)
+    exact_term_shared_rcp<kMass>(dx, dy, dz, mj, softening_sq, ax, ay, az);
+  else
+    exact_term_ieee<kMass>(dx, dy, dz, mj, softening_sq, ax, ay, az);
 }
 
 // Coordinates for which the shared-reciprocal term, summed into a target's
