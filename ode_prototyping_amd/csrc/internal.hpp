@@ -79,9 +79,11 @@ hipError_t launch_probe_fp64(double* out, long long* clk, int blocks, int iters,
                              hipStream_t s);
 hipError_t launch_momentum_terms(const double* x, int n, const double* mass,
                                  double* out, hipStream_t s);
-hipError_t launch_nbody_energy(const double* x, int n, double eps2,
-                               const double* mass, double* per_particle,
-                               hipStream_t s);
+// Kinetic and potential energy into out[0], out[1]; scratch holds
+// nbody_energy_scratch(n) doubles.
+size_t nbody_energy_scratch(int n);
+hipError_t launch_nbody_energy(const double* x, int n, double eps2, const double* mass,
+                               double* scratch, double* out, hipStream_t s);
 
 // ---- tableaux (built in, or registered at run time; odehip_abi.hip) ----
 bool valid_tableau(int id);

@@ -826,17 +826,14 @@ int odehip_nbody_energy(odehip_context* ctx, const double* x, size_t n,
   ODEHIP_USE_DEVICE(ctx);
   if (!ctx || !x || !host_out) return fail(ctx, ODEHIP_ERR_INVALID, "null argument");
   if (n == 0) return fail(ctx, ODEHIP_ERR_INVALID, "n is 0");
-  const size_t ng = static_cast<size_t>(n_groups_for(n));
-  int rc = ensure_scratch(ctx, 2 * n + 2 * (ng + 1) + 8);
+  const size_t need = nbody_energy_scratch(static_cast<int>(n));
+  int rc = ensure_scratch(ctx, need + 2);
   if (rc) return rc;
-  double* per = ctx->scratch;
-  double* sums = ctx->scratch + 2 * n;
-  HIP_TRY(ctx, launch_nbody_energy(x, static_cast<int>(n), softening * softening,
-                                   masses, per, ctx->stream));
-  HIP_TRY(ctx, launch_sum_tree(per, n, sums, ctx->stream));
-  HIP_TRY(ctx, launch_sum_tree(per + n, n, sums + ng + 1, ctx->stream));
-  HIP_TRY(ctx, hipMemcpyAsync(ctx->h_scalar, sums, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  HIP_TRY(ctx, hipMemcpyAsync(ctx->h_scalar + 1, sums + ng + 1, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+  double* sums = ctx->scratch + need;
+  HIP_TRY(ctx, launch_nbody_energy(x, static_cast<int>(n), softening * softening, masses,
+                                   ctx->scratch, sums, ctx->stream));
+  HIP_TRY(ctx, hipMemcpyAsync(ctx->h_scalar, sums, 2 * sizeof(double), hipMemcpyDeviceToHost,
+                              ctx->stream));
   HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
   host_out[0] = ctx->h_scalar[0];
   host_out[1] = ctx->h_scalar[1];
