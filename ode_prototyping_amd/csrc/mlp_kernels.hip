@@ -3,11 +3,10 @@
 // with the odehip_mlp_* C ABI (declarations in odehip.h).
 //
 // Training: a mini-batch is split over workgroups of 256 threads; each
-// workgroup streams its samples through LDS in chunks of 64, runs the
-// forward and backward pass for the chunk as small LDS-resident matrix
-// products, and keeps its share of the weight gradient in registers; the
-// per-workgroup partial gradients are then summed in a fixed order by the
-// Adam kernel (the run is deterministic).  Samples are visited in the order
+// workgroup takes its samples in chunks of 64, runs the forward and backward
+// pass for the chunk as FP32 matrix-core products, and keeps its share of the
+// weight gradient in registers; the per-workgroup partial gradients are then
+// summed in a fixed order by the Adam kernel (the run is deterministic).  Samples are visited in the order
 // of an affine permutation i -> (a i + c) mod n per epoch.
 #include <algorithm>
 #include <cmath>
@@ -60,185 +59,245 @@ struct GradArgs {
   float* loss_part;
 };
 
+// One chunk is 64 samples; wave w computes the samples 16 w .. 16 w + 15
+// forward and back, and rows 16 w .. of the weight gradients over all 64.  The
+// five products run on v_mfma_f32_16x16x4_f32 (FP32 operands, products and
+// sums); lane l holds A[l % 16][l / 16], B[l / 16][l % 16] and D[4 (l / 16) +
+// i][l % 16].  220 of them per wave and chunk, 3 us; as LDS-fed multiply-adds,
+// one LDS read each, a chunk took 36 us, and 4096 samples ran on 16 workgroups
+// of 4 chunks (145 us a batch, now 7).
+// Row strides: 72 floats keep the operand reads along rows and along columns
+// at two lanes per bank.
+constexpr int kRow = 72;
+
+struct GradLds {
+  float w2[kMlpHid][kRow];
+  float h1[kChunk][kRow];
+  float d2[kChunk][kRow];
+  float d1[kChunk][kRow];
+  float xs[kChunk][20];  // normalised inputs, columns 10 .. 15 zero
+  float tgt[kChunk];
+  long idx[kChunk];  // -1: past the end
+  float red[4][3][kMlpHid];
+  float red1[4][2];
+};
+
+__device__ __forceinline__ mlp_float4 mfma4(float a, float b, mlp_float4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
 __global__ __launch_bounds__(kGradThreads) void k_mlp_grad(GradArgs g) {
-  __shared__ float sw[kMlpParams + 3];
-  __shared__ float xs[kChunk][kMlpIn + 1];
-  __shared__ float h1[kChunk][kMlpHid + 1];
-  __shared__ float h2[kChunk][kMlpHid + 1];
-  __shared__ float d2[kChunk][kMlpHid + 1];
-  __shared__ float d1[kChunk][kMlpHid + 1];
-  __shared__ float dy[kChunk];
-  __shared__ float tgt[kChunk];
-  __shared__ int vld[kChunk];
-  __shared__ float red[kGradThreads];
-  const int tid = threadIdx.x;
-  for (int p = tid; p < kMlpParams; p += kGradThreads) sw[p] = g.w[p];
-  float aw2[16], aw1[3], ab = 0.0f, loss = 0.0f;
+  __shared__ GradLds L;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, kq = lane >> 4;
+  for (int e = tid; e < kMlpHid * kMlpHid; e += kGradThreads)
+    L.w2[e / kMlpHid][e % kMlpHid] = g.w[kMlpOffW2 + e];
+  float w1f[4][3], b1[4], b2[4], w3[4];
 #pragma unroll
-  for (int q = 0; q < 16; ++q) aw2[q] = 0.0f;
+  for (int nb = 0; nb < 4; ++nb) {
+    const int u = 16 * nb + r;
 #pragma unroll
-  for (int q = 0; q < 3; ++q) aw1[q] = 0.0f;
-  const int per = (g.count + gridDim.x - 1) / gridDim.x;
+    for (int ks = 0; ks < 3; ++ks) {
+      const int i = 4 * ks + kq;
+      w1f[nb][ks] = i < kMlpIn ? g.w[kMlpOffW1 + u * kMlpIn + i] : 0.0f;
+    }
+    b1[nb] = g.w[kMlpOffB1 + u];
+    b2[nb] = g.w[kMlpOffB2 + u];
+    w3[nb] = g.w[kMlpOffW3 + u];
+  }
+  const float b3 = g.w[kMlpOffB3];
+  const mlp_float4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  // this wave's rows of the gradients: W2 (4 column tiles), W1; and its
+  // samples' share of b1, b2, w3 (column 16 nb + r), b3 and the loss
+  mlp_float4 gw2[4] = {zero, zero, zero, zero}, gw1 = zero;
+  float gb1[4] = {}, gb2[4] = {}, gw3[4] = {}, gb3 = 0.0f, loss = 0.0f;
+  const int per = ((g.count + static_cast<int>(gridDim.x) * kChunk - 1) /
+                   (static_cast<int>(gridDim.x) * kChunk)) * kChunk;
   const int begin = blockIdx.x * per;
   const int end = min(g.count, begin + per);
   for (int c0 = begin; c0 < end; c0 += kChunk) {
     __syncthreads();
-    for (int e = tid; e < kChunk * kMlpIn; e += kGradThreads) {
-      const int s = e / kMlpIn, i = e % kMlpIn;
-      const int b = c0 + s;
-      float val = 0.0f;
-      if (b < end) {
-        const unsigned long long pos = static_cast<unsigned long long>(g.first + b);
-        const long idx = static_cast<long>((g.perm_a * pos + g.perm_c) % g.n);
-        val = (g.x[idx * kMlpIn + i] - g.mean[i]) * g.inv_std[i];
-      }
-      xs[s][i] = val;
-    }
     if (tid < kChunk) {
       const int b = c0 + tid;
-      vld[tid] = b < end;
-      float tv = 0.0f;
+      long idx = -1;
       if (b < end) {
         const unsigned long long pos = static_cast<unsigned long long>(g.first + b);
-        tv = g.t[static_cast<long>((g.perm_a * pos + g.perm_c) % g.n)];
+        idx = static_cast<long>((g.perm_a * pos + g.perm_c) % g.n);
       }
-      tgt[tid] = tv;
+      L.idx[tid] = idx;
+      L.tgt[tid] = idx >= 0 ? g.t[idx] : 0.0f;
     }
     __syncthreads();
-    // Thread tid owns unit u = tid % 64 of the samples s = tid / 64 + 4 q,
-    // q = 0..15, in the forward and backward passes, and the weight entries
-    // W2[tid / 64 + 4 q][tid % 64] of the gradient.
-    const int u = tid & 63;
-    const int s0 = tid >> 6;
-    {
-      float z[16];
-#pragma unroll
-      for (int q = 0; q < 16; ++q) z[q] = sw[kMlpOffB1 + u];
-      for (int i = 0; i < kMlpIn; ++i) {
-        const float wv = sw[kMlpOffW1 + u * kMlpIn + i];
-#pragma unroll
-        for (int q = 0; q < 16; ++q) z[q] += wv * xs[s0 + 4 * q][i];
-      }
-#pragma unroll
-      for (int q = 0; q < 16; ++q) h1[s0 + 4 * q][u] = tanhf(z[q]);
+    for (int e = tid; e < kChunk * 16; e += kGradThreads) {
+      const int s = e >> 4, i = e & 15;
+      const long idx = L.idx[s];
+      float v = 0.0f;
+      if (idx >= 0 && i < kMlpIn) v = (g.x[idx * kMlpIn + i] - g.mean[i]) * g.inv_std[i];
+      L.xs[s][i] = v;
     }
     __syncthreads();
-    {
-      float z[16];
+    // layer 1
+    const int row = 16 * wave + r;  // the sample of this lane's A operands
+    mlp_float4 h1[4], h2[4];
 #pragma unroll
-      for (int q = 0; q < 16; ++q) z[q] = sw[kMlpOffB2 + u];
-      for (int i = 0; i < kMlpHid; ++i) {
-        const float wv = sw[kMlpOffW2 + u * kMlpHid + i];
+    for (int nb = 0; nb < 4; ++nb) h1[nb] = zero;
 #pragma unroll
-        for (int q = 0; q < 16; ++q) z[q] += wv * h1[s0 + 4 * q][i];
+    for (int ks = 0; ks < 3; ++ks) {
+      const float a = L.xs[row][4 * ks + kq];
+#pragma unroll
+      for (int nb = 0; nb < 4; ++nb) h1[nb] = mfma4(a, w1f[nb][ks], h1[nb]);
+    }
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        h1[nb][i] = tanhf(h1[nb][i] + b1[nb]);
+        L.h1[16 * wave + 4 * kq + i][16 * nb + r] = h1[nb][i];
+      }
+    __syncthreads();
+    // layer 2
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) h2[nb] = zero;
+#pragma unroll 4
+    for (int ks = 0; ks < 16; ++ks) {
+      const float a = L.h1[row][4 * ks + kq];
+#pragma unroll
+      for (int nb = 0; nb < 4; ++nb) h2[nb] = mfma4(a, L.w2[16 * nb + r][4 * ks + kq], h2[nb]);
+    }
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) h2[nb][i] = tanhf(h2[nb][i] + b2[nb]);
+    // output, residual and the last layer's gradients, for the samples 4 kq + i
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float y = 0.0f;
+#pragma unroll
+      for (int nb = 0; nb < 4; ++nb) y += w3[nb] * h2[nb][i];
+#pragma unroll
+      for (int m = 1; m < 16; m <<= 1) y += __shfl_xor(y, m, 64);
+      const int s = 16 * wave + 4 * kq + i;
+      const float res = L.idx[s] >= 0 ? y + b3 - L.tgt[s] : 0.0f;
+      const float dy = res * g.inv_count;
+      if (r == 0) {
+        loss += 0.5f * res * res;
+        gb3 += dy;
       }
 #pragma unroll
-      for (int q = 0; q < 16; ++q) h2[s0 + 4 * q][u] = tanhf(z[q]);
+      for (int nb = 0; nb < 4; ++nb) {
+        const float hv = h2[nb][i];
+        const float d = dy * w3[nb] * (1.0f - hv * hv);
+        L.d2[s][16 * nb + r] = d;
+        gw3[nb] += dy * hv;
+        gb2[nb] += d;
+      }
     }
     __syncthreads();
-    if (tid < kChunk) {
-      float y = sw[kMlpOffB3];
-      for (int j = 0; j < kMlpHid; ++j) y += sw[kMlpOffW3 + j] * h2[tid][j];
-      const float r = vld[tid] ? y - tgt[tid] : 0.0f;
-      dy[tid] = r * g.inv_count;
-      loss += 0.5f * r * r;
+    // back through layer 2
+    mlp_float4 d1[4] = {zero, zero, zero, zero};
+#pragma unroll 4
+    for (int ks = 0; ks < 16; ++ks) {
+      const float a = L.d2[row][4 * ks + kq];
+#pragma unroll
+      for (int nb = 0; nb < 4; ++nb) d1[nb] = mfma4(a, L.w2[4 * ks + kq][16 * nb + r], d1[nb]);
     }
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float hv = h1[nb][i];
+        const float d = d1[nb][i] * (1.0f - hv * hv);
+        L.d1[16 * wave + 4 * kq + i][16 * nb + r] = d;
+        gb1[nb] += d;
+      }
     __syncthreads();
-    // backward
+    // weight gradients: rows 16 wave + ., summed over the chunk's samples
+#pragma unroll 4
+    for (int ks = 0; ks < 16; ++ks) {
+      const int s = 4 * ks + kq;
+      const float a = L.d2[s][row];
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int s = s0 + 4 * q;
-      const float hv = h2[s][u];
-      d2[s][u] = dy[s] * sw[kMlpOffW3 + u] * (1.0f - hv * hv);
-    }
-    __syncthreads();
-    {
-      float acc[16];
-#pragma unroll
-      for (int q = 0; q < 16; ++q) acc[q] = 0.0f;
-      for (int j = 0; j < kMlpHid; ++j) {
-        const float wv = sw[kMlpOffW2 + j * kMlpHid + u];
-#pragma unroll
-        for (int q = 0; q < 16; ++q) acc[q] += d2[s0 + 4 * q][j] * wv;
-      }
-#pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const float hv = h1[s0 + 4 * q][u];
-        d1[s0 + 4 * q][u] = acc[q] * (1.0f - hv * hv);
-      }
-    }
-    __syncthreads();
-    // this chunk's weight gradient, accumulated in registers
-    for (int s = 0; s < kChunk; ++s) {
-      const float hv = h1[s][u];
-#pragma unroll
-      for (int q = 0; q < 16; ++q) aw2[q] += d2[s][s0 + 4 * q] * hv;
-    }
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      const int e = tid + kGradThreads * q;
-      if (e < kMlpHid * kMlpIn) {
-        const int j = e / kMlpIn, i = e % kMlpIn;
-        float acc = 0.0f;
-        for (int s = 0; s < kChunk; ++s) acc += d1[s][j] * xs[s][i];
-        aw1[q] += acc;
-      }
-    }
-    {
-      float acc = 0.0f;
-      if (tid < 64) {
-        for (int s = 0; s < kChunk; ++s) acc += d1[s][tid];
-      } else if (tid < 128) {
-        for (int s = 0; s < kChunk; ++s) acc += d2[s][tid - 64];
-      } else if (tid < 192) {
-        for (int s = 0; s < kChunk; ++s) acc += dy[s] * h2[s][tid - 128];
-      } else if (tid == 192) {
-        for (int s = 0; s < kChunk; ++s) acc += dy[s];
-      }
-      ab += acc;
+      for (int nb = 0; nb < 4; ++nb) gw2[nb] = mfma4(a, L.h1[s][16 * nb + r], gw2[nb]);
+      gw1 = mfma4(L.d1[s][row], L.xs[s][r], gw1);
     }
   }
   float* P = g.partial + static_cast<size_t>(blockIdx.x) * kMlpParams;
-  const int u_out = tid & 63, s0_out = tid >> 6;
 #pragma unroll
-  for (int q = 0; q < 16; ++q) P[kMlpOffW2 + (s0_out + 4 * q) * kMlpHid + u_out] = aw2[q];
+  for (int i = 0; i < 4; ++i) {
+    const int j = 16 * wave + 4 * kq + i;
 #pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    const int e = tid + kGradThreads * q;
-    if (e < kMlpHid * kMlpIn) P[kMlpOffW1 + e] = aw1[q];
+    for (int nb = 0; nb < 4; ++nb) P[kMlpOffW2 + j * kMlpHid + 16 * nb + r] = gw2[nb][i];
+    if (r < kMlpIn) P[kMlpOffW1 + j * kMlpIn + r] = gw1[i];
   }
-  if (tid < 64)
-    P[kMlpOffB1 + tid] = ab;
-  else if (tid < 128)
-    P[kMlpOffB2 + tid - 64] = ab;
-  else if (tid < 192)
-    P[kMlpOffW3 + tid - 128] = ab;
-  else if (tid == 192)
-    P[kMlpOffB3] = ab;
+  // the vectors: over the wave's sample rows, then over the waves
+#pragma unroll
+  for (int m = 16; m < 64; m <<= 1) {
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) {
+      gb1[nb] += __shfl_xor(gb1[nb], m, 64);
+      gb2[nb] += __shfl_xor(gb2[nb], m, 64);
+      gw3[nb] += __shfl_xor(gw3[nb], m, 64);
+    }
+    gb3 += __shfl_xor(gb3, m, 64);
+    loss += __shfl_xor(loss, m, 64);
+  }
+  if (kq == 0) {
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) {
+      L.red[wave][0][16 * nb + r] = gb1[nb];
+      L.red[wave][1][16 * nb + r] = gb2[nb];
+      L.red[wave][2][16 * nb + r] = gw3[nb];
+    }
+  }
+  if (lane == 0) {
+    L.red1[wave][0] = gb3;
+    L.red1[wave][1] = loss;
+  }
   __syncthreads();
-  red[tid] = loss;
-  __syncthreads();
-  if (tid == 0) {
-    float s = 0.0f;
-    for (int k = 0; k < kChunk; ++k) s += red[k];
-    g.loss_part[blockIdx.x] = s;
+  if (tid < 192) {
+    const int v = tid >> 6;
+    const float sum = (L.red[0][v][lane] + L.red[1][v][lane]) +
+                      (L.red[2][v][lane] + L.red[3][v][lane]);
+    P[(v == 0 ? kMlpOffB1 : v == 1 ? kMlpOffB2 : kMlpOffW3) + lane] = sum;
+  } else if (tid < 194) {
+    const int v = tid - 192;
+    const float sum = (L.red1[0][v] + L.red1[1][v]) + (L.red1[2][v] + L.red1[3][v]);
+    if (v == 0)
+      P[kMlpOffB3] = sum;
+    else
+      g.loss_part[blockIdx.x] = sum;
   }
 }
 
-// Sums the partial gradients in workgroup order; optionally one Adam step.
-__global__ void k_mlp_adam(const float* partial, int nblk, float* w, float* m,
-                           float* v, float* grad, float lr, float b1, float b2,
-                           float eps, float bc1, float bc2, int apply,
-                           const float* loss_part, double* loss_acc) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p == 0) {
-    double s = 0.0;
-    for (int b = 0; b < nblk; ++b) s += loss_part[b];
-    *loss_acc += s;
+// Sums the partial gradients in a fixed order (four interleaved shares of the
+// workgroups' partials per parameter, then the shares); optionally one Adam
+// step.  A share of 16 partials at 4096 samples is one round trip of loads.
+constexpr int kAdamParams = 64;  // parameters per workgroup
+__global__ __launch_bounds__(4 * kAdamParams) void k_mlp_adam(
+    const float* partial, int nblk, float* w, float* m, float* v, float* grad, float lr,
+    float b1, float b2, float eps, float bc1, float bc2, int apply, const float* loss_part,
+    double* loss_acc) {
+  __shared__ float part[4][kAdamParams];
+  const int lane = threadIdx.x & 63, share = threadIdx.x >> 6;
+  const int p = blockIdx.x * kAdamParams + lane;
+  float s = 0.0f;
+  if (p < kMlpParams) {
+    const float* src = partial + p;
+#pragma unroll 16
+    for (int b = share; b < nblk; b += 4) s += src[static_cast<size_t>(b) * kMlpParams];
   }
-  if (p >= kMlpParams) return;
-  float gsum = 0.0f;
-  for (int b = 0; b < nblk; ++b) gsum += partial[static_cast<size_t>(b) * kMlpParams + p];
+  part[share][lane] = s;
+  if (blockIdx.x == 0 && share == 3) {
+    double l = 0.0;
+    for (int b = lane; b < nblk; b += 64) l += loss_part[b];
+#pragma unroll
+    for (int k = 32; k >= 1; k >>= 1) l += __shfl_xor(l, k, 64);
+    if (lane == 0) *loss_acc += l;
+  }
+  __syncthreads();
+  if (share != 0 || p >= kMlpParams) return;
+  const float gsum = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
   grad[p] = gsum;
   if (!apply) return;
   const float mm = b1 * m[p] + (1.0f - b1) * gsum;
@@ -313,7 +372,7 @@ int publish(odehip_context* ctx, odehip_mlp* m, hipStream_t s) {
 int batch_step(odehip_context* ctx, odehip_mlp* m, const float* x, const float* t, long n,
                unsigned long long a, unsigned long long c, long first, int count,
                bool apply, float lr, float b1, float b2, float eps, hipStream_t s) {
-  const int nblk = std::min(kMaxGradBlocks, std::max(1, (count + 255) / 256));
+  const int nblk = std::min(kMaxGradBlocks, std::max(1, (count + kChunk - 1) / kChunk));
   GradArgs g{};
   g.w = m->w;
   g.mean = m->mean;
@@ -336,7 +395,8 @@ int batch_step(odehip_context* ctx, odehip_mlp* m, const float* x, const float* 
     bc1 = 1.0f - std::pow(b1, static_cast<float>(m->step));
     bc2 = 1.0f - std::pow(b2, static_cast<float>(m->step));
   }
-  hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + 255) / 256), dim3(256), 0, s,
+  hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + kAdamParams - 1) / kAdamParams),
+                     dim3(4 * kAdamParams), 0, s,
                      m->partial, nblk, m->w, m->m, m->v, m->grad, lr, b1, b2, eps, bc1, bc2,
                      apply ? 1 : 0, m->loss_part, m->loss_acc);
   HIP_TRY(ctx, hipGetLastError());
