@@ -248,6 +248,135 @@ __global__ __launch_bounds__(64 * kFastWaves) void k_nbody_fast(NBodyArgs a) {
   copy_velocities(y, k, n, i0);
 }
 
+// The fast sum for grids of 64-target workgroups that would leave CUs empty: R
+// targets per workgroup, wave-uniform; each lane takes one partner of every 64
+// and sums its terms for the R targets, and the lanes' sums are folded at the
+// end.  n / R workgroups of W waves: 1000 bodies take 3.3 us instead of 13, 4096
+// 17 instead of 40, 8192 57 instead of 85.  Per-term masses throughout: finding
+// that they are equal would cost a second memory latency.
+constexpr int kFastRowsWaves = 8;
+
+// {a's lower half | b's lower half} and {a's upper | b's upper}, halves of the
+// wave (32 lanes) or of each pair of rows (16 lanes).
+__device__ __forceinline__ void swap_halves(double a, double b, double& lo, double& hi) {
+  const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
+  const auto l = __builtin_amdgcn_permlane32_swap(static_cast<uint32_t>(x),
+                                                  static_cast<uint32_t>(y), false, false);
+  const auto h = __builtin_amdgcn_permlane32_swap(static_cast<uint32_t>(x >> 32),
+                                                  static_cast<uint32_t>(y >> 32), false, false);
+  lo = __builtin_bit_cast(double, (static_cast<uint64_t>(h[0]) << 32) | l[0]);
+  hi = __builtin_bit_cast(double, (static_cast<uint64_t>(h[1]) << 32) | l[1]);
+}
+__device__ __forceinline__ void swap_rows(double a, double b, double& lo, double& hi) {
+  const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
+  const auto l = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(x),
+                                                  static_cast<uint32_t>(y), false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(x >> 32),
+                                                  static_cast<uint32_t>(y >> 32), false, false);
+  lo = __builtin_bit_cast(double, (static_cast<uint64_t>(h[0]) << 32) | l[0]);
+  hi = __builtin_bit_cast(double, (static_cast<uint64_t>(h[1]) << 32) | l[1]);
+}
+template <int kRotate>
+__device__ __forceinline__ double rotated_in_row(double v) {
+  const uint64_t x = __builtin_bit_cast(uint64_t, v);
+  const uint32_t l = __builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x120 + kRotate, 0xf,
+                                                 0xf, true);
+  const uint32_t h = __builtin_amdgcn_update_dpp(0, static_cast<int>(x >> 32), 0x120 + kRotate,
+                                                 0xf, 0xf, true);
+  return __builtin_bit_cast(double, (static_cast<uint64_t>(h) << 32) | l);
+}
+
+// Sums v[0 .. V - 1] over the wave's lanes into out[0 .. V - 1] (LDS).  Two
+// values share each swap, so halving the lanes halves the values.
+template <int V>
+__device__ __forceinline__ void wave_sums(const double (&v)[V], double* out, int lane) {
+  constexpr int V1 = (V + 1) / 2, V2 = (V1 + 1) / 2;
+  double u[V1], w[V2];
+#pragma unroll
+  for (int m = 0; m < V1; ++m) {
+    double lo, hi;
+    swap_halves(v[2 * m], 2 * m + 1 < V ? v[2 * m + 1] : 0.0, lo, hi);
+    u[m] = lo + hi;
+  }
+#pragma unroll
+  for (int m = 0; m < V2; ++m) {
+    double lo, hi;
+    swap_rows(u[2 * m], 2 * m + 1 < V1 ? u[2 * m + 1] : 0.0, lo, hi);
+    w[m] = lo + hi;
+  }
+  // row r of w[m] holds the sums of value 4 m + 2 (r & 1) + (r >> 1)
+  const int r = lane >> 4;
+#pragma unroll
+  for (int m = 0; m < V2; ++m) {
+    double s = w[m];
+    s += rotated_in_row<8>(s);
+    s += rotated_in_row<4>(s);
+    s += rotated_in_row<2>(s);
+    s += rotated_in_row<1>(s);
+    const int id = 4 * m + 2 * (r & 1) + (r >> 1);
+    if ((lane & 15) == 0 && id < V) out[id] = s;
+  }
+}
+
+// The last workgroup's targets are the last R bodies (n >= R).
+template <int R, bool kMass, bool kGuard>
+__global__ __launch_bounds__(64 * kFastRowsWaves) void k_nbody_fast_rows(NBodyArgs a) {
+  if (prologue_skip(a)) return;
+  __shared__ double red[kFastRowsWaves][3 * R];
+  const double* __restrict__ y = select_input(a);
+  const uniform_ptr yu = as_uniform(y);
+  double* __restrict__ k = a.k;
+  const double* __restrict__ mass = a.mass;
+  const int n = a.n;
+  const double eps2 = a.eps2;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int step = blockDim.x;
+  const int i0 = min(static_cast<int>(blockIdx.x) * R, n - R);
+  const int j = min(wave * 64 + lane, n - 1);
+  double px = y[3 * j], py = y[3 * j + 1], pz = y[3 * j + 2];
+  double pm = kMass ? mass[j] : 1.0;
+  double tx[R], ty[R], tz[R], v[3 * R];
+#pragma unroll
+  for (int t = 0; t < R; ++t) {
+    tx[t] = yu[3 * (i0 + t)];
+    ty[t] = yu[3 * (i0 + t) + 1];
+    tz[t] = yu[3 * (i0 + t) + 2];
+    v[3 * t] = v[3 * t + 1] = v[3 * t + 2] = 0.0;
+  }
+  const int e = threadIdx.x;
+  if (e < 3 * R) k[3L * i0 + e] = y[3L * n + 3L * i0 + e];
+  for (int b = wave * 64; b < n; b += step) {
+    const int jn = min(b + step + lane, n - 1);  // the next partner, loaded ahead
+    const double qx = y[3 * jn], qy = y[3 * jn + 1], qz = y[3 * jn + 2];
+    const double qm = kMass ? mass[jn] : 1.0;
+    if (b + 64 <= n) {
+#pragma unroll
+      for (int t = 0; t < R; ++t)
+        fast_term<kMass, kGuard>(px, py, pz, pm, b + lane, i0 + t, tx[t], ty[t], tz[t], eps2,
+                                 v[3 * t], v[3 * t + 1], v[3 * t + 2]);
+    } else {
+      // lanes past the end pass as the target itself: their terms are left out
+      const bool in = b + lane < n;
+#pragma unroll
+      for (int t = 0; t < R; ++t)
+        fast_term<kMass, true>(px, py, pz, pm, in ? (kGuard ? b + lane : -1) : i0 + t, i0 + t,
+                               tx[t], ty[t], tz[t], eps2, v[3 * t], v[3 * t + 1], v[3 * t + 2]);
+    }
+    px = qx;
+    py = qy;
+    pz = qz;
+    pm = qm;
+  }
+  wave_sums<3 * R>(v, red[wave], lane);
+  __syncthreads();
+  if (e < 3 * R) {
+    double s = 0.0;
+    for (int w = 0; w < step / 64; ++w) s += red[w][e];
+    k[3L * n + 3L * i0 + e] = s;
+  }
+}
+
 // ------------------------------------------------------------------ mixed --
 constexpr int kMixedWaves = 16;
 constexpr int kMixedFlush = 32;
@@ -552,6 +681,24 @@ int device_cus() {
 }
 }  // namespace
 
+namespace {
+template <int R>
+void launch_fast_rows(const NBodyArgs& a, bool guard, int waves, hipStream_t s) {
+  auto* kern = a.mass ? (guard ? k_nbody_fast_rows<R, true, true> : k_nbody_fast_rows<R, true, false>)
+                      : (guard ? k_nbody_fast_rows<R, false, true>
+                               : k_nbody_fast_rows<R, false, false>);
+  hipLaunchKernelGGL(kern, dim3((a.n + R - 1) / R), dim3(64 * waves), 0, s, a);
+}
+// R so that up to 4 bodies per CU the grid is one workgroup per CU; more waves
+// than steps of 64 partners would idle.
+void launch_fast_rows(const NBodyArgs& a, bool guard, hipStream_t s) {
+  const int cus = device_cus(), steps = (a.n + 63) / 64;
+  if (a.n <= cus) return launch_fast_rows<1>(a, guard, std::min(4, steps), s);
+  if (a.n <= 2 * cus) return launch_fast_rows<2>(a, guard, std::min(4, steps), s);
+  launch_fast_rows<4>(a, guard, std::min(kFastRowsWaves, steps), s);
+}
+}  // namespace
+
 hipError_t launch_nbody_rhs(const NBodyArgs& a, int variant, hipStream_t s) {
   if (a.n <= 0) return hipSuccess;
   const unsigned blocks = static_cast<unsigned>((a.n + 63) / 64);
@@ -563,6 +710,12 @@ hipError_t launch_nbody_rhs(const NBodyArgs& a, int variant, hipStream_t s) {
       break;
     }
     case ODEHIP_NBODY_FAST: {
+      // 64-target workgroups for less than 0.7 of the CUs (MI355X: up to 11468
+      // bodies; at 8192 57 us against 85, at 16384 220 against 157)
+      if (10L * blocks < 7L * device_cus()) {
+        launch_fast_rows(a, guard, s);
+        break;
+      }
       // one workgroup per CU at most: 4 waves per SIMD, prefetching partner loop
       const bool prefetch = static_cast<long>(blocks) <= device_cus();
       auto* kern = mass ? (guard ? (prefetch ? k_nbody_fast<true, true, true>

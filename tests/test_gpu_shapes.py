@@ -28,6 +28,17 @@ def test_exact_rhs_at_shape_edges(exe, n, form):
         f"n={n}: max abs diff {np.max(np.abs(got - want))}"
 
 
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 256, 257, 512, 513, 517, 1027, 11467, 11521])
+@pytest.mark.parametrize("eps,masses", [(1e-2, False), (1e-2, True), (0.0, True)])
+def test_fast_rhs_at_shape_edges(exe, n, eps, masses):
+    x, m = ic(n, seed=n + 2, masses=masses)
+    got = gpu_rhs(exe, x, eps, m, "fast")
+    want = O.rhs(O.RHS_NBODY, x, eps, m, threads=8)
+    assert np.array_equal(got[:3 * n], want[:3 * n])
+    scale = np.max(np.abs(want[3 * n:])) if n > 1 else 1.0
+    assert np.max(np.abs(got - want)) <= 5e-14 * scale  # the variant's bar
+
+
 @pytest.mark.parametrize("n", [33000, 40000])
 def test_exact_rhs_several_workgroups_per_cu(exe, n):
     """Two and more 64-target workgroups per CU (four waves each); rows of a few targets
