@@ -31,7 +31,7 @@ struct EnsBufs {
   const EnsTile* tiles;  // RHS work items in dispatch order
   int n_tiles;           // slots: RHS workgroups x waves per workgroup
   SolverState* st;       // one per system
-  int* n_active;         // systems still running
+  int* n_active;         // systems still running: in rounds, one-workgroup ones
   double* xb0;
   double* xb1;
   double* ks;
@@ -48,6 +48,9 @@ struct EnsBufs {
   double atol, rtol;
   size_t nv;
   int n_sys;
+  int solo_n;    // systems of up to this many bodies are solved by
+                 // one workgroup each (solo.hpp); 0: none
+  int n_solo;    // their number
   int n_groups;  // entries of `groups` (workgroups of an element launch)
   int tableau;
   int variant;
@@ -81,9 +84,11 @@ constexpr EnsTileConfig kEnsTileConfigs[ODEHIP_ENS_TILE_CONFIGS] = {
     {1, kEnsNoTpl2, 0, 2}, {1, kEnsNoTpl2, 1, 2}, {1, kEnsNoTpl2, 0, 4},
     {1, kEnsNoTpl2, 1, 4}, {1, kEnsNoTpl2, 0, 8}, {1, kEnsNoTpl2, 1, 8}};
 constexpr int kEnsDefaultTileConfig = 1;
-// Partners per chunk of the fast and mixed sums (a multiple of the mixed
-// variant's FP32 flush interval, 32).
+// Partners per chunk of the fast and mixed sums (see ens_chunks.hpp).
 constexpr int kEnsChunk = 128;
+// SIMDs of the device (256 CUs x 4): the waves one launch needs to give
+// each SIMD one.
+constexpr long kEnsSimds = 1024;
 // Waves that give each of the 1024 SIMDs (256 CUs x 4) four, the depth that
 // hides the RHS arithmetic's latency.
 constexpr long kEnsFillWaves = 4096;

@@ -4,7 +4,9 @@
 // The driver mirrors odehip_rk_solve: initial step for every system, then K
 // lockstep rounds (one attempt of each active system per round) captured in
 // a HIP graph and replayed until the device-side count of running systems
-// reaches zero; the host polls that count one replay behind.
+// reaches zero; the host polls that count one replay behind.  Systems small
+// enough for one workgroup run beside the rounds, on a stream of their own,
+// each at its own pace (solo_kernels.hip).
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -16,14 +18,19 @@
 #include "ensemble.hpp"
 #include "ensemble_plan.hpp"
 #include "mlp.hpp"
+#include "solo.hpp"
 
 namespace odehip {
 
 struct EnsembleWorkspace {
   char* dev = nullptr;  // device arena
   size_t cap = 0;       // bytes
-  int* h_active = nullptr;  // pinned, 2 slots
+  int* h_active = nullptr;  // pinned, 2 slots for the rounds, 2 for `side`
   hipEvent_t ev[2] = {nullptr, nullptr};
+  // the one-workgroup solves' stream
+  hipStream_t side = nullptr;
+  hipEvent_t ev_side[2] = {nullptr, nullptr};
+  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   hipEvent_t t0 = nullptr, t1 = nullptr;
   // cached graph of K rounds and the arguments it was captured with
   hipGraph_t graph = nullptr;
@@ -44,6 +51,14 @@ struct EnsembleWorkspace {
 
 void destroy_ensemble_workspace(EnsembleWorkspace* w) {
   if (!w) return;
+  if (w->side) {
+    (void)hipStreamSynchronize(w->side);
+    (void)hipStreamDestroy(w->side);
+  }
+  for (auto& e : w->ev_side)
+    if (e) (void)hipEventDestroy(e);
+  if (w->ev_fork) (void)hipEventDestroy(w->ev_fork);
+  if (w->ev_join) (void)hipEventDestroy(w->ev_join);
   if (w->exec) (void)hipGraphExecDestroy(w->exec);
   if (w->graph) (void)hipGraphDestroy(w->graph);
   if (w->dev) (void)hipFree(w->dev);
@@ -72,8 +87,11 @@ int workspace(odehip_context* ctx, size_t bytes, EnsembleWorkspace** out) {
     auto* w = new (std::nothrow) EnsembleWorkspace();
     if (!w) return fail(ctx, ODEHIP_ERR_NOMEM, "ensemble workspace");
     ctx->ens = w;
-    HIP_TRY(ctx, hipHostMalloc(reinterpret_cast<void**>(&w->h_active), 2 * sizeof(int)));
-    for (auto& e : w->ev) HIP_TRY(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    HIP_TRY(ctx, hipHostMalloc(reinterpret_cast<void**>(&w->h_active), 4 * sizeof(int)));
+    HIP_TRY(ctx, hipStreamCreateWithFlags(&w->side, hipStreamNonBlocking));
+    for (hipEvent_t* e : {&w->ev[0], &w->ev[1], &w->ev_side[0], &w->ev_side[1], &w->ev_fork,
+                          &w->ev_join})
+      HIP_TRY(ctx, hipEventCreateWithFlags(e, hipEventDisableTiming));
     HIP_TRY(ctx, hipEventCreate(&w->t0));
     HIP_TRY(ctx, hipEventCreate(&w->t1));
   }
@@ -306,7 +324,8 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
   const size_t tcap = tiles_capacity(L);
   const Plan p = plan(L, tcap, S, trace_cap, true, n_dense);
   EnsembleWorkspace* w = nullptr;
-  if ((rc = workspace(ctx, p.total, &w))) return rc;
+  // (after the plan's regions: the list of one-workgroup systems)
+  if ((rc = workspace(ctx, p.total + L.sys.size() * sizeof(int), &w))) return rc;
   const double eps2 = softening * softening;
   const double near_c = nbody_variant == ODEHIP_NBODY_MIXED ? ctx->near_c : 0.0;
   hipStream_t s = begin_work(ctx);
@@ -353,9 +372,29 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
     for (int c = 0; c < ODEHIP_ENS_TILE_CONFIGS; ++c)
       opt->tune_ms[c] = tuned ? w->tuned_ms[c] : 0.0;
   }
+  // Small systems are solved by one workgroup each (solo.hpp) unless the caller
+  // names a tile configuration; dense output is written by the rounds only.
+  const bool exact = nbody_variant == ODEHIP_NBODY_EXACT;
+  std::vector<int> solo;
+  std::vector<char> live(L.sys.size(), 1);
+  int solo_max = 0;
+  if (opt->tile_config == ODEHIP_ENS_TILE_AUTO && n_dense == 0) {
+    b.solo_n = solo_limit(S, nbody_variant);
+    for (size_t k = 0; k < L.sys.size(); ++k) {
+      if (L.sys[k].n > b.solo_n) continue;
+      solo.push_back(static_cast<int>(k));
+      live[k] = 0;
+      solo_max = std::max(solo_max, L.sys[k].n);
+    }
+    // the longest evaluations first
+    std::stable_sort(solo.begin(), solo.end(),
+                     [&](int p, int q) { return L.sys[p].n > L.sys[q].n; });
+  }
+  b.n_solo = static_cast<int>(solo.size());
+  const int n_rounds = n_systems - b.n_solo;
+
   // a tile's partners are shared by several waves from the start when the
   // ensemble's tiles would leave SIMDs idle
-  const bool exact = nbody_variant == ODEHIP_NBODY_EXACT;
   int run_cfg = tail_config(L, nullptr, cfg, exact);
   int n_tiles = 0;
   if ((rc = upload_tables(ctx, w, p, L, tcap, run_cfg, &n_tiles, s))) return rc;
@@ -364,6 +403,66 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
   HIP_TRY(ctx, ens_enqueue_init(b, x0, opt->t0, opt->tf, opt->max_accepted,
                                 opt->max_attempts, opt->fsal ? 1 : 0, opt->controller, s));
   HIP_TRY(ctx, ens_enqueue_initial_step(b, s));
+
+  // The one-workgroup solves: launches of kSoloAttempts attempts, two ahead of
+  // the host, until their count of running systems has been seen at zero.
+  SoloArgs sa{};
+  long solo_pushed = 0, solo_seen = 0;
+  bool solo_done = solo.empty();
+  auto push_solo = [&]() -> int {
+    const int at = static_cast<int>(solo_pushed & 1);
+    HIP_TRY(ctx, launch_solo(sa, solo_max, nbody_variant, static_cast<unsigned>(solo.size()),
+                             w->side));
+    HIP_TRY(ctx, hipMemcpyAsync(&w->h_active[2 + at], b.n_active + 1, sizeof(int),
+                                hipMemcpyDeviceToHost, w->side));
+    HIP_TRY(ctx, hipEventRecord(w->ev_side[at], w->side));
+    ++solo_pushed;
+    return ODEHIP_OK;
+  };
+  // Takes in finished launches (waiting for the oldest one if `wait`) and keeps
+  // two in flight.
+  auto poll_solo = [&](bool wait) -> int {
+    while (!solo_done) {
+      if (solo_pushed - solo_seen < 2) {
+        if (const int prc = push_solo()) return prc;
+        continue;
+      }
+      const int at = static_cast<int>(solo_seen & 1);
+      const hipError_t q = wait ? hipEventSynchronize(w->ev_side[at])
+                                : hipEventQuery(w->ev_side[at]);
+      if (q == hipErrorNotReady) return ODEHIP_OK;
+      if (q != hipSuccess) return hip_fail(ctx, q, "one-workgroup solves");
+      ++solo_seen;
+      solo_done = w->h_active[2 + at] == 0;
+    }
+    return ODEHIP_OK;
+  };
+  if (!solo.empty()) {
+    HIP_TRY(ctx, hipStreamSynchronize(s));  // earlier launches read the list's region
+    HIP_TRY(ctx, hipMemcpy(w->dev + p.total, solo.data(), solo.size() * sizeof(int),
+                           hipMemcpyHostToDevice));
+    sa.sys = b.sys;
+    sa.list = reinterpret_cast<const int*>(w->dev + p.total);
+    sa.st = b.st;
+    sa.xb0 = b.xb0;
+    sa.xb1 = b.xb1;
+    sa.ks = b.ks;
+    sa.kfsal = b.kfsal;
+    sa.mass = b.mass;
+    sa.atol = b.atol;
+    sa.rtol = b.rtol;
+    sa.trace = b.trace;
+    sa.trace_cap = b.trace_cap;
+    sa.mlp = static_cast<const MlpInfer*>(b.mlp);
+    sa.n_active = b.n_active + 1;
+    sa.eps2 = b.eps2;
+    sa.near_c = b.near_c;
+    sa.tableau = tableau;
+    sa.attempts = kSoloAttempts;
+    HIP_TRY(ctx, hipEventRecord(w->ev_fork, s));
+    HIP_TRY(ctx, hipStreamWaitEvent(w->side, w->ev_fork, 0));
+    if ((rc = poll_solo(false))) return rc;
+  }
 
   // Rounds run on lists of the running systems' workgroups: every system at
   // first, rebuilt (and the graph re-captured) each time the number of
@@ -405,21 +504,54 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
     return ODEHIP_OK;
   };
   EnsBufs rb = b;  // run_cfg: the tile shape of the running systems
-  int K = rounds_per_replay(L.work);
-  if ((rc = capture(rb, K))) return rc;
+  int K = 0, n_live = n_rounds;
+  // Lists and graph for the systems `live` marks (the stream is idle).
+  auto set_running = [&]() -> int {
+    std::vector<int2> act;
+    double sum_n2 = 0.0;
+    for (size_t k = 0; k < L.sys.size(); ++k) {
+      if (!live[k]) continue;
+      sum_n2 += static_cast<double>(L.sys[k].n) * L.sys[k].n;
+      for (int g = 0; g < L.sys[k].n_groups; ++g) act.push_back(L.groups[L.sys[k].gbase + g]);
+    }
+    // once the running systems' tiles no longer give every SIMD four
+    // waves: 64-target tiles, then partners shared by several waves per
+    // tile; same results
+    run_cfg = tail_config(L, &live, run_cfg, exact);
+    const std::vector<EnsTile> tiles = make_tiles(L, kEnsTileConfigs[run_cfg], &live);
+    if (const char* why = check_tiles(tiles, L, tcap)) return fail(ctx, ODEHIP_ERR_INVALID, why);
+    HIP_TRY(ctx, hipMemcpy(w->dev + p.groups_act, act.data(), act.size() * sizeof(int2),
+                           hipMemcpyHostToDevice));
+    HIP_TRY(ctx, hipMemcpy(w->dev + p.tiles, tiles.data(), tiles.size() * sizeof(EnsTile),
+                           hipMemcpyHostToDevice));
+    w->tables.invalidate();  // the tile region now holds the running systems' tiles
+    rb.groups = reinterpret_cast<const int2*>(w->dev + p.groups_act);
+    rb.n_groups = static_cast<int>(act.size());
+    set_tile_cfg(&rb, run_cfg, static_cast<int>(tiles.size()));
+    K = rounds_per_replay(sum_n2);
+    return capture(rb, K);
+  };
+  if (n_rounds == n_systems) {
+    K = rounds_per_replay(L.work);
+    if ((rc = capture(rb, K))) return rc;
+  } else if (n_rounds > 0) {
+    HIP_TRY(ctx, hipStreamSynchronize(s));
+    if ((rc = set_running())) return rc;
+  }
 
   const long cap_rounds = opt->max_attempts > 0 ? opt->max_attempts : (1L << 40);
   long launched = 0;
   int slot = 0;
   bool have_prev = false;
-  int compact_below = n_systems * 7 / 8;
+  int compact_below = n_rounds * 7 / 8;
   std::vector<SolverState> hst;
-  for (;;) {
+  while (n_rounds > 0) {
     HIP_TRY(ctx, hipGraphLaunch(w->exec, s));
     launched += K;
     HIP_TRY(ctx, hipMemcpyAsync(&w->h_active[slot], b.n_active, sizeof(int),
                                 hipMemcpyDeviceToHost, s));
     HIP_TRY(ctx, hipEventRecord(w->ev[slot], s));
+    if ((rc = poll_solo(false))) return rc;
     if (launched >= cap_rounds + 2L * K) break;
     if (have_prev) {
       HIP_TRY(ctx, hipEventSynchronize(w->ev[slot ^ 1]));
@@ -430,36 +562,13 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
         hst.resize(L.sys.size());
         HIP_TRY(ctx, hipMemcpy(hst.data(), b.st, hst.size() * sizeof(SolverState),
                                hipMemcpyDeviceToHost));
-        std::vector<char> live(L.sys.size());
-        std::vector<int2> act;
-        double sum_n2 = 0.0;
-        int n_live = 0;
+        n_live = 0;
         for (size_t k = 0; k < L.sys.size(); ++k) {
-          live[k] = hst[k].done ? 0 : 1;
-          if (!live[k]) continue;
-          ++n_live;
-          sum_n2 += static_cast<double>(L.sys[k].n) * L.sys[k].n;
-          for (int g = 0; g < L.sys[k].n_groups; ++g)
-            act.push_back(L.groups[L.sys[k].gbase + g]);
+          live[k] = live[k] && !hst[k].done;
+          n_live += live[k];
         }
         if (n_live == 0) break;
-        // once the running systems' tiles no longer give every SIMD four
-        // waves: 64-target tiles, then partners shared by several waves per
-        // tile; same results
-        run_cfg = tail_config(L, &live, run_cfg, exact);
-        const std::vector<EnsTile> tiles = make_tiles(L, kEnsTileConfigs[run_cfg], &live);
-        if (const char* why = check_tiles(tiles, L, tcap))
-          return fail(ctx, ODEHIP_ERR_INVALID, why);
-        HIP_TRY(ctx, hipMemcpy(w->dev + p.groups_act, act.data(), act.size() * sizeof(int2),
-                               hipMemcpyHostToDevice));
-        HIP_TRY(ctx, hipMemcpy(w->dev + p.tiles, tiles.data(), tiles.size() * sizeof(EnsTile),
-                               hipMemcpyHostToDevice));
-        w->tables.invalidate();  // the tile region now holds the running systems' tiles
-        rb.groups = reinterpret_cast<const int2*>(w->dev + p.groups_act);
-        rb.n_groups = static_cast<int>(act.size());
-        set_tile_cfg(&rb, run_cfg, static_cast<int>(tiles.size()));
-        K = rounds_per_replay(sum_n2);
-        if ((rc = capture(rb, K))) return rc;
+        if ((rc = set_running())) return rc;
         compact_below = n_live * 7 / 8;
         have_prev = false;
         slot = 0;
@@ -468,6 +577,11 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
     }
     have_prev = true;
     slot ^= 1;
+  }
+  if (!solo.empty()) {
+    if ((rc = poll_solo(true))) return rc;
+    HIP_TRY(ctx, hipEventRecord(w->ev_join, w->side));
+    HIP_TRY(ctx, hipStreamWaitEvent(s, w->ev_join, 0));
   }
   HIP_TRY(ctx, ens_enqueue_copy_out(b, x_out, s));
   std::vector<SolverState> hs(L.sys.size());

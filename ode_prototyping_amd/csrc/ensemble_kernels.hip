@@ -20,7 +20,7 @@
 // list is built on the host per tile configuration.  When few systems still
 // run, a tile can instead be shared by the 2, 4 or 8 waves of a workgroup
 // (k_ens_rhs_split, k_ens_rhs_exact_split), with the same bits.
-#include "ensemble.hpp"
+#include "ens_chunks.hpp"
 #include "mlp.hpp"
 #include "nbody_terms.hpp"
 #include "rk_device.hpp"
@@ -190,41 +190,6 @@ __device__ __forceinline__ void exact_tile(const double* __restrict__ y,
   tile_velocities<TPL>(y, k, n, i0);
 }
 
-// Partner chunks of the reorderable variants (fast, mixed): each target's
-// sum is the sum, in chunk order, of the sums over partners
-// [c kEnsChunk, (c + 1) kEnsChunk) taken in increasing j.  The order does not
-// depend on how many waves share a tile, so the split kernel below (chunks
-// of one tile on several waves, folded in order) gives the same bits as one
-// wave walking every chunk.
-
-// fast: partners j0 .. j1 - 1 summed into p* (which the caller zeroes).
-template <bool kMass, bool kGuard, int TPL>
-__device__ inline void fast_chunk(uniform_ptr yu, uniform_ptr mu, int j0, int j1,
-                                  const int* ic, const double* xi, const double* yi,
-                                  const double* zi, double eps2, double* px, double* py,
-                                  double* pz) {
-  constexpr int U = TPL == 1 ? 8 : 4;
-  int j = j0;
-  for (; j + U <= j1; j += U) {
-    const uniform_ptr pp = yu + 3 * j;
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const double mj = kMass ? mu[j + u] : 1.0;
-#pragma unroll
-      for (int t = 0; t < TPL; ++t)
-        fast_term<kMass, kGuard>(pp[3 * u], pp[3 * u + 1], pp[3 * u + 2], mj, j + u,
-                                 ic[t], xi[t], yi[t], zi[t], eps2, px[t], py[t], pz[t]);
-    }
-  }
-  for (; j < j1; ++j) {
-    const double mj = kMass ? mu[j] : 1.0;
-#pragma unroll
-    for (int t = 0; t < TPL; ++t)
-      fast_term<kMass, kGuard>(yu[3 * j], yu[3 * j + 1], yu[3 * j + 2], mj, j, ic[t],
-                               xi[t], yi[t], zi[t], eps2, px[t], py[t], pz[t]);
-  }
-}
-
 // The targets of a tile: coordinates of i0 + 64 t + lane (lanes past n
 // clamped to n - 1, their results not stored).
 template <int TPL>
@@ -275,112 +240,6 @@ __device__ inline void fast_tile(const double* __restrict__ y,
   }
   tile_store<TPL>(k, n, i0, ax, ay, az);
   tile_velocities<TPL>(y, k, n, i0);
-}
-
-// mixed: FP64 displacement rounded to FP32, FP32 pair force, partial sums
-// in FP32 flushed into FP64 every 32 partners.  kNear: near pairs (FP32
-// r^2 < near2) are left out of the FP32 sums and their FP64 term is added
-// into the FP64 sums; without it every pair is FP32.
-// Partners j0 .. j1 - 1 (j0 a multiple of kFlush) summed into the FP64
-// sums a* (which the caller zeroes).
-template <bool kMass, bool kGuard, bool kNear, int TPL>
-__device__ inline void mixed_chunk(uniform_ptr yu, uniform_ptr mu, int j0, int j1,
-                                   const int* ic, const double* xi, const double* yi,
-                                   const double* zi, double eps2, float near2, double* ax,
-                                   double* ay, double* az) {
-  constexpr int kFlush = 32;
-  constexpr int U = 8;
-  static_assert(kEnsChunk % kFlush == 0, "chunks start on a flush boundary");
-  const float eps2f = static_cast<float>(eps2);
-  int j = j0;
-  while (j < j1) {
-    const int jstop = min(j1, j + kFlush);
-    float fx[TPL], fy[TPL], fz[TPL];
-#pragma unroll
-    for (int t = 0; t < TPL; ++t) fx[t] = fy[t] = fz[t] = 0.0f;
-    if constexpr (!kNear) {
-      for (; j + U <= jstop; j += U) {
-        const uniform_ptr pp = yu + 3 * j;
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const float mj = kMass ? static_cast<float>(mu[j + u]) : 1.0f;
-#pragma unroll
-          for (int t = 0; t < TPL; ++t)
-            mixed_term_fp32<kMass, kGuard>(pp[3 * u], pp[3 * u + 1], pp[3 * u + 2], mj,
-                                           j + u, ic[t], xi[t], yi[t], zi[t], eps2f, fx[t],
-                                           fy[t], fz[t]);
-        }
-      }
-      for (; j < jstop; ++j) {
-        const float mj = kMass ? static_cast<float>(mu[j]) : 1.0f;
-#pragma unroll
-        for (int t = 0; t < TPL; ++t)
-          mixed_term_fp32<kMass, kGuard>(yu[3 * j], yu[3 * j + 1], yu[3 * j + 2], mj, j,
-                                         ic[t], xi[t], yi[t], zi[t], eps2f, fx[t], fy[t],
-                                         fz[t]);
-      }
-    } else {
-      for (; j + U <= jstop; j += U) {
-        const uniform_ptr pp = yu + 3 * j;
-        // bit u: some lane has partner j + u in the near field of one of its targets
-        uint32_t near = 0;
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const double mj = kMass ? mu[j + u] : 1.0;
-          uint64_t lanes = 0;
-#pragma unroll
-          for (int t = 0; t < TPL; ++t)
-            lanes |= ballot_not(mixed_term<kMass, kGuard>(pp[3 * u], pp[3 * u + 1],
-                                                          pp[3 * u + 2], mj, j + u, ic[t],
-                                                          xi[t], yi[t], zi[t], eps2f, near2,
-                                                          fx[t], fy[t], fz[t]));
-          near |= lanes ? (1u << u) : 0u;
-        }
-#pragma unroll
-        for (int t = 0; t < TPL; ++t) {
-          fx[t] = opaque(fx[t]);
-          fy[t] = opaque(fy[t]);
-          fz[t] = opaque(fz[t]);
-        }
-        if (near) {
-          double xo[TPL], yo[TPL], zo[TPL];
-#pragma unroll
-          for (int t = 0; t < TPL; ++t) {
-            xo[t] = opaque(xi[t]);
-            yo[t] = opaque(yi[t]);
-            zo[t] = opaque(zi[t]);
-          }
-          do {
-            const int u = __builtin_ctz(near);
-            near &= near - 1;
-            const double mj = kMass ? mu[j + u] : 1.0;
-#pragma unroll
-            for (int t = 0; t < TPL; ++t)
-              mixed_near_term<kMass, kGuard>(pp[3 * u], pp[3 * u + 1], pp[3 * u + 2], mj,
-                                             j + u, ic[t], xo[t], yo[t], zo[t], eps2f, eps2,
-                                             near2, ax[t], ay[t], az[t]);
-          } while (near);
-        }
-      }
-      for (; j < jstop; ++j) {
-        const double mj = kMass ? mu[j] : 1.0;
-#pragma unroll
-        for (int t = 0; t < TPL; ++t)
-          if (!mixed_term<kMass, kGuard>(yu[3 * j], yu[3 * j + 1], yu[3 * j + 2], mj, j,
-                                         ic[t], xi[t], yi[t], zi[t], eps2f, near2, fx[t],
-                                         fy[t], fz[t]))
-            mixed_near_term<kMass, kGuard>(yu[3 * j], yu[3 * j + 1], yu[3 * j + 2], mj, j,
-                                           ic[t], xi[t], yi[t], zi[t], eps2f, eps2, near2,
-                                           ax[t], ay[t], az[t]);
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < TPL; ++t) {
-      ax[t] += static_cast<double>(fx[t]);
-      ay[t] += static_cast<double>(fy[t]);
-      az[t] += static_cast<double>(fz[t]);
-    }
-  }
 }
 
 template <bool kMass, bool kGuard, bool kNear, int TPL>
@@ -774,11 +633,29 @@ __global__ void k_ens_controller(EnsBufs b) {
   SolverState* st = b.st + s;
   if (st->done) return;
   const EnsSys sy = b.sys[s];
+  if (sy.n <= b.solo_n) return;
   const double sum = fold_partials(b.partA + sy.gbase, sy.n_groups);
   double* trace = b.trace ? b.trace + static_cast<size_t>(s) * b.trace_cap * 3 : nullptr;
   ctrl_attempt(st, e_tab[st->tableau], sum, 6 * static_cast<size_t>(sy.n), nullptr,
                trace);
   if (st->done) atomicSub(b.n_active, 1);
+}
+
+// One wave per system, the reference and PI controllers on its first lane:
+// the partials come in side by side, and systems do not wait for each other's
+// branches.
+__global__ __launch_bounds__(64) void k_ens_controller_wave(EnsBufs b) {
+  __shared__ float x[16], h[64];
+  const int s = blockIdx.x;
+  SolverState* st = b.st + s;
+  const EnsSys sy = b.sys[s];
+  if (st->done || sy.n <= b.solo_n) return;  // read by every lane before lane 0 writes it
+  const Tableau& T = e_tab[b.tableau];
+  const double sum = fold_partials_block(b.partA + sy.gbase, sy.n_groups);
+  double* trace = b.trace ? b.trace + static_cast<size_t>(s) * b.trace_cap * 3 : nullptr;
+  ctrl_attempt_wave(st, T, sum, 6 * static_cast<size_t>(sy.n), nullptr, trace,
+                    static_cast<const MlpInfer*>(b.mlp), sy.n, x, h);
+  if (threadIdx.x == 0 && st->done) atomicSub(b.n_active, 1);
 }
 
 // The same with the learned controller: one wave per 16 systems; their
@@ -789,7 +666,7 @@ __global__ __launch_bounds__(64) void k_ens_controller_learned(EnsBufs b) {
   const int lane = threadIdx.x;
   const int s = blockIdx.x * 16 + lane;
   SolverState* st = (lane < 16 && s < b.n_sys) ? b.st + s : nullptr;
-  const bool active = st && !st->done;
+  const bool active = st && !st->done && b.sys[s].n > b.solo_n;
   bool accept = false, judged = false;
   float raw[kMlpIn];
   for (int i = 0; i < kMlpIn; ++i) raw[i] = 0.0f;
@@ -807,9 +684,7 @@ __global__ __launch_bounds__(64) void k_ens_controller_learned(EnsBufs b) {
   mlp_tile_forward(M, tile);
   if (active) {
     if (judged) {
-      double y = tile.y[lane];
-      y = y < kMlpLogRatioMin ? kMlpLogRatioMin : (y > kMlpLogRatioMax ? kMlpLogRatioMax : y);
-      ctrl_step(st, accept, std::isfinite(y) ? std::exp(y) : NAN);
+      ctrl_step(st, accept, mlp_ratio(tile.y[lane]));
     }
     if (st->done) atomicSub(b.n_active, 1);
   }
@@ -855,7 +730,10 @@ __global__ __launch_bounds__(kBlock) void k_ens_dense_out5(EnsBufs b) {
 __global__ void k_ens_init(EnsBufs b, double t0, double tf, long max_acc,
                            long max_att, int fsal, int controller) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s == 0) *b.n_active = (t0 < tf) ? b.n_sys : 0;
+  if (s == 0) {
+    b.n_active[0] = (t0 < tf) ? b.n_sys - b.n_solo : 0;
+    b.n_active[1] = (t0 < tf) ? b.n_solo : 0;
+  }
   if (s >= b.n_sys) return;
   ctrl_init(b.st + s, e_tab[b.tableau], t0, tf, max_acc, max_att, fsal, b.tableau,
             b.sys[s].n_groups, 0, b.trace ? b.trace_cap : 0, controller);
@@ -1066,7 +944,11 @@ hipError_t ens_enqueue_round(const EnsBufs& b, hipStream_t s) {
       return e;
   }
   hipLaunchKernelGGL(k_ens_final, dim3(groups_grid(b)), dim3(kBlock), 0, s, b);
-  if (b.controller == ODEHIP_CONTROLLER_LEARNED) {
+  // a wave per system while they fit the chip at once (eight waves a SIMD);
+  // beyond, 64 systems a wave, 16 with the network
+  if (b.n_sys <= kEnsSimds * 8) {
+    hipLaunchKernelGGL(k_ens_controller_wave, dim3(b.n_sys), dim3(64), 0, s, b);
+  } else if (b.controller == ODEHIP_CONTROLLER_LEARNED) {
     hipLaunchKernelGGL(k_ens_controller_learned, dim3((b.n_sys + 15) / 16), dim3(64), 0, s,
                        b);
   } else {

@@ -185,9 +185,6 @@ inline int split_config(int xcd, int split) {
   return -1;
 }
 
-// SIMDs of the device (256 CUs x 4): the waves one launch needs to give
-// each SIMD one.
-constexpr long kEnsSimds = 1024;
 // Tiles from which the reorderable variants keep the tuned configuration.
 constexpr long kEnsSplitAmple = 8192;
 
@@ -277,7 +274,7 @@ inline Plan plan(const Layout& L, size_t tiles_cap, int S, long trace_cap,
   p.tiles = take(tiles_cap * sizeof(EnsTile));
   p.groups_act = with_state ? take(L.groups.size() * sizeof(int2)) : p.groups;
   p.st = take(ns * sizeof(SolverState));
-  p.n_active = take(sizeof(int));
+  p.n_active = take(2 * sizeof(int));
   const size_t v = L.nv * sizeof(double);
   if (with_state) {
     p.xb0 = take(v);

@@ -45,7 +45,7 @@ struct SolverState {
   int controller;      // ODEHIP_CONTROLLER_*
   int rejects_in_row;  // consecutive rejections up to now
   int just_accepted;   // the last judged attempt was accepted
-  int pad;
+  int root_k;          // 1 + q: inv_q1 is the double nearest to 1 / root_k
 };
 
 // Arguments of the N-body RHS kernels.  Exactly one of y / (xb0, xb1, st)

@@ -14,7 +14,7 @@
 #include <cmath>
 #include <cstdint>
 
-#include "internal.hpp"
+#include "rk_device.hpp"
 
 namespace odehip {
 
@@ -158,6 +158,143 @@ __device__ inline void mlp_tile_forward(const MlpInfer* M, MlpTileLds& t) {
     for (int i = 0; i < 4; ++i) t.y[4 * kq + i] = c[i] + M->b3;
   }
   __syncthreads();
+}
+
+// One system's forward pass by one wave, row 0 of the same tile: every weight is
+// loaded up front (no load waits for an activation) and only row 0's activations
+// go through tanh, 8 of them per lane instead of 32.  The row's products and
+// sums are those of mlp_tile_forward.  `x`: the 16 normalised features, `h`: 64
+// floats, both in LDS and used by this wave alone.  The result is in lane 0.
+struct MlpRowWeights {
+  mlp_short4 w1[4], w2[4][4], w3[4];
+  float b1[4], b2[4], b3;
+};
+
+__device__ inline MlpRowWeights mlp_row_weights(const MlpInfer* M) {
+  const int lane = threadIdx.x & 63;
+  const int r = lane & 15;
+  const int kq = lane >> 4;
+  MlpRowWeights w;
+#pragma unroll
+  for (int nb = 0; nb < 4; ++nb) {
+    const int o = 16 * nb + r;
+    w.w1[nb] = *reinterpret_cast<const mlp_short4*>(&M->w1[o][4 * kq]);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+      w.w2[nb][ks] = *reinterpret_cast<const mlp_short4*>(&M->w2[o][16 * ks + 4 * kq]);
+    w.w3[nb] = *reinterpret_cast<const mlp_short4*>(&M->w3[r][16 * nb + 4 * kq]);
+    w.b1[nb] = M->b1[o];
+    w.b2[nb] = M->b2[o];
+  }
+  w.b3 = M->b3;
+  return w;
+}
+
+// Orders a wave's own LDS writes before its later reads.
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+__device__ inline float mlp_row_forward(const MlpRowWeights& w, const float* x, float* h) {
+  const int lane = threadIdx.x & 63;
+  const int r = lane & 15;
+  const int kq = lane >> 4;
+  auto operand = [&](const float* v, int k0) {  // row 0 of A, the other rows zero
+    mlp_short4 a;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      a[i] = r == 0 ? static_cast<short>(float_to_bf16(v[k0 + 4 * kq + i])) : short{0};
+    return a;
+  };
+  const mlp_float4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  float z[4];
+  wave_lds_fence();
+  const mlp_short4 a1 = operand(x, 0);
+#pragma unroll
+  for (int nb = 0; nb < 4; ++nb)
+    z[nb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a1, w.w1[nb], zero, 0, 0, 0)[0];
+#pragma unroll
+  for (int nb = 0; nb < 4; ++nb) {
+    const float t = tanhf(z[nb] + w.b1[nb]);
+    if (kq == 0) h[16 * nb + r] = t;
+  }
+  wave_lds_fence();
+  mlp_short4 a[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) a[ks] = operand(h, 16 * ks);
+#pragma unroll
+  for (int nb = 0; nb < 4; ++nb) {
+    mlp_float4 c = zero;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+      c = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[ks], w.w2[nb][ks], c, 0, 0, 0);
+    z[nb] = c[0];
+  }
+  wave_lds_fence();
+#pragma unroll
+  for (int nb = 0; nb < 4; ++nb) {
+    const float t = tanhf(z[nb] + w.b2[nb]);
+    if (kq == 0) h[16 * nb + r] = t;
+  }
+  wave_lds_fence();
+  mlp_float4 c = zero;
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks)
+    c = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(operand(h, 16 * ks), w.w3[ks], c, 0, 0, 0);
+  return c[0] + w.b3;
+}
+
+// The step ratio the network's output stands for (NaN if it is not finite).
+__device__ inline double mlp_ratio(double y) {
+  y = y < kMlpLogRatioMin ? kMlpLogRatioMin : (y > kMlpLogRatioMax ? kMlpLogRatioMax : y);
+  return std::isfinite(y) ? std::exp(y) : NAN;
+}
+
+// Feature `i` of mlp_features, normalised (0 from kMlpIn on): a wave's first 16
+// lanes take one each, so the logarithms run side by side.
+__device__ inline float mlp_feature(const MlpInfer* M, const SolverState* st, int n_particles,
+                                    int i) {
+  if (i >= kMlpIn) return 0.0f;
+  double f;
+  if (i >= 6 && i < 9) {
+    f = st->hist_acc[i - 6];
+  } else {
+    const double d0 = st->hist_dt[0];
+    double v;
+    if (i < 3) {
+      v = st->hist_err[i];
+      v = v < 1.0e-12 ? 1.0e-12 : (v > 1.0e12 ? 1.0e12 : v);
+    } else {
+      v = i == 3 ? d0 / (st->tf - st->t0) : i == 9 ? static_cast<double>(n_particles)
+                                                   : st->hist_dt[i - 3] / d0;
+    }
+    f = std::log(v);
+  }
+  const float raw = std::isfinite(f) ? static_cast<float>(f) : 0.0f;
+  return (raw - M->mean[i]) * M->inv_std[i];
+}
+
+// An attempt's end by one wave (every lane calls): judge and step on lane 0
+// (`sum` is read there), the learned controller's features and network on all
+// lanes.  `st` is this wave's alone to change; `x` (16) and `h` (64) are its LDS.
+__device__ inline void ctrl_attempt_wave(SolverState* st, const Tableau& T, double sum,
+                                         size_t n_var, double* times, double* trace,
+                                         const MlpInfer* M, int n_particles, float* x,
+                                         float* h) {
+  const int lane = threadIdx.x & 63;
+  if (st->controller != ODEHIP_CONTROLLER_LEARNED) {
+    if (lane == 0) ctrl_attempt(st, T, sum, n_var, times, trace);
+    return;
+  }
+  const MlpRowWeights w = mlp_row_weights(M);
+  bool accept = false, judged = false;
+  if (lane == 0) judged = ctrl_judge(st, T, sum, n_var, times, trace, &accept);
+  wave_lds_fence();
+  const float f = mlp_feature(M, st, n_particles, lane < 16 ? lane : 15);
+  if (lane < 16) x[lane] = f;
+  const float out = mlp_row_forward(w, x, h);
+  if (lane == 0 && judged) ctrl_step(st, accept, mlp_ratio(out));
 }
 
 // The published inference copy of a network handle (mlp_kernels.hip).

@@ -20,6 +20,7 @@
 
 #include "context.hpp"
 #include "mlp.hpp"
+#include "solo.hpp"
 
 using namespace odehip;
 
@@ -78,6 +79,7 @@ int odehip::use_tableau(odehip_context* ctx, int id) {
   for (int& next = r.resident[d]; next <= id; ++next) {
     HIP_TRY(ctx, upload_rk_tableau(next, r.tab[next]));
     HIP_TRY(ctx, upload_ens_tableau(next, r.tab[next]));
+    HIP_TRY(ctx, upload_solo_tableau(next, r.tab[next]));
   }
   return ODEHIP_OK;
 }
@@ -700,7 +702,32 @@ int odehip_rk_solve(odehip_context* ctx, int tableau, const odehip_ode* ode,
                                   opt->max_attempts, opt->fsal ? 1 : 0, s));
   HIP_TRY(ctx, enqueue_initial_step(b, s));
 
-  if (K > 0) {
+  // Small systems: whole attempts by one workgroup (solo.hpp), unless the
+  // caller says how the attempts are launched or every state is kept.
+  const bool solo = ode->rhs_kind == ODEHIP_RHS_NBODY && opt->attempts_per_launch == 0 &&
+                    ode->nbody_variant != ODEHIP_NBODY_MIXED && n_dense == 0 &&
+                    states_cap == 0 && b.n_particles <= solo_limit(S, ode->nbody_variant);
+  SoloArgs sa{};
+  if (solo) {
+    K = kSoloAttempts;
+    sa.one = EnsSys{0, b.n_particles, 0, n_groups_for(n), 0};
+    sa.st = b.st;
+    sa.xb0 = b.xb0;
+    sa.xb1 = b.xb1;
+    sa.ks = b.ks;
+    sa.kfsal = b.kfsal;
+    sa.mass = b.mass;
+    sa.atol_v = b.atol;
+    sa.rtol_v = b.rtol;
+    sa.times = b.times;
+    sa.trace = b.trace;
+    sa.trace_cap = b.trace_cap;
+    sa.mlp = b.mlp;
+    sa.eps2 = b.eps2;
+    sa.tableau = tableau;
+    sa.attempts = K;
+  }
+  if (K > 0 && !solo) {
     GraphKey key;
     key.tableau = tableau;
     key.rhs_kind = ode->rhs_kind;
@@ -756,7 +783,10 @@ int odehip_rk_solve(odehip_context* ctx, int tableau, const odehip_ode* ode,
   int slot = 0;
   bool have_prev = false;
   for (;;) {
-    if (K > 0) {
+    if (solo) {
+      HIP_TRY(ctx, launch_solo(sa, b.n_particles, ode->nbody_variant, 1, s));
+      launched += K;
+    } else if (K > 0) {
       HIP_TRY(ctx, hipGraphLaunch(ctx->exec, s));
       launched += K;
     } else {

@@ -100,7 +100,8 @@ __device__ inline void ctrl_init(SolverState* st, const Tableau& T, double t0,
   st->err = 0.0;
   st->dt_initial = 0.0;
   st->inv_q1 = 1.0 / (1.0 + q);
-  st->safety = cr_pow(0.38, (1.0 / (1.0 + q)));
+  st->root_k = 1 + q;
+  st->safety = cr_root(0.38, st->inv_q1, st->root_k);
   st->dt0 = 0.0;
   st->d1 = 0.0;
   st->err_prev = 1.0e-4;
@@ -233,7 +234,7 @@ __device__ inline void ctrl_step(SolverState* st, bool accept,
       dtnew = pi_proposal(st, scaled_error, accept);
     }
   } else {
-    dtnew = dt * st->safety / cr_pow(scaled_error, st->inv_q1);
+    dtnew = dt * st->safety / cr_root(scaled_error, st->inv_q1, st->root_k);
   }
   if (accept) st->err_prev = scaled_error < 1.0e-4 ? 1.0e-4 : scaled_error;
   const double max_step_scale = 6.0;
@@ -402,7 +403,7 @@ __device__ inline void ctrl_init_step_b(SolverState* st, const Tableau& T,
   const double m = (d1 < d2) ? d2 : d1;
   const double hi = 1.0e-6, lo = dt0 * 1.0e-3;
   const double dt1 = (m <= 1.0e-15) ? ((hi < lo) ? lo : hi)
-                                    : cr_pow(0.01 / m, (1.0 / (1.0 + p)));
+                                    : cr_root(0.01 / m, 1.0 / (1.0 + p), 1 + p);
   const double cap = 100.0 * dt0;
   const double dt = (dt1 < cap) ? dt1 : cap;
   st->dt = dt;

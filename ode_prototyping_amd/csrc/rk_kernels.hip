@@ -134,29 +134,14 @@ __global__ void k_controller(SolverState* st, const double* partials,
   ctrl_attempt(st, c_tab[st->tableau], sum, n_var, times, trace);
 }
 
-// The same with the learned controller (a tile of one system).
+// The same with the learned controller's network.
 __global__ __launch_bounds__(64) void k_controller_learned(
     SolverState* st, const double* partials, size_t n_var, double* times,
     double* trace, const MlpInfer* M, int n_particles) {
-  __shared__ MlpTileLds tile;
+  __shared__ float x[16], h[64];
   if (st->done) return;  // read by every thread before thread 0 writes it
   const double sum = fold_partials_block(partials, st->n_groups);
-  bool accept = false, judged = false;
-  float raw[kMlpIn];
-  for (int i = 0; i < kMlpIn; ++i) raw[i] = 0.0f;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    judged = ctrl_judge(st, c_tab[st->tableau], sum, n_var, times, trace, &accept);
-    if (judged) mlp_features(st, n_particles, raw);
-  }
-  if (threadIdx.x < 16) mlp_tile_set_row(M, tile, threadIdx.x, raw);
-  __syncthreads();
-  mlp_tile_forward(M, tile);
-  if (threadIdx.x == 0 && judged) {
-    double y = tile.y[0];
-    y = y < kMlpLogRatioMin ? kMlpLogRatioMin : (y > kMlpLogRatioMax ? kMlpLogRatioMax : y);
-    ctrl_step(st, accept, std::isfinite(y) ? std::exp(y) : NAN);
-  }
+  ctrl_attempt_wave(st, c_tab[st->tableau], sum, n_var, times, trace, M, n_particles, x, h);
 }
 
 // ------------------------------------------------------ initial step -------

@@ -1,0 +1,83 @@
+// One-workgroup solves of small systems (solo_kernels.hip): arguments, LDS use
+// and the sizes they take.
+#pragma once
+
+#include <algorithm>
+
+#include "ensemble.hpp"
+
+namespace odehip {
+
+struct MlpInfer;
+
+constexpr int kSoloWaves = 16;    // at most, per workgroup
+constexpr int kSoloTerms = 4;     // exact: partners per wave and block
+constexpr int kSoloMaxN = 320;    // fast, mixed: 192 threads per 64 targets
+constexpr int kSoloExactN = 128;  // sizes up to which it is the faster form
+constexpr int kSoloSumN = 256;
+constexpr int kSoloAttempts = 64; // per launch
+constexpr int kSoloMaxQuads = 4 * ((6 * kSoloMaxN + ODEHIP_REDUCE_GROUP - 1) / ODEHIP_REDUCE_GROUP);
+// LDS of a CU less the kernel's static use and some to spare.
+constexpr int kSoloLdsDoubles = (160 * 1024 - 2048) / 8;
+
+struct SoloArgs {
+  const EnsSys* sys;   // systems' table, or null: the one system `one`
+  const int* list;     // system per workgroup, or null (with sys null)
+  EnsSys one;
+  SolverState* st;
+  double* xb0;
+  double* xb1;
+  double* ks;          // its first stage vector holds a kept k1 between launches
+  double* kfsal;
+  const double* mass;
+  const double* atol_v;  // per element (one system), or null: atol, rtol
+  const double* rtol_v;
+  double atol, rtol;
+  double* times;
+  double* trace;
+  long trace_cap;      // per system of `trace`
+  const MlpInfer* mlp;
+  int* n_active;       // counted down as systems end, or null
+  double eps2;
+  double near_c;
+  int tableau;
+  int attempts;        // of this launch, per system
+  int lds_doubles;     // set by launch_solo
+};
+
+// LDS of a system of n bodies: state, stage input, S stage vectors, masses and
+// the partial sums of the waves.
+__host__ __device__ inline int solo_lds_doubles(int n, int S, int variant, int waves) {
+  const int sums = variant == ODEHIP_NBODY_EXACT ? 3 * 64 * kSoloTerms : 192;
+  return (S + 2) * 6 * n + ((n + 1) & ~1) + waves * sums;
+}
+
+// Waves of the workgroup for systems of up to n bodies, 0 if they do not fit.
+inline int solo_waves(int n, int S, int variant) {
+  if (n < 1 || n > kSoloMaxN) return 0;
+  for (int w : {kSoloWaves, 8}) {
+    // fast, mixed: a thread per target and coordinate; more waves than units
+    // of 64 targets and 32 partners would only wait
+    if (variant != ODEHIP_NBODY_EXACT) {
+      if (w == kSoloWaves && n <= 128) continue;
+      if (192 * ((n + 63) / 64) > 64 * w) continue;
+    }
+    if (solo_lds_doubles(n, S, variant, w) <= kSoloLdsDoubles) return w;
+  }
+  return 0;
+}
+
+// Bodies up to which a solve is one workgroup's.
+inline int solo_limit(int S, int variant) {
+  const int want = variant == ODEHIP_NBODY_EXACT ? kSoloExactN : kSoloSumN;
+  for (int n = want; n > 0; --n)
+    if (solo_waves(n, S, variant) > 0) return n;
+  return 0;
+}
+
+// One launch: `blocks` systems of at most n_max bodies.
+hipError_t launch_solo(const SoloArgs& a, int n_max, int variant, unsigned blocks,
+                       hipStream_t s);
+hipError_t upload_solo_tableau(int id, const Tableau& T);
+
+}  // namespace odehip
