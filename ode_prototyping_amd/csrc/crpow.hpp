@@ -176,13 +176,13 @@ ODEHIP_HD inline double cr_pow(double x, double y) {
 // cr_pow(x, y) (correctly rounded but within ~2^-98 of a tie), by a shorter way
 // than logarithm and exponential: the controller runs on one lane while
 // everything else waits, and cr_pow's two series take it 7 us of dependent
-// arithmetic on MI355X, this under 1.
+// arithmetic on MI355X, this about 1.
 //
 // r, a k-th root of x to a few ulp, comes from FP32 log2 / exp2 and Newton
-// steps.  With P = r^k in double-double and s = (x - P) / P (P.hi and x are
-// neighbours, so the difference is exact), x^(1/k) = r (1 + s)^(1/k), and
-// y = 1/k + d with d known exactly from the fma residual, so x^y is
-// r (1 + s/k - (k-1) s^2 / (2 k^2)) (1 + z + z^2/2), z = d log x: one rounding
+// steps.  With P = r^k in double-double and s = (x - P) / x (P.hi and x are
+// neighbours, so the difference is exact), x^(1/k) = r (1 - s)^(-1/k), and
+// x^y = x^(1/k) x^d with d = y - 1/k known exactly from the fma residual, so x^y is
+// r (1 + s/k + (1/k + 1) s^2 / (2 k)) (1 + z + z^2/2), z = d log x: one rounding
 // of r plus a correction of some 2^-51 r.
 ODEHIP_HD inline double cr_root(double x, double y, int k) {
   using namespace crpow_detail;
@@ -191,20 +191,22 @@ ODEHIP_HD inline double cr_root(double x, double y, int k) {
   const uint64_t bits = to_bits(x);
   const int e = static_cast<int>(bits >> 52) - 1023;
   const double m = from_bits((bits & 0x000fffffffffffffULL) | 0x3ff0000000000000ULL);
-  const double kd = k;
-  const double l = (static_cast<double>(e) + static_cast<double>(log2f(static_cast<float>(m)))) / kd;
+  const double ix = 1.0 / x;
+  const double d = std::fma(y, static_cast<double>(k), -1.0) * y;  // y - 1/k
+  const double z = d != 0.0 ? d * std::log(x) : 0.0;
+  const double l = (static_cast<double>(e) + static_cast<double>(log2f(static_cast<float>(m)))) * y;
   const double n = std::nearbyint(l);
-  double r = scale2(static_cast<double>(exp2f(static_cast<float>(l - n))), static_cast<int>(n));
+  double r = static_cast<double>(exp2f(static_cast<float>(l - n))) *
+             from_bits(static_cast<uint64_t>(static_cast<int>(n) + 1023) << 52);
   for (int it = 0; it < 2; ++it) {  // 1e-6 -> 1e-11 -> rounding
     double p = r;
     for (int i = 1; i < k; ++i) p *= r;
-    r += r * ((x - p) / (kd * p));
+    r += r * (((x - p) * ix) * y);
   }
   dd p{r, 0.0};
   for (int i = 1; i < k; ++i) p = mul_d(p, r);
-  const double s = ((x - p.hi) - p.lo) / p.hi;
-  const double c = (s / kd) * (1.0 - s * ((kd - 1.0) / (2.0 * kd)));
-  const double z = std::fma(y, kd, -1.0) / kd * std::log(x);
+  const double s = ((x - p.hi) - p.lo) * ix;
+  const double c = (s * y) * (1.0 + s * (0.5 * y + 0.5));
   const double w = z + 0.5 * z * z;
   return r + r * (c + w + c * w);
 }

@@ -17,6 +17,127 @@ namespace odehip {
 constexpr int kEnsGroup = 32;
 static_assert(kEnsChunk % kEnsGroup == 0, "chunks are whole groups");
 
+// U partners of one lane, coordinates c and masses m already loaded: the terms of
+// fast_term (nbody_terms.hpp) step by step for all of them, so that a wave that
+// has its SIMD to itself does not wait out each partner's chain of a dozen
+// instructions (one partner after the other took 200 cycles each), then their sums
+// in increasing j.
+template <bool kMass, bool kGuard, int U>
+__device__ __forceinline__ void fast_terms(const double (&c)[3 * U], const double (&m)[U], int j,
+                                           int i, double xi, double yi, double zi, double eps2,
+                                           double& ax, double& ay, double& az) {
+  double dx[U], dy[U], dz[U], r2[U], y0[U], y2[U], e[U], w[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    dx[u] = c[3 * u] - xi;
+    dy[u] = c[3 * u + 1] - yi;
+    dz[u] = c[3 * u + 2] - zi;
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    r2[u] = __builtin_fma(dx[u], dx[u],
+                          __builtin_fma(dy[u], dy[u], __builtin_fma(dz[u], dz[u], eps2)));
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < U; ++u) y0[u] = __builtin_amdgcn_rsq(r2[u]);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < U; ++u) y2[u] = y0[u] * y0[u];
+#pragma unroll
+  for (int u = 0; u < U; ++u) e[u] = __builtin_fma(-r2[u], y2[u], 1.0);
+#pragma unroll
+  for (int u = 0; u < U; ++u) y0[u] = y2[u] * (kMass ? y0[u] * m[u] : y0[u]);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < U; ++u) e[u] = e[u] * __builtin_fma(e[u], 1.25, 1.0);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    w[u] = __builtin_fma(y0[u] * e[u], 1.5, y0[u]);
+    if (kGuard) w[u] = j + u == i ? 0.0 : w[u];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    ax = __builtin_fma(dx[u], w[u], ax);
+    ay = __builtin_fma(dy[u], w[u], ay);
+    az = __builtin_fma(dz[u], w[u], az);
+  }
+}
+
+// The same for mixed_term_fp32.
+template <bool kMass, bool kGuard, int U>
+__device__ __forceinline__ void mixed_terms(const double (&c)[3 * U], const double (&m)[U], int j,
+                                            int i, double xi, double yi, double zi, float eps2f,
+                                            float& fx, float& fy, float& fz) {
+  float dx[U], dy[U], dz[U], r2[U], w[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    dx[u] = static_cast<float>(c[3 * u] - xi);
+    dy[u] = static_cast<float>(c[3 * u + 1] - yi);
+    dz[u] = static_cast<float>(c[3 * u + 2] - zi);
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    r2[u] = __builtin_fmaf(dx[u], dx[u],
+                           __builtin_fmaf(dy[u], dy[u], __builtin_fmaf(dz[u], dz[u], eps2f)));
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const float rinv = __builtin_amdgcn_rsqf(r2[u]);
+    w[u] = (rinv * rinv) * rinv;
+    if (kMass) w[u] *= static_cast<float>(m[u]);
+    if (kGuard) w[u] = j + u == i ? 0.0f : w[u];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    fx = __builtin_fmaf(dx[u], w[u], fx);
+    fy = __builtin_fmaf(dy[u], w[u], fy);
+    fz = __builtin_fmaf(dz[u], w[u], fz);
+  }
+}
+
+// The sum over one group of `count` partners from j0 on, in LDS at p (3 doubles
+// each) with masses at m; p, m, j0 and count may differ between the lanes.
+template <int kVariant, bool kMass, bool kGuard>
+__device__ __forceinline__ void lds_group(const __attribute__((address_space(3))) double* p,
+                                          const __attribute__((address_space(3))) double* m,
+                                          int j0, int count, int i, double xi, double yi,
+                                          double zi, double eps2, double& ax, double& ay,
+                                          double& az) {
+  constexpr int U = 4;
+  float fx = 0.0f, fy = 0.0f, fz = 0.0f;
+  ax = ay = az = 0.0;
+  const float eps2f = static_cast<float>(eps2);
+  int q = 0;
+  for (; q + U <= count; q += U) {
+    double c[3 * U], ms[U];
+#pragma unroll
+    for (int v = 0; v < 3 * U; ++v) c[v] = p[3 * q + v];
+#pragma unroll
+    for (int u = 0; u < U; ++u) ms[u] = kMass ? m[q + u] : 1.0;
+    if constexpr (kVariant == ODEHIP_NBODY_FAST)
+      fast_terms<kMass, kGuard, U>(c, ms, j0 + q, i, xi, yi, zi, eps2, ax, ay, az);
+    else
+      mixed_terms<kMass, kGuard, U>(c, ms, j0 + q, i, xi, yi, zi, eps2f, fx, fy, fz);
+  }
+  for (; q < count; ++q) {
+    const double mj = kMass ? m[q] : 1.0;
+    if constexpr (kVariant == ODEHIP_NBODY_FAST)
+      fast_term<kMass, kGuard>(p[3 * q], p[3 * q + 1], p[3 * q + 2], mj, j0 + q, i, xi, yi, zi,
+                               eps2, ax, ay, az);
+    else
+      mixed_term_fp32<kMass, kGuard>(p[3 * q], p[3 * q + 1], p[3 * q + 2],
+                                     static_cast<float>(mj), j0 + q, i, xi, yi, zi, eps2f, fx,
+                                     fy, fz);
+  }
+  if constexpr (kVariant != ODEHIP_NBODY_FAST) {
+    ax = static_cast<double>(fx);
+    ay = static_cast<double>(fy);
+    az = static_cast<double>(fz);
+  }
+}
+
 // P: pointer to the partners' coordinates and masses (scalar loads or LDS).
 
 // fast: partners j0 .. j1 - 1 (of one group) summed into p* (which the caller

@@ -36,6 +36,7 @@ struct EnsBufs {
   double* xb1;
   double* ks;
   double* ytmp;
+  double* ytmp2;  // (the initial step's sc0)
   double* kfsal;
   double* sc0;
   double* partA;
@@ -89,6 +90,9 @@ constexpr int kEnsChunk = 128;
 // SIMDs of the device (256 CUs x 4): the waves one launch needs to give
 // each SIMD one.
 constexpr long kEnsSimds = 1024;
+// 64-target tiles up to which a shared tile of the fast and mixed sums is split
+// into 16-target workgroups.
+constexpr int kEnsFineTiles = 512;
 // Waves that give each of the 1024 SIMDs (256 CUs x 4) four, the depth that
 // hides the RHS arithmetic's latency.
 constexpr long kEnsFillWaves = 4096;
@@ -96,7 +100,7 @@ constexpr long kEnsFillWaves = 4096;
 // y == null: each system's current x0 buffer (solve); else a packed state.
 // st == null in b: plain evaluation of every system.
 hipError_t ens_launch_rhs(const EnsBufs& b, const double* y, double* k,
-                          int stage0, hipStream_t s);
+                          int stage0, hipStream_t s, const NextStage& next = NextStage{});
 hipError_t ens_enqueue_init(const EnsBufs& b, const double* x_in, double t0,
                             double tf, long max_acc, long max_att, int fsal,
                             int controller, hipStream_t s);

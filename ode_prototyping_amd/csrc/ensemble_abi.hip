@@ -150,6 +150,7 @@ EnsBufs make_bufs(EnsembleWorkspace* w, const Plan& p, const Layout& L,
     b.ks = reinterpret_cast<double*>(d + p.ks);
     b.ytmp = reinterpret_cast<double*>(d + p.ytmp);
     b.kfsal = reinterpret_cast<double*>(d + p.kfsal);
+    b.ytmp2 = reinterpret_cast<double*>(d + p.sc0);
     b.sc0 = reinterpret_cast<double*>(d + p.sc0);
     b.partA = reinterpret_cast<double*>(d + p.partA);
     b.partB = reinterpret_cast<double*>(d + p.partB);
@@ -379,7 +380,7 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
   std::vector<char> live(L.sys.size(), 1);
   int solo_max = 0;
   if (opt->tile_config == ODEHIP_ENS_TILE_AUTO && n_dense == 0) {
-    b.solo_n = solo_limit(S, nbody_variant);
+    b.solo_n = solo_limit(S, nbody_variant, b.mlp != nullptr);
     for (size_t k = 0; k < L.sys.size(); ++k) {
       if (L.sys[k].n > b.solo_n) continue;
       solo.push_back(static_cast<int>(k));

@@ -45,10 +45,50 @@ __device__ inline uniform_ptr as_uniform(const double* p) {
 
 // ------------------------------------------------------------- RHS tiles --
 
+// Where a system's right-hand side goes: its stage vector, and (in a solve) the
+// next stage's input (L: next_stage).
+template <int L>
+struct EnsSink {
+  double* k;  // the system's part of the stage vector
+  const NextStage* next;
+  const double* x0;  // with next->y: the packed current state
+  double dt;
+  size_t nv, off;  // packed length, the system's first element
+
+  __device__ void put(long e, double v) const {
+    k[e] = v;
+    if (next->y) next_stage<L>(*next, e_tab[next->tab], nv, off + e, v, x0[off + e], dt);
+  }
+};
+
+template <int L>
+__device__ inline EnsSink<L> ens_sink(const EnsBufs& b, const NextStage& next,
+                                   const SolverState* st, double* k_out, const EnsSys& sy) {
+  EnsSink<L> o{k_out + sy.eoff, &next, nullptr, 0.0, b.nv, static_cast<size_t>(sy.eoff)};
+  if (next.y) {
+    o.x0 = st->cur ? b.xb1 : b.xb0;
+    o.dt = st->dt;
+  }
+  return o;
+}
+
+// An attempt whose k1 is the FSAL copy (or kept in place after a rejection):
+// the tile's part of it by one wave.
+template <int L>
+__device__ inline void tile_reuse_k1(const EnsBufs& b, const SolverState* st, const EnsSink<L>& out,
+                                     int n, int i0, int targets) {
+  const int lane = threadIdx.x & 63;
+  const long lim = 3L * n, end = min(lim, 3L * (i0 + targets));
+  const double* src = st->k1_valid == 1 ? b.kfsal + out.off : out.k;
+  for (long e = 3L * i0 + lane; e < end; e += 64) {
+    out.put(e, src[e]);
+    out.put(lim + e, src[lim + e]);
+  }
+}
+
 // dxdt[0:3n] = x[3n:6n] for the tile's targets (NBodyODE.hpp:51-56).
-template <int TPL>
-__device__ inline void tile_velocities(const double* __restrict__ y,
-                                       double* __restrict__ k, int n,
+template <int TPL, int L>
+__device__ inline void tile_velocities(const double* __restrict__ y, const EnsSink<L>& out, int n,
                                        int i0) {
   const int lane = threadIdx.x & 63;
   const long lim = 3L * n;
@@ -56,22 +96,21 @@ __device__ inline void tile_velocities(const double* __restrict__ y,
 #pragma unroll
   for (int c = 0; c < 3 * TPL; ++c) {
     const long e = base + 64 * c + lane;
-    if (e < lim) k[e] = y[lim + e];
+    if (e < lim) out.put(e, y[lim + e]);
   }
 }
 
-template <int TPL>
-__device__ inline void tile_store(double* __restrict__ k, int n, int i0,
-                                  const double* ax, const double* ay,
-                                  const double* az) {
+template <int TPL, int L>
+__device__ inline void tile_store(const EnsSink<L>& out, int n, int i0, const double* ax,
+                                  const double* ay, const double* az) {
   const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int t = 0; t < TPL; ++t) {
     const int i = i0 + 64 * t + lane;
     if (i < n) {
-      k[3L * n + 3 * i] = ax[t];
-      k[3L * n + 3 * i + 1] = ay[t];
-      k[3L * n + 3 * i + 2] = az[t];
+      out.put(3L * n + 3 * i, ax[t]);
+      out.put(3L * n + 3 * i + 1, ay[t]);
+      out.put(3L * n + 3 * i + 2, az[t]);
     }
   }
 }
@@ -153,7 +192,7 @@ __device__ __forceinline__ void exact_sweep(uniform_ptr yu, uniform_ptr mu, int 
 template <bool kMass, bool kSharedRcp, int TPL>
 __device__ __forceinline__ void exact_tile(const double* __restrict__ y,
                                            const double* __restrict__ mass,
-                                           double* __restrict__ k, int n, int i0,
+                                           const EnsSink<kStageLoadsLean>& out, int n, int i0,
                                            double eps2) {
   const int lane = threadIdx.x & 63;
   const uniform_ptr yu = as_uniform(y);
@@ -186,8 +225,8 @@ __device__ __forceinline__ void exact_tile(const double* __restrict__ y,
     exact_sweep<kMass, false, true, TPL>(yu, mu, i0, s1, ic, xi, yi, zi, eps2, ax, ay, az);
     exact_sweep<kMass, false, false, TPL>(yu, mu, s1, n, ic, xi, yi, zi, eps2, ax, ay, az);
   }
-  tile_store<TPL>(k, n, i0, ax, ay, az);
-  tile_velocities<TPL>(y, k, n, i0);
+  tile_store<TPL>(out, n, i0, ax, ay, az);
+  tile_velocities<TPL>(y, out, n, i0);
 }
 
 // The targets of a tile: coordinates of i0 + 64 t + lane (lanes past n
@@ -210,7 +249,7 @@ __device__ inline void tile_targets(const double* __restrict__ y, int n, int i0,
 template <bool kMass, bool kGuard, int TPL>
 __device__ inline void fast_tile(const double* __restrict__ y,
                                  const double* __restrict__ mass,
-                                 double* __restrict__ k, int n, int i0,
+                                 const EnsSink<kStageLoadsLean>& out, int n, int i0,
                                  double eps2, double scale) {
   const uniform_ptr yu = as_uniform(y);
   const uniform_ptr mu = as_uniform(mass);
@@ -238,14 +277,14 @@ __device__ inline void fast_tile(const double* __restrict__ y,
     ay[t] *= scale;
     az[t] *= scale;
   }
-  tile_store<TPL>(k, n, i0, ax, ay, az);
-  tile_velocities<TPL>(y, k, n, i0);
+  tile_store<TPL>(out, n, i0, ax, ay, az);
+  tile_velocities<TPL>(y, out, n, i0);
 }
 
 template <bool kMass, bool kGuard, bool kNear, int TPL>
 __device__ inline void mixed_tile(const double* __restrict__ y,
                                   const double* __restrict__ mass,
-                                  double* __restrict__ k, int n, int i0,
+                                  const EnsSink<kStageLoadsLean>& out, int n, int i0,
                                   double eps2, float near2, double scale) {
   const uniform_ptr yu = as_uniform(y);
   const uniform_ptr mu = as_uniform(mass);
@@ -273,8 +312,8 @@ __device__ inline void mixed_tile(const double* __restrict__ y,
     ay[t] *= scale;
     az[t] *= scale;
   }
-  tile_store<TPL>(k, n, i0, ax, ay, az);
-  tile_velocities<TPL>(y, k, n, i0);
+  tile_store<TPL>(out, n, i0, ax, ay, az);
+  tile_velocities<TPL>(y, out, n, i0);
 }
 
 // The system's common mass when all its masses are equal (finite, nonzero),
@@ -291,7 +330,8 @@ template <int kVariant, bool kMass, bool kSpecial, bool kNear, int WPB>
 __global__ __launch_bounds__(64 * WPB) void k_ens_rhs(EnsBufs b,
                                                       const double* y_in,
                                                       double* k_out,
-                                                      int stage0) {
+                                                      int stage0,
+                                                                 NextStage next) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int slot = blockIdx.x * WPB + wave;
   if (slot >= b.n_tiles) return;
@@ -304,30 +344,18 @@ __global__ __launch_bounds__(64 * WPB) void k_ens_rhs(EnsBufs b,
   const EnsSys sy = b.sys[tile.sys];
   const int n = sy.n;
   const int tpl = n >= b.tpl2_min_n ? 2 : 1;
-  double* k = k_out + sy.eoff;
+  const auto out = ens_sink<kStageLoadsLean>(b, next, st, k_out, sy);
   if (st && stage0 == 1 && st->k1_valid) {
-    // k1 of this attempt is the FSAL copy (or kept after a rejection)
-    if (st->k1_valid == 1) {
-      const int lane = threadIdx.x & 63;
-      const long lim = 3L * n;
-      const double* src = b.kfsal + sy.eoff;
-      for (int c = 0; c < 3 * tpl; ++c) {
-        const long e = 3L * tile.i0 + 64 * c + lane;
-        if (e < lim) {
-          k[e] = src[e];
-          k[lim + e] = src[lim + e];
-        }
-      }
-    }
+    tile_reuse_k1(b, st, out, n, tile.i0, 64 * tpl);
     return;
   }
   const double* y = (y_in ? y_in : (st->cur ? b.xb1 : b.xb0)) + sy.eoff;
   const double* m = kMass ? b.mass + sy.eoff / 6 : nullptr;
   if (kVariant == ODEHIP_NBODY_EXACT) {
     if (tpl == 2)
-      exact_tile<kMass, kSpecial, 2>(y, m, k, n, tile.i0, b.eps2);
+      exact_tile<kMass, kSpecial, 2>(y, m, out, n, tile.i0, b.eps2);
     else
-      exact_tile<kMass, kSpecial, 1>(y, m, k, n, tile.i0, b.eps2);
+      exact_tile<kMass, kSpecial, 1>(y, m, out, n, tile.i0, b.eps2);
   } else {
     // equal masses: unit-mass terms, each finished sum scaled once
     const double m_uni = kMass ? system_uniform_mass(st, m, n) : 0.0;
@@ -336,27 +364,27 @@ __global__ __launch_bounds__(64 * WPB) void k_ens_rhs(EnsBufs b,
     if (kVariant == ODEHIP_NBODY_FAST) {
       if (per_term) {
         if (tpl == 2)
-          fast_tile<true, kSpecial, 2>(y, m, k, n, tile.i0, b.eps2, 1.0);
+          fast_tile<true, kSpecial, 2>(y, m, out, n, tile.i0, b.eps2, 1.0);
         else
-          fast_tile<true, kSpecial, 1>(y, m, k, n, tile.i0, b.eps2, 1.0);
+          fast_tile<true, kSpecial, 1>(y, m, out, n, tile.i0, b.eps2, 1.0);
       } else {
         if (tpl == 2)
-          fast_tile<false, kSpecial, 2>(y, m, k, n, tile.i0, b.eps2, scale);
+          fast_tile<false, kSpecial, 2>(y, m, out, n, tile.i0, b.eps2, scale);
         else
-          fast_tile<false, kSpecial, 1>(y, m, k, n, tile.i0, b.eps2, scale);
+          fast_tile<false, kSpecial, 1>(y, m, out, n, tile.i0, b.eps2, scale);
       }
     } else {
       const float near2 = kNear ? mixed_near2(b.near_c, n) : 0.0f;
       if (per_term) {
         if (tpl == 2)
-          mixed_tile<true, kSpecial, kNear, 2>(y, m, k, n, tile.i0, b.eps2, near2, 1.0);
+          mixed_tile<true, kSpecial, kNear, 2>(y, m, out, n, tile.i0, b.eps2, near2, 1.0);
         else
-          mixed_tile<true, kSpecial, kNear, 1>(y, m, k, n, tile.i0, b.eps2, near2, 1.0);
+          mixed_tile<true, kSpecial, kNear, 1>(y, m, out, n, tile.i0, b.eps2, near2, 1.0);
       } else {
         if (tpl == 2)
-          mixed_tile<false, kSpecial, kNear, 2>(y, m, k, n, tile.i0, b.eps2, near2, scale);
+          mixed_tile<false, kSpecial, kNear, 2>(y, m, out, n, tile.i0, b.eps2, near2, scale);
         else
-          mixed_tile<false, kSpecial, kNear, 1>(y, m, k, n, tile.i0, b.eps2, near2, scale);
+          mixed_tile<false, kSpecial, kNear, 1>(y, m, out, n, tile.i0, b.eps2, near2, scale);
       }
     }
   }
@@ -373,7 +401,8 @@ template <bool kMass, bool kSharedRcp, int C>
 __global__ __launch_bounds__(64 * C) void k_ens_rhs_exact_split(EnsBufs b,
                                                                 const double* y_in,
                                                                 double* k_out,
-                                                                int stage0) {
+                                                                int stage0,
+                                                                 NextStage next) {
   constexpr int B = C * kExactP;
   __shared__ double term[3][B][64];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -386,19 +415,9 @@ __global__ __launch_bounds__(64 * C) void k_ens_rhs_exact_split(EnsBufs b,
   if (st && (stage0 == 2 ? st->dense_go == 0 : st->done)) return;
   const EnsSys sy = b.sys[tile.sys];
   const int n = sy.n;
-  double* k = k_out + sy.eoff;
+  const auto out = ens_sink<kStageLoads>(b, next, st, k_out, sy);
   if (st && stage0 == 1 && st->k1_valid) {
-    if (st->k1_valid == 1 && wave == 0) {
-      const long lim = 3L * n;
-      const double* src = b.kfsal + sy.eoff;
-      for (int c = 0; c < 3; ++c) {
-        const long e = 3L * tile.i0 + 64 * c + lane;
-        if (e < lim) {
-          k[e] = src[e];
-          k[lim + e] = src[lim + e];
-        }
-      }
-    }
+    if (wave == 0) tile_reuse_k1(b, st, out, n, tile.i0, 64);
     return;
   }
   const double* y = (y_in ? y_in : (st->cur ? b.xb1 : b.xb0)) + sy.eoff;
@@ -462,12 +481,12 @@ __global__ __launch_bounds__(64 * C) void k_ens_rhs_exact_split(EnsBufs b,
   }
   const int i = i0 + lane;
   if (i < n) {
-    if (wave < 3) k[3L * n + 3 * i + wave] = acc0;
+    if (wave < 3) out.put(3L * n + 3 * i + wave, acc0);
     if constexpr (C == 2) {
-      if (wave == 0) k[3L * n + 3 * i + 2] = acc1;
+      if (wave == 0) out.put(3L * n + 3 * i + 2, acc1);
     }
   }
-  if (wave == C - 1) tile_velocities<1>(y, k, n, i0);
+  if (wave == C - 1) tile_velocities<1>(y, out, n, i0);
 }
 
 // The reorderable variants with one tile per workgroup of C waves: wave w
@@ -480,7 +499,8 @@ template <int kVariant, bool kMass, bool kSpecial, bool kNear, int C>
 __global__ __launch_bounds__(64 * C) void k_ens_rhs_split(EnsBufs b,
                                                           const double* y_in,
                                                           double* k_out,
-                                                          int stage0) {
+                                                          int stage0,
+                                                                 NextStage next) {
   static_assert(kVariant != ODEHIP_NBODY_EXACT, "the exact order is sequential");
   __shared__ double part[C][3][64];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -493,19 +513,9 @@ __global__ __launch_bounds__(64 * C) void k_ens_rhs_split(EnsBufs b,
   if (st && (stage0 == 2 ? st->dense_go == 0 : st->done)) return;
   const EnsSys sy = b.sys[tile.sys];
   const int n = sy.n;
-  double* k = k_out + sy.eoff;
+  const auto out = ens_sink<kStageLoads>(b, next, st, k_out, sy);
   if (st && stage0 == 1 && st->k1_valid) {
-    if (st->k1_valid == 1 && wave == 0) {
-      const long lim = 3L * n;
-      const double* src = b.kfsal + sy.eoff;
-      for (int c = 0; c < 3; ++c) {
-        const long e = 3L * tile.i0 + 64 * c + lane;
-        if (e < lim) {
-          k[e] = src[e];
-          k[lim + e] = src[lim + e];
-        }
-      }
-    }
+    if (wave == 0) tile_reuse_k1(b, st, out, n, tile.i0, 64);
     return;
   }
   const double* y = (y_in ? y_in : (st->cur ? b.xb1 : b.xb0)) + sy.eoff;
@@ -564,9 +574,114 @@ __global__ __launch_bounds__(64 * C) void k_ens_rhs_split(EnsBufs b,
     ax *= scale;
     ay *= scale;
     az *= scale;
-    tile_store<1>(k, n, tile.i0, &ax, &ay, &az);
+    tile_store<1>(out, n, tile.i0, &ax, &ay, &az);
   }
-  if (wave == C - 1) tile_velocities<1>(y, k, n, tile.i0);
+  if (wave == C - 1) tile_velocities<1>(y, out, n, tile.i0);
+}
+
+// The reorderable variants when the running systems' 64-target tiles would not
+// fill the chip: a workgroup takes 16 of a tile's targets (blockIdx.y: which), a
+// lane one target and one of kFineSlots groups of partners at a time, so a
+// launch spreads over four times the CUs and a system's longest walk is a
+// quarter.  Partners go through LDS (the lanes of a wave read kFineSlots different
+// ones; the groups' stride keeps those reads off each other's banks); the groups'
+// sums are added in order, chunk by chunk, as everywhere.
+constexpr int kFineTargets = 16;
+constexpr int kFineSlots = 64 / kFineTargets;
+constexpr int kFineWaves = 8;
+constexpr int kFineGroups = kFineWaves * kFineSlots;     // groups per round
+constexpr int kFineStride = 3 * kEnsGroup + 2;           // doubles per group
+
+template <int kVariant, bool kMass, bool kSpecial>
+__global__ __launch_bounds__(64 * kFineWaves) void k_ens_rhs_fine(EnsBufs b, const double* y_in,
+                                                                  double* k_out, int stage0,
+                                                                  NextStage next) {
+  static_assert(kVariant != ODEHIP_NBODY_EXACT, "the exact order is sequential");
+  constexpr int T = kFineTargets;
+  __shared__ __attribute__((aligned(16))) double pos_[kFineGroups * kFineStride];
+  __shared__ double mass_[kMass ? kFineGroups * (kEnsGroup + 1) : 1];
+  __shared__ double part[kFineGroups][3 * T];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  // every return up to the rounds is uniform over the workgroup
+  if (static_cast<int>(blockIdx.x) >= b.n_tiles) return;
+  const EnsTile tile = b.tiles[blockIdx.x];
+  if (tile.sys < 0 || tile.sys >= b.n_sys) return;
+  const EnsSys sy = b.sys[tile.sys];
+  const int n = sy.n, i0 = tile.i0 + T * static_cast<int>(blockIdx.y);
+  if (i0 >= n) return;
+  const SolverState* st = b.st ? b.st + tile.sys : nullptr;
+  if (st && (stage0 == 2 ? st->dense_go == 0 : st->done)) return;
+  const auto out = ens_sink<kStageLoads>(b, next, st, k_out, sy);
+  if (st && stage0 == 1 && st->k1_valid) {
+    if (wave == 0) tile_reuse_k1(b, st, out, n, i0, T);
+    return;
+  }
+  const double* y = (y_in ? y_in : (st->cur ? b.xb1 : b.xb0)) + sy.eoff;
+  const double* m = kMass ? b.mass + sy.eoff / 6 : nullptr;
+  // equal masses: unit-mass terms, each finished sum scaled once (as k_ens_rhs)
+  const double m_uni = kMass ? system_uniform_mass(st, m, n) : 0.0;
+  const bool per_term = kMass && m_uni == 0.0;
+  const double scale = per_term || !kMass ? 1.0 : m_uni;
+  const int slot = lane / T, t = lane % T;
+  const int i = min(i0 + t, n - 1);
+  const double xi = y[3 * i], yi = y[3 * i + 1], zi = y[3 * i + 2];
+  // a thread's velocity element, written at the end
+  const int f = threadIdx.x;  // 0 .. 3T - 1: accelerations; 3T .. 6T - 1: velocities
+  const long ve = 3L * i0 + f - 3 * T;
+  const bool has_v = f >= 3 * T && f < 6 * T && ve < 3L * n;
+  const double vel = has_v ? y[3L * n + ve] : 0.0;
+  auto* pos = (__attribute__((address_space(3))) double*)pos_;
+  auto* mass = (__attribute__((address_space(3))) double*)mass_;
+  constexpr int kRound = kFineGroups * kEnsGroup;  // partners
+  double acc = 0.0, chunk = 0.0;
+  for (int r0 = 0; r0 < n; r0 += kRound) {
+    const int cnt = min(kRound, n - r0);
+    for (int e = threadIdx.x; e < 3 * cnt; e += 64 * kFineWaves)
+      pos[e / (3 * kEnsGroup) * kFineStride + e % (3 * kEnsGroup)] = y[3 * r0 + e];
+    if (per_term)
+      for (int e = threadIdx.x; e < cnt; e += 64 * kFineWaves)
+        mass[e / kEnsGroup * (kEnsGroup + 1) + e % kEnsGroup] = m[r0 + e];
+    __syncthreads();
+    const int g = wave * kFineSlots + slot;
+    const int have = min(kEnsGroup, cnt - g * kEnsGroup);
+    if (have > 0) {
+      const int j0 = r0 + g * kEnsGroup;
+      double sx, sy_, sz;
+      if (kMass && per_term)
+        lds_group<kVariant, true, kSpecial>(pos + g * kFineStride, mass + g * (kEnsGroup + 1), j0,
+                                            have, i, xi, yi, zi, b.eps2, sx, sy_, sz);
+      else
+        lds_group<kVariant, false, kSpecial>(pos + g * kFineStride, mass, j0, have, i, xi, yi, zi,
+                                             b.eps2, sx, sy_, sz);
+      part[g][t] = sx;
+      part[g][T + t] = sy_;
+      part[g][2 * T + t] = sz;
+    }
+    __syncthreads();
+    if (f < 3 * T) {
+      const int groups = (cnt + kEnsGroup - 1) / kEnsGroup;
+      constexpr int kPer = kEnsChunk / kEnsGroup;
+      int q = 0;
+      for (; q + kPer <= groups; q += kPer) {
+        double v[kPer];
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) v[u] = part[q + u][f];
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) chunk += v[u];
+        acc += chunk;
+        chunk = 0.0;
+      }
+      for (; q < groups; ++q) chunk += part[q][f];
+      if (groups % kPer != 0) acc += chunk;  // (only the last round has a partial chunk)
+    }
+    if (r0 + kRound < n) __syncthreads();  // LDS is written again
+  }
+  if (f < 3 * T) {
+    const long e = 3L * (i0 + f % T) + f / T;
+    if (i0 + f % T < n) out.put(3L * n + e, acc * scale);
+  }
+  if (has_v) out.put(ve, vel);
 }
 
 // ------------------------------------------------------ element kernels --
@@ -591,22 +706,15 @@ __device__ inline GroupPos group_pos(const EnsBufs& b) {
   return p;
 }
 
-// rk_stage_kernel (RKEmbeddedParallel.hpp:91-101) for every active system.
-__global__ __launch_bounds__(kBlock) void k_ens_stage(EnsBufs b, int stage) {
-  const GroupPos p = group_pos(b);
-  const SolverState* st = b.st + p.sys;
-  if (st->done) return;
-  if (!p.valid) return;
-  const double* x0 = st->cur ? b.xb1 : b.xb0;
-  b.ytmp[p.e] = stage_value(e_tab[b.tableau], stage, st->dt, b.ks, x0, p.e, b.nv);
-}
-
-// The fused final pass of an attempt (RKEmbeddedParallel.hpp:47-55,
-// 103-137): new state, embedded error, error target, the scaled squared
-// error reduced into this group's partial, and the FSAL copy.
+// The fused end of an attempt (RKEmbeddedParallel.hpp:47-55, 103-137): new
+// state, embedded error, error target, the scaled squared error reduced into
+// this group's partial and the FSAL copy; then, in the last of the system's
+// groups to get there, accept/reject and step size.  kLearned: with the network
+// (its weights' registers would halve the waves of the other controllers' pass).
+template <bool kLearned>
 __global__ __launch_bounds__(kBlock) void k_ens_final(EnsBufs b) {
   const GroupPos p = group_pos(b);
-  const SolverState* st = b.st + p.sys;
+  SolverState* st = b.st + p.sys;
   if (st->done) return;  // uniform over the workgroup
   const Tableau& T = e_tab[b.tableau];
   const int cur = st->cur;
@@ -624,70 +732,23 @@ __global__ __launch_bounds__(kBlock) void k_ens_final(EnsBufs b) {
   }
   const double g = group_reduce(term);
   if (threadIdx.x == 0) b.partA[p.g] = g;
-}
-
-// Accept/reject and step size, one thread per system.
-__global__ void k_ens_controller(EnsBufs b) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= b.n_sys) return;
-  SolverState* st = b.st + s;
-  if (st->done) return;
-  const EnsSys sy = b.sys[s];
-  if (sy.n <= b.solo_n) return;
-  const double sum = fold_partials(b.partA + sy.gbase, sy.n_groups);
-  double* trace = b.trace ? b.trace + static_cast<size_t>(s) * b.trace_cap * 3 : nullptr;
-  ctrl_attempt(st, e_tab[st->tableau], sum, 6 * static_cast<size_t>(sy.n), nullptr,
-               trace);
-  if (st->done) atomicSub(b.n_active, 1);
-}
-
-// One wave per system, the reference and PI controllers on its first lane:
-// the partials come in side by side, and systems do not wait for each other's
-// branches.
-__global__ __launch_bounds__(64) void k_ens_controller_wave(EnsBufs b) {
-  __shared__ float x[16], h[64];
-  const int s = blockIdx.x;
-  SolverState* st = b.st + s;
-  const EnsSys sy = b.sys[s];
-  if (st->done || sy.n <= b.solo_n) return;  // read by every lane before lane 0 writes it
-  const Tableau& T = e_tab[b.tableau];
+  const EnsSys sy = b.sys[p.sys];
+  if (!last_group(st, sy.n_groups)) return;
   const double sum = fold_partials_block(b.partA + sy.gbase, sy.n_groups);
-  double* trace = b.trace ? b.trace + static_cast<size_t>(s) * b.trace_cap * 3 : nullptr;
-  ctrl_attempt_wave(st, T, sum, 6 * static_cast<size_t>(sy.n), nullptr, trace,
-                    static_cast<const MlpInfer*>(b.mlp), sy.n, x, h);
-  if (threadIdx.x == 0 && st->done) atomicSub(b.n_active, 1);
-}
-
-// The same with the learned controller: one wave per 16 systems; their
-// features go through the network on the matrix cores together.
-__global__ __launch_bounds__(64) void k_ens_controller_learned(EnsBufs b) {
-  __shared__ MlpTileLds tile;
-  const MlpInfer* M = static_cast<const MlpInfer*>(b.mlp);
-  const int lane = threadIdx.x;
-  const int s = blockIdx.x * 16 + lane;
-  SolverState* st = (lane < 16 && s < b.n_sys) ? b.st + s : nullptr;
-  const bool active = st && !st->done && b.sys[s].n > b.solo_n;
-  bool accept = false, judged = false;
-  float raw[kMlpIn];
-  for (int i = 0; i < kMlpIn; ++i) raw[i] = 0.0f;
-  if (active) {
-    const EnsSys sy = b.sys[s];
-    const double sum = fold_partials(b.partA + sy.gbase, sy.n_groups);
-    double* trace =
-        b.trace ? b.trace + static_cast<size_t>(s) * b.trace_cap * 3 : nullptr;
-    judged = ctrl_judge(st, e_tab[st->tableau], sum, 6 * static_cast<size_t>(sy.n),
-                        nullptr, trace, &accept);
-    if (judged) mlp_features(st, sy.n, raw);
+  __shared__ SolverState ls;
+  if (threadIdx.x >= 64) return;
+  state_words(&ls, st);
+  double* trace = b.trace ? b.trace + static_cast<size_t>(p.sys) * b.trace_cap * 3 : nullptr;
+  if constexpr (kLearned) {
+    __shared__ MlpRowLds lds;
+    ctrl_attempt_wave(&ls, T, sum, 6 * static_cast<size_t>(sy.n), nullptr, trace,
+                      static_cast<const MlpInfer*>(b.mlp), sy.n, &lds);
+  } else if (threadIdx.x == 0) {
+    ctrl_attempt(&ls, T, sum, 6 * static_cast<size_t>(sy.n), nullptr, trace);
   }
-  if (lane < 16) mlp_tile_set_row(M, tile, lane, raw);
-  __syncthreads();
-  mlp_tile_forward(M, tile);
-  if (active) {
-    if (judged) {
-      ctrl_step(st, accept, mlp_ratio(tile.y[lane]));
-    }
-    if (st->done) atomicSub(b.n_active, 1);
-  }
+  wave_lds_fence();
+  state_words(st, &ls);
+  if (threadIdx.x == 0 && ls.done) atomicSub(b.n_active, 1);
 }
 
 // Dense output of every system whose attempt of this round was accepted and
@@ -812,7 +873,7 @@ __global__ __launch_bounds__(kBlock) void k_ens_copy_out(EnsBufs b,
 
 template <int kVariant, bool kMass, bool kSpecial, bool kNear>
 hipError_t launch_rhs_v(const EnsBufs& b, const double* y, double* k,
-                        int stage0, hipStream_t s) {
+                        int stage0, const NextStage& next, hipStream_t s) {
   if (b.split > 1) {
     // one 64-target tile per workgroup of b.split waves
     if (b.wpb != 1 || b.tpl2_min_n != kEnsNoTpl2) return hipErrorInvalidValue;
@@ -821,26 +882,34 @@ hipError_t launch_rhs_v(const EnsBufs& b, const double* y, double* k,
     if constexpr (kVariant == ODEHIP_NBODY_EXACT) {
       if (b.split == 2)
         hipLaunchKernelGGL((k_ens_rhs_exact_split<kMass, kSpecial, 2>), dim3(blocks),
-                           dim3(128), 0, s, b, y, k, stage0);
+                           dim3(128), 0, s, b, y, k, stage0, next);
       else if (b.split == 4)
         hipLaunchKernelGGL((k_ens_rhs_exact_split<kMass, kSpecial, 4>), dim3(blocks),
-                           dim3(256), 0, s, b, y, k, stage0);
+                           dim3(256), 0, s, b, y, k, stage0, next);
       else if (b.split == 8)
         hipLaunchKernelGGL((k_ens_rhs_exact_split<kMass, kSpecial, 8>), dim3(blocks),
-                           dim3(512), 0, s, b, y, k, stage0);
+                           dim3(512), 0, s, b, y, k, stage0, next);
       else
         return hipErrorInvalidValue;
       return hipGetLastError();
     } else {
+      if constexpr (!kNear) {
+        if (b.n_tiles <= kEnsFineTiles) {
+          hipLaunchKernelGGL((k_ens_rhs_fine<kVariant, kMass, kSpecial>),
+                             dim3(blocks, 64 / kFineTargets), dim3(64 * kFineWaves), 0, s, b, y, k,
+                             stage0, next);
+          return hipGetLastError();
+        }
+      }
       if (b.split == 2)
         hipLaunchKernelGGL((k_ens_rhs_split<kVariant, kMass, kSpecial, kNear, 2>),
-                           dim3(blocks), dim3(128), 0, s, b, y, k, stage0);
+                           dim3(blocks), dim3(128), 0, s, b, y, k, stage0, next);
       else if (b.split == 4)
         hipLaunchKernelGGL((k_ens_rhs_split<kVariant, kMass, kSpecial, kNear, 4>),
-                           dim3(blocks), dim3(256), 0, s, b, y, k, stage0);
+                           dim3(blocks), dim3(256), 0, s, b, y, k, stage0, next);
       else if (b.split == 8)
         hipLaunchKernelGGL((k_ens_rhs_split<kVariant, kMass, kSpecial, kNear, 8>),
-                           dim3(blocks), dim3(512), 0, s, b, y, k, stage0);
+                           dim3(blocks), dim3(512), 0, s, b, y, k, stage0, next);
       else
         return hipErrorInvalidValue;
       return hipGetLastError();
@@ -850,10 +919,10 @@ hipError_t launch_rhs_v(const EnsBufs& b, const double* y, double* k,
   if (blocks == 0) return hipSuccess;
   if (b.wpb == 4) {
     hipLaunchKernelGGL((k_ens_rhs<kVariant, kMass, kSpecial, kNear, 4>), dim3(blocks),
-                       dim3(256), 0, s, b, y, k, stage0);
+                       dim3(256), 0, s, b, y, k, stage0, next);
   } else if (b.wpb == 1) {
     hipLaunchKernelGGL((k_ens_rhs<kVariant, kMass, kSpecial, kNear, 1>), dim3(blocks),
-                       dim3(64), 0, s, b, y, k, stage0);
+                       dim3(64), 0, s, b, y, k, stage0, next);
   } else {
     return hipErrorInvalidValue;
   }
@@ -862,12 +931,12 @@ hipError_t launch_rhs_v(const EnsBufs& b, const double* y, double* k,
 
 template <int kVariant, bool kNear = false>
 hipError_t launch_rhs_m(const EnsBufs& b, const double* y, double* k,
-                        int stage0, hipStream_t s, bool special) {
+                        int stage0, const NextStage& next, hipStream_t s, bool special) {
   if (b.mass)
-    return special ? launch_rhs_v<kVariant, true, true, kNear>(b, y, k, stage0, s)
-                   : launch_rhs_v<kVariant, true, false, kNear>(b, y, k, stage0, s);
-  return special ? launch_rhs_v<kVariant, false, true, kNear>(b, y, k, stage0, s)
-                 : launch_rhs_v<kVariant, false, false, kNear>(b, y, k, stage0, s);
+    return special ? launch_rhs_v<kVariant, true, true, kNear>(b, y, k, stage0, next, s)
+                   : launch_rhs_v<kVariant, true, false, kNear>(b, y, k, stage0, next, s);
+  return special ? launch_rhs_v<kVariant, false, true, kNear>(b, y, k, stage0, next, s)
+                 : launch_rhs_v<kVariant, false, false, kNear>(b, y, k, stage0, next, s);
 }
 
 inline unsigned groups_grid(const EnsBufs& b) {
@@ -880,19 +949,19 @@ inline unsigned sys_grid(const EnsBufs& b) {
 }  // namespace
 
 hipError_t ens_launch_rhs(const EnsBufs& b, const double* y, double* k,
-                          int stage0, hipStream_t s) {
+                          int stage0, hipStream_t s, const NextStage& next) {
   switch (b.variant) {
     case ODEHIP_NBODY_EXACT: {
       const bool shared = b.eps2 >= 0x1p-200 && b.eps2 <= 0x1p100;
-      return launch_rhs_m<ODEHIP_NBODY_EXACT>(b, y, k, stage0, s, shared);
+      return launch_rhs_m<ODEHIP_NBODY_EXACT>(b, y, k, stage0, next, s, shared);
     }
     case ODEHIP_NBODY_FAST:
-      return launch_rhs_m<ODEHIP_NBODY_FAST>(b, y, k, stage0, s, !(b.eps2 >= 1e-150));
+      return launch_rhs_m<ODEHIP_NBODY_FAST>(b, y, k, stage0, next, s, !(b.eps2 >= 1e-150));
     case ODEHIP_NBODY_MIXED: {
       const bool guard = !(static_cast<float>(b.eps2) >= 1e-12f);
       return b.near_c > 0.0
-                 ? launch_rhs_m<ODEHIP_NBODY_MIXED, true>(b, y, k, stage0, s, guard)
-                 : launch_rhs_m<ODEHIP_NBODY_MIXED, false>(b, y, k, stage0, s, guard);
+                 ? launch_rhs_m<ODEHIP_NBODY_MIXED, true>(b, y, k, stage0, next, s, guard)
+                 : launch_rhs_m<ODEHIP_NBODY_MIXED, false>(b, y, k, stage0, next, s, guard);
     }
     default:
       return hipErrorInvalidValue;
@@ -935,25 +1004,20 @@ hipError_t ens_enqueue_initial_step(const EnsBufs& b, hipStream_t s) {
 // One lockstep round: an attempt of every active system.
 hipError_t ens_enqueue_round(const EnsBufs& b, hipStream_t s) {
   const Tableau& T = host_tableau(b.tableau);
-  hipError_t e = ens_launch_rhs(b, nullptr, b.ks, 1, s);
-  if (e != hipSuccess) return e;
-  for (int stage = 1; stage < T.S; ++stage) {
-    hipLaunchKernelGGL(k_ens_stage, dim3(groups_grid(b)), dim3(kBlock), 0, s, b,
-                       stage);
-    if ((e = ens_launch_rhs(b, b.ytmp, b.ks + stage * b.nv, 0, s)) != hipSuccess)
-      return e;
+  hipError_t e = hipSuccess;
+  const double* in = nullptr;  // every system's current state
+  for (int stage = 0; stage < T.S; ++stage) {
+    // two buffers in turn: a stage's input is read while the next one is written
+    double* y = stage + 1 < T.S ? ((stage & 1) ? b.ytmp2 : b.ytmp) : nullptr;
+    e = ens_launch_rhs(b, in, b.ks + stage * b.nv, stage == 0 ? 1 : 0, s,
+                       NextStage{y, b.ks, stage, b.tableau});
+    if (e != hipSuccess) return e;
+    in = y;
   }
-  hipLaunchKernelGGL(k_ens_final, dim3(groups_grid(b)), dim3(kBlock), 0, s, b);
-  // a wave per system while they fit the chip at once (eight waves a SIMD);
-  // beyond, 64 systems a wave, 16 with the network
-  if (b.n_sys <= kEnsSimds * 8) {
-    hipLaunchKernelGGL(k_ens_controller_wave, dim3(b.n_sys), dim3(64), 0, s, b);
-  } else if (b.controller == ODEHIP_CONTROLLER_LEARNED) {
-    hipLaunchKernelGGL(k_ens_controller_learned, dim3((b.n_sys + 15) / 16), dim3(64), 0, s,
-                       b);
-  } else {
-    hipLaunchKernelGGL(k_ens_controller, dim3(sys_grid(b)), dim3(64), 0, s, b);
-  }
+  if (b.controller == ODEHIP_CONTROLLER_LEARNED)
+    hipLaunchKernelGGL(k_ens_final<true>, dim3(groups_grid(b)), dim3(kBlock), 0, s, b);
+  else
+    hipLaunchKernelGGL(k_ens_final<false>, dim3(groups_grid(b)), dim3(kBlock), 0, s, b);
   if (b.n_dense > 0 && b.tableau == ODEHIP_TABLEAU_DOPRI5) {
     hipLaunchKernelGGL(k_ens_dense_begin, dim3(sys_grid(b)), dim3(64), 0, s, b, 0);
     hipLaunchKernelGGL(k_ens_dense_out5, dim3(groups_grid(b)), dim3(kBlock), 0, s, b);

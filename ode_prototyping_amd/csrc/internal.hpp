@@ -34,7 +34,7 @@ struct SolverState {
   long dense_steps, dense_rhs_evals;
   double mass_uniform;  // ensembles: the system's common mass (all equal), else 0
   int dense_go;        // the dense pass of this attempt runs
-  int pad2;
+  int arrived;         // reduction groups of this attempt's final pass that are done
   int cur;       // which ping-pong buffer holds x0
   int done;      // nonzero: every kernel returns immediately
   int status;    // ODEHIP_STATUS_*
@@ -46,6 +46,16 @@ struct SolverState {
   int rejects_in_row;  // consecutive rejections up to now
   int just_accepted;   // the last judged attempt was accepted
   int root_k;          // 1 + q: inv_q1 is the double nearest to 1 / root_k
+};
+
+// What a right-hand-side launch of an attempt does with each element of the
+// stage vector k_n it writes: the next stage's input there,
+// x0 + dt (a_0 k_0 + ... + a_n k_n), with row n of the tableau's a.
+struct NextStage {
+  double* y;             // that input, or null: none
+  const double* ks;      // the attempt's stage vectors
+  int n;                 // index of the one being written
+  int tab;
 };
 
 // Arguments of the N-body RHS kernels.  Exactly one of y / (xb0, xb1, st)
@@ -64,6 +74,7 @@ struct NBodyArgs {
   double eps2;
   float near2;          // mixed variant: pairs with FP32 r^2 below this are
                         // computed in FP64 (0: none)
+  NextStage next;       // (solve only)
 };
 
 // Near-field threshold of the mixed RHS for a system of n bodies: pairs with
@@ -90,15 +101,16 @@ bool valid_tableau(int id);
 // The host copy of a valid tableau id.
 const Tableau& host_tableau(int id);
 // Constant-table slot uploads of a registered tableau, on the current device
-// (rk_kernels.hip, ensemble_kernels.hip).
+// (rk_kernels.hip, ensemble_kernels.hip, nbody_kernels.hip).
 hipError_t upload_rk_tableau(int id, const Tableau& T);
 hipError_t upload_ens_tableau(int id, const Tableau& T);
+hipError_t upload_nbody_tableau(int id, const Tableau& T);
 
 // ---- launchers (rk_kernels.hip) ----
 hipError_t launch_simple_rhs(int kind, const double* y, const double* xb0,
                              const double* xb1, const SolverState* st,
                              double* k, const double* kfsal, int stage0,
-                             size_t n_var, hipStream_t s);
+                             const NextStage& next, size_t n_var, hipStream_t s);
 hipError_t launch_rk_stage_host_dt(int tab, int stage, double dt, double* temp,
                                    const double* ks, const double* x0,
                                    size_t n_var, hipStream_t s);
@@ -166,7 +178,7 @@ hipError_t enqueue_attempt(const SolveBufs& b, hipStream_t s);
 hipError_t enqueue_solve_finish(const SolveBufs& b, double* x_out,
                                 hipStream_t s);
 hipError_t enqueue_rhs(const SolveBufs& b, const double* y_fixed, double* k,
-                       int stage0, hipStream_t s);
+                       int stage0, hipStream_t s, const NextStage& next = NextStage{});
 
 inline int n_groups_for(size_t n) {
   return static_cast<int>((n + ODEHIP_REDUCE_GROUP - 1) / ODEHIP_REDUCE_GROUP);

@@ -53,28 +53,6 @@ __host__ __device__ inline uint16_t float_to_bf16(float f) {
   return static_cast<uint16_t>(u >> 16);
 }
 
-// Raw controller features of one system after an attempt: log error norms of
-// the last three attempts, log(dt / (tf - t0)) of the last, the log ratios of
-// the two before to it, the three accept flags, log N.  Non-finite entries
-// (history not filled yet) are 0.
-__device__ inline void mlp_features(const SolverState* st, int n_particles,
-                                    float* raw) {
-  double f[kMlpIn];
-  for (int h = 0; h < 3; ++h) {
-    double e = st->hist_err[h];
-    e = e < 1.0e-12 ? 1.0e-12 : (e > 1.0e12 ? 1.0e12 : e);
-    f[h] = std::log(e);
-  }
-  const double d0 = st->hist_dt[0];
-  f[3] = std::log(d0 / (st->tf - st->t0));
-  f[4] = std::log(st->hist_dt[1] / d0);
-  f[5] = std::log(st->hist_dt[2] / d0);
-  for (int h = 0; h < 3; ++h) f[6 + h] = st->hist_acc[h];
-  f[9] = std::log(static_cast<double>(n_particles));
-  for (int i = 0; i < kMlpIn; ++i)
-    raw[i] = std::isfinite(f[i]) ? static_cast<float>(f[i]) : 0.0f;
-}
-
 typedef short mlp_short4 __attribute__((ext_vector_type(4)));
 typedef float mlp_float4 __attribute__((ext_vector_type(4)));
 
@@ -251,50 +229,66 @@ __device__ inline double mlp_ratio(double y) {
   return std::isfinite(y) ? std::exp(y) : NAN;
 }
 
-// Feature `i` of mlp_features, normalised (0 from kMlpIn on): a wave's first 16
-// lanes take one each, so the logarithms run side by side.
-__device__ inline float mlp_feature(const MlpInfer* M, const SolverState* st, int n_particles,
-                                    int i) {
-  if (i >= kMlpIn) return 0.0f;
-  double f;
-  if (i >= 6 && i < 9) {
-    f = st->hist_acc[i - 6];
-  } else {
-    const double d0 = st->hist_dt[0];
-    double v;
-    if (i < 3) {
-      v = st->hist_err[i];
-      v = v < 1.0e-12 ? 1.0e-12 : (v > 1.0e12 ? 1.0e12 : v);
-    } else {
-      v = i == 3 ? d0 / (st->tf - st->t0) : i == 9 ? static_cast<double>(n_particles)
-                                                   : st->hist_dt[i - 3] / d0;
-    }
-    f = std::log(v);
+// LDS of one wave's learned controller.
+struct MlpRowLds {
+  double arg[16];
+  float x[16];
+  float h[64];
+};
+
+// Controller features of one system after an attempt: log error norms of the
+// last three attempts, log(dt / (tf - t0)) of the last, the log ratios of the two
+// before to it, the three accept flags, log N; non-finite ones (history not
+// filled yet) are 0.  Lane 0 gathers what they are made of, then 16 lanes take one
+// each (0 from kMlpIn on), so the logarithms run side by side.
+__device__ inline void mlp_gather(const SolverState* st, int n_particles, double* arg) {
+  const double d0 = st->hist_dt[0];
+#pragma unroll
+  for (int h = 0; h < 3; ++h) {
+    const double e = st->hist_err[h];
+    arg[h] = e < 1.0e-12 ? 1.0e-12 : (e > 1.0e12 ? 1.0e12 : e);
+    arg[6 + h] = st->hist_acc[h];
   }
+  arg[3] = d0 / (st->tf - st->t0);
+  arg[4] = st->hist_dt[1] / d0;
+  arg[5] = st->hist_dt[2] / d0;
+  arg[9] = static_cast<double>(n_particles);
+}
+__device__ inline float mlp_feature(const MlpInfer* M, const double* arg, int i) {
+  if (i >= kMlpIn) return 0.0f;
+  const double f = i >= 6 && i < 9 ? arg[i] : std::log(arg[i]);
   const float raw = std::isfinite(f) ? static_cast<float>(f) : 0.0f;
   return (raw - M->mean[i]) * M->inv_std[i];
 }
 
 // An attempt's end by one wave (every lane calls): judge and step on lane 0
 // (`sum` is read there), the learned controller's features and network on all
-// lanes.  `st` is this wave's alone to change; `x` (16) and `h` (64) are its LDS.
+// lanes.  `st`, in LDS, is this wave's alone to change.
 __device__ inline void ctrl_attempt_wave(SolverState* st, const Tableau& T, double sum,
                                          size_t n_var, double* times, double* trace,
-                                         const MlpInfer* M, int n_particles, float* x,
-                                         float* h) {
+                                         const MlpInfer* M, int n_particles, MlpRowLds* lds) {
   const int lane = threadIdx.x & 63;
-  if (st->controller != ODEHIP_CONTROLLER_LEARNED) {
-    if (lane == 0) ctrl_attempt(st, T, sum, n_var, times, trace);
-    return;
-  }
   const MlpRowWeights w = mlp_row_weights(M);
   bool accept = false, judged = false;
-  if (lane == 0) judged = ctrl_judge(st, T, sum, n_var, times, trace, &accept);
+  if (lane == 0) {
+    judged = ctrl_judge(st, T, sum, n_var, times, trace, &accept);
+    mlp_gather(st, n_particles, lds->arg);
+  }
   wave_lds_fence();
-  const float f = mlp_feature(M, st, n_particles, lane < 16 ? lane : 15);
-  if (lane < 16) x[lane] = f;
-  const float out = mlp_row_forward(w, x, h);
+  const float f = mlp_feature(M, lds->arg, lane < 16 ? lane : 15);
+  if (lane < 16) lds->x[lane] = f;
+  const float out = mlp_row_forward(w, lds->x, lds->h);
   if (lane == 0 && judged) ctrl_step(st, accept, mlp_ratio(out));
+}
+
+// The solve state from global memory to LDS and back, by one wave: the
+// controller's reads and writes of it follow one another, each a memory latency.
+static_assert(sizeof(SolverState) % 8 == 0 && sizeof(SolverState) <= 64 * 8, "one word a lane");
+__device__ inline void state_words(SolverState* to, const SolverState* from) {
+  const int lane = threadIdx.x & 63;
+  if (lane < static_cast<int>(sizeof(SolverState) / 8))
+    reinterpret_cast<uint64_t*>(to)[lane] = reinterpret_cast<const uint64_t*>(from)[lane];
+  wave_lds_fence();
 }
 
 // The published inference copy of a network handle (mlp_kernels.hip).

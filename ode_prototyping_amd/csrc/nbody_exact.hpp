@@ -179,7 +179,6 @@ __global__ __launch_bounds__(64 * W) void k_exact_relay(NBodyArgs a) {
   __shared__ RelaySums box;
   const double* __restrict__ y = select_input(a);
   const uniform_ptr yu = as_uniform(y);
-  double* __restrict__ k = a.k;
   const uniform_ptr mu = as_uniform(a.mass);
   const int n = a.n;
   const int lane = threadIdx.x & 63;
@@ -188,11 +187,11 @@ __global__ __launch_bounds__(64 * W) void k_exact_relay(NBodyArgs a) {
   const int i = i0 + lane;
   const int ic = i < n ? i : n - 1;
   const double xi = y[3 * ic], yi = y[3 * ic + 1], zi = y[3 * ic + 2];
+  const Velocity vel = load_velocity(a, y, i0, 64, 192);
   if (threadIdx.x < 64) {
     box.x[lane] = box.y[lane] = box.z[lane] = 0.0;
     box.turn = 0;
   }
-  copy_velocities(y, k, n, i0);
   const ExactForm f = exact_form<kMass, kSharedRcp>(y, a.mass, n, kUniformMassMinN);
   volatile ODEHIP_LDS RelaySums* sums = (volatile ODEHIP_LDS RelaySums*)&box;
   double scale = 1.0;
@@ -207,8 +206,9 @@ __global__ __launch_bounds__(64 * W) void k_exact_relay(NBodyArgs a) {
   __syncthreads();
   if (wave < 3 && i < n) {
     const double acc = wave == 0 ? box.x[lane] : wave == 1 ? box.y[lane] : box.z[lane];
-    k[3L * n + 3 * i + wave] = acc * scale;
+    put<kStageLoads>(a, 3L * n + 3 * i + wave, acc * scale);
   }
+  put_velocity<kStageLoads>(a, vel);
 }
 
 // ------------------------------------------------------------------- slot --
@@ -328,7 +328,6 @@ __global__ __launch_bounds__(64 * W) void k_exact_slot(NBodyArgs a) {
   __shared__ SlotSums<T> box;
   __shared__ double2_t stage[W][C][2];
   const double* __restrict__ y = select_input(a);
-  double* __restrict__ k = a.k;
   const double* __restrict__ mass = a.mass;
   const int n = a.n;
   const int lane = threadIdx.x & 63;
@@ -337,10 +336,8 @@ __global__ __launch_bounds__(64 * W) void k_exact_slot(NBodyArgs a) {
   const int i = i0 + lane % T;
   const double xi = y[3 * i], yi = y[3 * i + 1], zi = y[3 * i + 2];
   const int e = threadIdx.x;
-  if (e < 3 * T) {
-    (&box.v[0][0])[e] = 0.0;
-    k[3L * i0 + e] = y[3L * n + 3L * i0 + e];
-  }
+  const Velocity vel = load_velocity(a, y, i0, T, 3 * T);
+  if (e < 3 * T) (&box.v[0][0])[e] = 0.0;
   if (e < 4) box.turn[e] = 0;
   const ExactForm f = exact_form<kMass, kSharedRcp>(y, mass, n, kUniformMassMinN);
   auto* sums = (volatile ODEHIP_LDS SlotSums<T>*)&box;
@@ -356,7 +353,8 @@ __global__ __launch_bounds__(64 * W) void k_exact_slot(NBodyArgs a) {
                                     i);
   }
   __syncthreads();
-  if (e < 3 * T) k[3L * n + 3 * (i0 + e % T) + e / T] = (&box.v[0][0])[e] * scale;
+  if (e < 3 * T) put<kStageLoads>(a, 3L * n + 3 * (i0 + e % T) + e / T, (&box.v[0][0])[e] * scale);
+  put_velocity<kStageLoads>(a, vel);
 }
 
 // ------------------------------------------------------------------- tile --
@@ -456,7 +454,6 @@ __global__ __launch_bounds__(64 * Sh::W) void k_exact_tile(NBodyArgs a) {
   constexpr int T = Sh::T, PL = Sh::PL;
   __shared__ __attribute__((aligned(16))) double term[2][3 * T][Sh::S];
   const double* __restrict__ y = select_input(a);
-  double* __restrict__ k = a.k;
   const double* __restrict__ mass = a.mass;
   const int n = a.n;
   const int lane = threadIdx.x & 63;
@@ -479,10 +476,7 @@ __global__ __launch_bounds__(64 * Sh::W) void k_exact_tile(NBodyArgs a) {
       L.tz[u] = y[3 * i + 2];
     }
   }
-  if (threadIdx.x < 3 * T) {
-    const long e = 3L * i0 + threadIdx.x;
-    k[e] = y[3L * n + e];
-  }
+  const Velocity vel = load_velocity(a, y, i0, T, 64);
   ExactForm f{false, 0.0};
   if (kSharedRcp && n <= Sh::TJ)  // the producers hold every partner
     f.shared = __syncthreads_and(pw < 0 || point_shared_ok(L.px, L.py, L.pz)) != 0;
@@ -499,7 +493,8 @@ __global__ __launch_bounds__(64 * Sh::W) void k_exact_tile(NBodyArgs a) {
   } else {
     acc = tile_sum<Sh, kMass, false>(term, L, y, mass, n, a.eps2, wave, pw, lane, i0);
   }
-  if (wave == 0 && lane < 3 * T) k[3L * n + 3 * (i0 + lane % T) + lane / T] = acc * scale;
+  if (wave == 0 && lane < 3 * T) put<kStageLoads>(a, 3L * n + 3 * (i0 + lane % T) + lane / T, acc * scale);
+  put_velocity<kStageLoads>(a, vel);
 }
 
 // --------------------------------------------------------------- dispatch --

@@ -28,6 +28,7 @@
 
 #include "internal.hpp"
 #include "nbody_terms.hpp"
+#include "rk_device.hpp"
 
 namespace odehip {
 namespace {
@@ -45,33 +46,70 @@ __device__ inline const double* select_input(const NBodyArgs& a) {
   return a.st->cur ? a.xb1 : a.xb0;
 }
 
+// built-in tableaux, then the slots of registered ones
+__constant__ Tableau n_tab[ODEHIP_MAX_TABLEAUS] = {
+    kTableaus[0], kTableaus[1], kTableaus[2],
+    kTableaus[3], kTableaus[4], kTableaus[5]};
+
+// The kernel's arguments (NBodyArgs its only parameter), read again: what only
+// the end of a kernel needs does not hold SGPRs through the partner loop.
+__device__ inline NBodyArgs late_args() {
+  typedef const __attribute__((address_space(4))) NBodyArgs* args_ptr;
+  args_ptr p = (args_ptr)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  NBodyArgs a;
+  __builtin_memcpy(&a, (const void*)p, sizeof a);
+  return a;
+}
+
+// Element e of the result, and of the next stage's input (L: next_stage).
+template <int L>
+__device__ inline void put(const NBodyArgs& a, long e, double v) {
+  a.k[e] = v;
+  if (a.next.y)
+    next_stage<L>(a.next, n_tab[a.next.tab], 6 * static_cast<size_t>(a.n), e, v,
+                  (a.st->cur ? a.xb1 : a.xb0)[e], a.st->dt);
+}
+
 // Returns true if the launch has nothing to compute (solve finished, or k1
 // of this attempt is reused, or a dense-output evaluation whose pass does not
-// run).  On FSAL reuse the launch copies k1 instead.
+// run).  On k1 reuse the launch copies k1 instead, unless it is in place, and
+// forms the next stage's input.
 __device__ inline bool prologue_skip(const NBodyArgs& a) {
   if (!a.st) return false;
   if (a.stage0 == 2) return a.st->dense_go == 0;
   if (a.st->done) return true;
   if (a.stage0 && a.st->k1_valid) {
-    if (a.st->k1_valid == 1) {
-      const size_t n_var = static_cast<size_t>(a.n) * 6;
-      for (size_t e = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-           e < n_var; e += static_cast<size_t>(gridDim.x) * blockDim.x)
-        a.k[e] = a.kfsal[e];
-    }
+    const double* from = a.st->k1_valid == 1 ? a.kfsal : a.k;
+    const long n_var = static_cast<long>(a.n) * 6;
+    for (long e = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x; e < n_var;
+         e += static_cast<long>(gridDim.x) * blockDim.x)
+      put<kStageLoadsLean>(a, e, from[e]);
     return true;
   }
   return false;
 }
 
-// dxdt[0:3N] = x[3N:6N] for this tile's particles (nbody_init_dxdt_kernel,
-// NBodyODE.hpp:51-56).
-__device__ inline void copy_velocities(const double* __restrict__ y,
-                                       double* __restrict__ k, int n, int i0) {
-  const int e = threadIdx.x;
-  const long base = 3L * i0;
-  const long lim = 3L * n;
-  if (e < 192 && base + e < lim) k[base + e] = y[lim + base + e];
+// dxdt[0:3N] = x[3N:6N] for `count` particles from i0
+// (nbody_init_dxdt_kernel, NBodyODE.hpp:51-56): one element per thread, loaded
+// at the start and written at the end (the load's latency passes meanwhile).
+// The threads before `first` write accelerations; a workgroup too small for
+// both starts from thread 0.
+struct Velocity {
+  long e;  // -1: none
+  double v;
+};
+__device__ inline Velocity load_velocity(const NBodyArgs& a, const double* __restrict__ y,
+                                         int i0, int count, int first) {
+  const int t = static_cast<int>(threadIdx.x) -
+                (first + 3 * count <= static_cast<int>(blockDim.x) ? first : 0);
+  const long e = 3L * i0 + t, lim = 3L * a.n;
+  if (t < 0 || t >= 3 * count || e >= lim) return Velocity{-1, 0.0};
+  return Velocity{e, y[lim + e]};
+}
+template <int L>
+__device__ inline void put_velocity(const NBodyArgs& a, const Velocity& v) {
+  if (v.e >= 0) put<L>(a, v.e, v.v);
 }
 
 // Whether every position coordinate of the state passes coord_shared_ok:
@@ -99,6 +137,12 @@ __device__ inline double uniform_pow2_mass(const double* __restrict__ mass, int 
 
 // ------------------------------------------------------------------- fast --
 constexpr int kFastWaves = 16;
+
+// Two 16-wave workgroups share a CU only while a wave's SGPRs fit eighty: the
+// SIMD's 800 hold eight waves of 80 and the 16 the trap handler keeps per wave.
+// (With 88, which the compiler counts as eight waves too, 65536 bodies took 2584
+// instead of 2391 us, and the mixed kernel 1789 instead of 1430.)
+#define ODEHIP_EIGHT_WAVES_SGPRS __attribute__((amdgpu_num_sgpr(80)))
 
 // kFastSet partners' coordinates (and masses), wave-uniform in SGPRs.
 constexpr int kFastSet = 4;
@@ -207,12 +251,11 @@ __device__ inline double workgroup_uniform_mass(const double* __restrict__ mass,
 }
 
 template <bool kMass, bool kGuard, bool kPrefetch>
-__global__ __launch_bounds__(64 * kFastWaves) void k_nbody_fast(NBodyArgs a) {
+__device__ __forceinline__ void fast_kernel(const NBodyArgs& a) {
   if (prologue_skip(a)) return;
   __shared__ double red[kFastWaves][3][64];
   const double* __restrict__ y = select_input(a);
   const uniform_ptr yu = as_uniform(y);
-  double* __restrict__ k = a.k;
   const uniform_ptr mass = as_uniform(a.mass);
   const int n = a.n;
   const double eps2 = a.eps2;
@@ -238,14 +281,27 @@ __global__ __launch_bounds__(64 * kFastWaves) void k_nbody_fast(NBodyArgs a) {
   red[wave][0][lane] = ax;
   red[wave][1][lane] = ay;
   red[wave][2][lane] = az;
+  const NBodyArgs late = late_args();
   __syncthreads();
   if (wave < 3 && valid_i) {
     double s = 0.0;
 #pragma unroll
     for (int w = 0; w < kFastWaves; ++w) s += red[w][wave][lane];
-    k[3L * n + 3 * i + wave] = kMass && m_uni != 0.0 ? s * m_uni : s;
+    put<kStageLoadsLean>(late, 3L * n + 3 * i + wave, kMass && m_uni != 0.0 ? s * m_uni : s);
   }
-  copy_velocities(y, k, n, i0);
+  // (loaded only here: held through the loop, two VGPRs cost it 1.5 %)
+  put_velocity<kStageLoadsLean>(late, load_velocity(late, select_input(late), i0, 64, 192));
+}
+
+template <bool kMass, bool kGuard>
+__global__ __launch_bounds__(64 * kFastWaves) ODEHIP_EIGHT_WAVES_SGPRS
+void k_nbody_fast(NBodyArgs a) {
+  fast_kernel<kMass, kGuard, false>(a);
+}
+// (one workgroup per CU: the two SGPR sets may take what they need)
+template <bool kMass, bool kGuard>
+__global__ __launch_bounds__(64 * kFastWaves) void k_nbody_fast_prefetch(NBodyArgs a) {
+  fast_kernel<kMass, kGuard, true>(a);
 }
 
 // The fast sum for grids of 64-target workgroups that would leave CUs empty: R
@@ -325,7 +381,6 @@ __global__ __launch_bounds__(64 * kFastRowsWaves) void k_nbody_fast_rows(NBodyAr
   __shared__ double red[kFastRowsWaves][3 * R];
   const double* __restrict__ y = select_input(a);
   const uniform_ptr yu = as_uniform(y);
-  double* __restrict__ k = a.k;
   const double* __restrict__ mass = a.mass;
   const int n = a.n;
   const double eps2 = a.eps2;
@@ -345,7 +400,7 @@ __global__ __launch_bounds__(64 * kFastRowsWaves) void k_nbody_fast_rows(NBodyAr
     v[3 * t] = v[3 * t + 1] = v[3 * t + 2] = 0.0;
   }
   const int e = threadIdx.x;
-  if (e < 3 * R) k[3L * i0 + e] = y[3L * n + 3L * i0 + e];
+  const Velocity vel = load_velocity(a, y, i0, R, 3 * R);
   for (int b = wave * 64; b < n; b += step) {
     const int jn = min(b + step + lane, n - 1);  // the next partner, loaded ahead
     const double qx = y[3 * jn], qy = y[3 * jn + 1], qz = y[3 * jn + 2];
@@ -373,8 +428,9 @@ __global__ __launch_bounds__(64 * kFastRowsWaves) void k_nbody_fast_rows(NBodyAr
   if (e < 3 * R) {
     double s = 0.0;
     for (int w = 0; w < step / 64; ++w) s += red[w][e];
-    k[3L * n + 3L * i0 + e] = s;
+    put<kStageLoads>(a, 3L * n + 3L * i0 + e, s);
   }
+  put_velocity<kStageLoads>(a, vel);
 }
 
 // ------------------------------------------------------------------ mixed --
@@ -451,12 +507,12 @@ __device__ __forceinline__ void mixed_partners(uniform_ptr yu, uniform_ptr mass,
 
 // kNear: near pairs (a.near2 > 0) in FP64; without it every pair is FP32.
 template <bool kMass, bool kGuard, bool kNear>
-__global__ __launch_bounds__(64 * kMixedWaves) void k_nbody_mixed(NBodyArgs a) {
+__global__ __launch_bounds__(64 * kMixedWaves) ODEHIP_EIGHT_WAVES_SGPRS
+void k_nbody_mixed(NBodyArgs a) {
   if (prologue_skip(a)) return;
   __shared__ double red[kMixedWaves][3][64];
   const double* __restrict__ y = select_input(a);
   const uniform_ptr yu = as_uniform(y);
-  double* __restrict__ k = a.k;
   const uniform_ptr mass = as_uniform(a.mass);
   const int n = a.n;
   const float eps2f = static_cast<float>(a.eps2);
@@ -483,14 +539,16 @@ __global__ __launch_bounds__(64 * kMixedWaves) void k_nbody_mixed(NBodyArgs a) {
   red[wave][0][lane] = ax;
   red[wave][1][lane] = ay;
   red[wave][2][lane] = az;
+  const NBodyArgs late = late_args();
   __syncthreads();
   if (wave < 3 && valid_i) {
     double s = 0.0;
 #pragma unroll
     for (int w = 0; w < kMixedWaves; ++w) s += red[w][wave][lane];
-    k[3L * n + 3 * i + wave] = kMass && m_uni != 0.0 ? s * m_uni : s;
+    put<kStageLoadsLean>(late, 3L * n + 3 * i + wave, kMass && m_uni != 0.0 ? s * m_uni : s);
   }
-  copy_velocities(y, k, n, i0);
+  // (loaded only here: held through the loop, two VGPRs cost it 1.5 %)
+  put_velocity<kStageLoadsLean>(late, load_velocity(late, select_input(late), i0, 64, 192));
 }
 
 // ----------------------------------------------------------------- energy --
@@ -718,14 +776,14 @@ hipError_t launch_nbody_rhs(const NBodyArgs& a, int variant, hipStream_t s) {
       }
       // one workgroup per CU at most: 4 waves per SIMD, prefetching partner loop
       const bool prefetch = static_cast<long>(blocks) <= device_cus();
-      auto* kern = mass ? (guard ? (prefetch ? k_nbody_fast<true, true, true>
-                                             : k_nbody_fast<true, true, false>)
-                                 : (prefetch ? k_nbody_fast<true, false, true>
-                                             : k_nbody_fast<true, false, false>))
-                        : (guard ? (prefetch ? k_nbody_fast<false, true, true>
-                                             : k_nbody_fast<false, true, false>)
-                                 : (prefetch ? k_nbody_fast<false, false, true>
-                                             : k_nbody_fast<false, false, false>));
+      auto* kern = mass ? (guard ? (prefetch ? k_nbody_fast_prefetch<true, true>
+                                             : k_nbody_fast<true, true>)
+                                 : (prefetch ? k_nbody_fast_prefetch<true, false>
+                                             : k_nbody_fast<true, false>))
+                        : (guard ? (prefetch ? k_nbody_fast_prefetch<false, true>
+                                             : k_nbody_fast<false, true>)
+                                 : (prefetch ? k_nbody_fast_prefetch<false, false>
+                                             : k_nbody_fast<false, false>));
       hipLaunchKernelGGL(kern, dim3(blocks), dim3(64 * kFastWaves), 0, s, a);
       break;
     }
@@ -780,6 +838,12 @@ hipError_t launch_nbody_energy(const double* x, int n, double eps2, const double
   hipLaunchKernelGGL(k_energy_sums, dim3(1), dim3(256), 0, s, kin, static_cast<long>(nt), pot,
                      static_cast<long>(nt) * parts, out);
   return hipGetLastError();
+}
+
+hipError_t upload_nbody_tableau(int id, const Tableau& T) {
+  if (id < ODEHIP_NUM_TABLEAUS || id >= ODEHIP_MAX_TABLEAUS) return hipErrorInvalidValue;
+  return hipMemcpyToSymbol(HIP_SYMBOL(n_tab), &T, sizeof(Tableau), id * sizeof(Tableau),
+                           hipMemcpyHostToDevice);
 }
 
 }  // namespace odehip

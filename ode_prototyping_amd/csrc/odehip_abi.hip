@@ -79,6 +79,7 @@ int odehip::use_tableau(odehip_context* ctx, int id) {
   for (int& next = r.resident[d]; next <= id; ++next) {
     HIP_TRY(ctx, upload_rk_tableau(next, r.tab[next]));
     HIP_TRY(ctx, upload_ens_tableau(next, r.tab[next]));
+    HIP_TRY(ctx, upload_nbody_tableau(next, r.tab[next]));
     HIP_TRY(ctx, upload_solo_tableau(next, r.tab[next]));
   }
   return ODEHIP_OK;
@@ -450,7 +451,7 @@ int odehip_ode_rhs(odehip_context* ctx, int kind, const double* x, double* dxdt,
   if (kind == ODEHIP_RHS_VANDERPOL && n_var != 2)
     return fail(ctx, ODEHIP_ERR_INVALID, "Van der Pol has n_var 2");
   hipError_t e = launch_simple_rhs(kind, x, nullptr, nullptr, nullptr, dxdt,
-                                   nullptr, 0, n_var, ctx->stream);
+                                   nullptr, 0, NextStage{}, n_var, ctx->stream);
   if (e != hipSuccess) return hip_fail(ctx, e, "ode_rhs");
   return ODEHIP_OK;
 }
@@ -706,7 +707,7 @@ int odehip_rk_solve(odehip_context* ctx, int tableau, const odehip_ode* ode,
   // caller says how the attempts are launched or every state is kept.
   const bool solo = ode->rhs_kind == ODEHIP_RHS_NBODY && opt->attempts_per_launch == 0 &&
                     ode->nbody_variant != ODEHIP_NBODY_MIXED && n_dense == 0 &&
-                    states_cap == 0 && b.n_particles <= solo_limit(S, ode->nbody_variant);
+                    states_cap == 0 && b.n_particles <= solo_limit(S, ode->nbody_variant, b.mlp != nullptr);
   SoloArgs sa{};
   if (solo) {
     K = kSoloAttempts;

@@ -42,19 +42,22 @@ __device__ inline double fold_partials(const double* p, int n_groups) {
   return r;
 }
 
-// The same fold, called by every thread of a 64-thread block: the partials
-// are first staged through LDS by all lanes (coalesced), then lane 0 adds
-// them in order from LDS.  Returns the sum in lane 0.
-constexpr int kFoldLds = 4096;
+// The same fold, called by every thread of a block: the partials are first
+// staged through LDS (coalesced), kFoldLds at a time, then thread 0 adds them in
+// order from LDS.  Returns the sum in thread 0.
+constexpr int kFoldLds = 512;
 __device__ inline double fold_partials_block(const double* p, int n_groups) {
   __shared__ double buf[kFoldLds];
-  if (n_groups > kFoldLds) return threadIdx.x == 0 ? fold_partials(p, n_groups) : 0.0;
-  for (int g = threadIdx.x; g < n_groups; g += blockDim.x) buf[g] = p[g];
-  __syncthreads();
   double r = 0.0;
-  if (threadIdx.x == 0) {
+  for (int g0 = 0; g0 < n_groups; g0 += kFoldLds) {
+    const int cnt = min(kFoldLds, n_groups - g0);
+    if (g0 > 0) __syncthreads();
+    for (int g = threadIdx.x; g < cnt; g += blockDim.x) buf[g] = p[g0 + g];
+    __syncthreads();
+    if (threadIdx.x == 0) {
 #pragma unroll 8
-    for (int g = 0; g < n_groups; ++g) r = r + buf[g];
+      for (int g = 0; g < cnt; ++g) r = r + buf[g];
+    }
   }
   return r;
 }
@@ -67,6 +70,30 @@ __device__ inline double stage_value(const Tableau& T, int stage, double dt,
   double tmp = 0.0;
   for (int j = 0; j < stage; ++j) tmp += T.a[stage - 1][j] * ks[j * n_var + i];
   return x0[i] + tmp * dt;
+}
+
+// The same for element e of the next stage by the launch that writes its last
+// stage vector (NextStage), whose element is k: the sum in the same order, L
+// loads per round trip (a load per step of the sum would wait for each in turn).
+// All of them for kernels whose launch is a chain of latencies; few for those
+// that fill the chip, whose occupancy the loads' registers would take.
+constexpr int kStageLoads = kMaxStages - 1;
+constexpr int kStageLoadsLean = 6;
+template <int L>
+__device__ inline void next_stage(const NextStage& N, const Tableau& T, size_t n_var, size_t e,
+                                  double k, double x0, double dt) {
+  double tmp = 0.0;
+  for (int j0 = 0; j0 < N.n; j0 += L) {
+    double v[L];
+#pragma unroll
+    for (int u = 0; u < L; ++u)
+      v[u] = N.ks[static_cast<size_t>(j0 + u < N.n ? j0 + u : j0) * n_var + e];
+#pragma unroll
+    for (int u = 0; u < L; ++u)
+      if (j0 + u < N.n) tmp += T.a[N.n][j0 + u] * v[u];
+  }
+  tmp += T.a[N.n][N.n] * k;
+  N.y[e] = x0 + tmp * dt;
 }
 
 // detail::update_state_and_error_kernel (RKEmbeddedParallel.hpp:103-123).
@@ -82,6 +109,23 @@ __device__ inline void update_values(const Tableau& T, double dt,
   }
   x = x0[i] + xs * dt;
   err = es * dt;
+}
+
+// Called by every thread of a workgroup of an attempt's final pass once thread 0
+// has written the workgroup's partial: true in the last of the n_groups
+// workgroups, which then sees every partial and may change the solve's state.
+// (The fences make the partials visible between the XCDs' L2s.)
+__device__ inline bool last_group(SolverState* st, int n_groups) {
+  __shared__ int last;
+  if (threadIdx.x == 0) {
+    __threadfence();
+    last = atomicAdd(&st->arrived, 1) == n_groups - 1;
+    if (last) st->arrived = 0;
+  }
+  __syncthreads();
+  if (!last) return false;
+  __threadfence();
+  return true;
 }
 
 // ---------------------------------------------------------- controller ----
@@ -127,7 +171,7 @@ __device__ inline void ctrl_init(SolverState* st, const Tableau& T, double t0,
   st->dense_steps = 0;
   st->dense_rhs_evals = 0;
   st->dense_go = 0;
-  st->pad2 = 0;
+  st->arrived = 0;
   st->cur = 0;
   st->fsal = fsal;
   st->tableau = tab;

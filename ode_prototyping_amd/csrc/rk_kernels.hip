@@ -30,34 +30,35 @@ __device__ inline size_t gid() {
 // ----------------------------------------------------------- simple RHS ----
 __global__ void k_exp_rhs(const double* y, const double* xb0, const double* xb1,
                           const SolverState* st, double* k, const double* kfsal,
-                          int stage0, size_t n_var) {
+                          int stage0, NextStage next, size_t n_var) {
   if (st && (stage0 == 2 ? st->dense_go == 0 : st->done)) return;
   const size_t i = gid();
-  if (st && stage0 == 1 && st->k1_valid) {
-    if (st->k1_valid == 1 && i < n_var) k[i] = kfsal[i];
-    return;
-  }
+  if (i >= n_var) return;
   const double* x = y ? y : (st->cur ? xb1 : xb0);
-  if (i < n_var) k[i] = x[i];  // ExponentialODE.hpp:16-18
+  // ExponentialODE.hpp:16-18, or the reused k1
+  if (st && stage0 == 1 && st->k1_valid) x = st->k1_valid == 1 ? kfsal : k;
+  const double v = x[i];
+  k[i] = v;
+  if (next.y) next_stage<kStageLoads>(next, c_tab[next.tab], n_var, i, v, (st->cur ? xb1 : xb0)[i], st->dt);
 }
 
 __global__ void k_vdp_rhs(const double* y, const double* xb0, const double* xb1,
                           const SolverState* st, double* k, const double* kfsal,
-                          int stage0) {
+                          int stage0, NextStage next) {
   if (st && (stage0 == 2 ? st->dense_go == 0 : st->done)) return;
   const int i = threadIdx.x;
+  if (i >= 2) return;
+  double v;
   if (st && stage0 == 1 && st->k1_valid) {
-    if (st->k1_valid == 1 && i < 2) k[i] = kfsal[i];
-    return;
-  }
-  const double* x = y ? y : (st->cur ? xb1 : xb0);
-  // VanDerPolODE.hpp:16-25 (eps = 1)
-  if (i == 0) {
-    k[0] = x[1];
-  } else if (i == 1) {
+    v = (st->k1_valid == 1 ? kfsal : k)[i];
+  } else {
+    const double* x = y ? y : (st->cur ? xb1 : xb0);
+    // VanDerPolODE.hpp:16-25 (eps = 1)
     const double eps = 1.0;
-    k[1] = eps * (1.0 - x[0] * x[0]) * x[1] - x[0];
+    v = i == 0 ? x[1] : eps * (1.0 - x[0] * x[0]) * x[1] - x[0];
   }
+  k[i] = v;
+  if (next.y) next_stage<kStageLoads>(next, c_tab[next.tab], 2, i, v, (st->cur ? xb1 : xb0)[i], st->dt);
 }
 
 // ------------------------------------------------------- stage kernels -----
@@ -66,15 +67,6 @@ __global__ void k_stage_host_dt(int tab, int stage, double dt, double* temp,
                                 size_t n_var) {
   const size_t i = gid();
   if (i < n_var) temp[i] = stage_value(c_tab[tab], stage, dt, ks, x0, i, n_var);
-}
-
-__global__ void k_stage_dev(const SolverState* st, int tab, int stage,
-                            double* temp, const double* ks, const double* xb0,
-                            const double* xb1, size_t n_var) {
-  if (st->done) return;
-  const size_t i = gid();
-  const double* x0 = st->cur ? xb1 : xb0;
-  if (i < n_var) temp[i] = stage_value(c_tab[tab], stage, st->dt, ks, x0, i, n_var);
 }
 
 __global__ void k_update_host_dt(int tab, double dt, double* x, double* err,
@@ -96,13 +88,16 @@ __global__ void k_target(double* sc, const double* atol, const double* rtol,
   if (i < n_var) sc[i] = atol[i] + rtol[i] * max_abs(x[i], x0[i]);
 }
 
-// Fused final stage of an attempt: new state, embedded error, error target
-// and the scaled squared error folded into this group's partial -- one
-// coalesced pass over ks (RKEmbeddedParallel.hpp:47-55, 103-137).
+// Fused end of an attempt: new state, embedded error, error target and the
+// scaled squared error folded into this group's partial -- one coalesced pass
+// over ks (RKEmbeddedParallel.hpp:47-55, 103-137) --, then, in the last group
+// to get there, accept/reject and step-size control (:57-79) with the
+// termination tests and counters.  kLearned: with the network.
+template <bool kLearned>
 __global__ __launch_bounds__(kBlock) void k_final_dev(
-    const SolverState* st, int tab, const double* ks, double* xb0, double* xb1,
+    SolverState* st, int tab, const double* ks, double* xb0, double* xb1,
     const double* atol, const double* rtol, double* partials, double* kfsal,
-    size_t n_var) {
+    size_t n_var, double* times, double* trace, const MlpInfer* M, int n_particles) {
   if (st->done) return;
   const Tableau& T = c_tab[tab];
   const int cur = st->cur;
@@ -122,26 +117,19 @@ __global__ __launch_bounds__(kBlock) void k_final_dev(
   }
   const double g = group_reduce(term);
   if (threadIdx.x == 0) partials[blockIdx.x] = g;
-}
-
-// Accept/reject and step-size control (RKEmbeddedParallel.hpp:57-79) on the
-// device, plus the termination tests and counters.
-__global__ void k_controller(SolverState* st, const double* partials,
-                             size_t n_var, double* times, double* trace) {
-  if (st->done) return;
-  const double sum = fold_partials_block(partials, st->n_groups);
-  if (threadIdx.x != 0) return;
-  ctrl_attempt(st, c_tab[st->tableau], sum, n_var, times, trace);
-}
-
-// The same with the learned controller's network.
-__global__ __launch_bounds__(64) void k_controller_learned(
-    SolverState* st, const double* partials, size_t n_var, double* times,
-    double* trace, const MlpInfer* M, int n_particles) {
-  __shared__ float x[16], h[64];
-  if (st->done) return;  // read by every thread before thread 0 writes it
-  const double sum = fold_partials_block(partials, st->n_groups);
-  ctrl_attempt_wave(st, c_tab[st->tableau], sum, n_var, times, trace, M, n_particles, x, h);
+  if (!last_group(st, gridDim.x)) return;
+  const double sum = fold_partials_block(partials, gridDim.x);
+  __shared__ SolverState ls;
+  if (threadIdx.x >= 64) return;
+  state_words(&ls, st);
+  if constexpr (kLearned) {
+    __shared__ MlpRowLds lds;
+    ctrl_attempt_wave(&ls, T, sum, n_var, times, trace, M, n_particles, &lds);
+  } else if (threadIdx.x == 0) {
+    ctrl_attempt(&ls, T, sum, n_var, times, trace);
+  }
+  wave_lds_fence();
+  state_words(st, &ls);
 }
 
 // ------------------------------------------------------ initial step -------
@@ -324,14 +312,14 @@ inline unsigned blocks_for(size_t n) {
 hipError_t launch_simple_rhs(int kind, const double* y, const double* xb0,
                              const double* xb1, const SolverState* st,
                              double* k, const double* kfsal, int stage0,
-                             size_t n_var, hipStream_t s) {
+                             const NextStage& next, size_t n_var, hipStream_t s) {
   if (kind == ODEHIP_RHS_EXPONENTIAL) {
     hipLaunchKernelGGL(k_exp_rhs, dim3(blocks_for(n_var)), dim3(kBlock), 0, s,
-                       y, xb0, xb1, st, k, kfsal, stage0, n_var);
+                       y, xb0, xb1, st, k, kfsal, stage0, next, n_var);
   } else if (kind == ODEHIP_RHS_VANDERPOL) {
     if (n_var != 2) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_vdp_rhs, dim3(1), dim3(64), 0, s, y, xb0, xb1, st, k,
-                       kfsal, stage0);
+                       kfsal, stage0, next);
   } else {
     return hipErrorInvalidValue;
   }
@@ -417,7 +405,7 @@ hipError_t launch_sum_tree(const double* v, size_t n, double* out,
 }
 
 hipError_t enqueue_rhs(const SolveBufs& b, const double* y_fixed, double* k,
-                       int stage0, hipStream_t s) {
+                       int stage0, hipStream_t s, const NextStage& next) {
   if (b.rhs_kind == ODEHIP_RHS_NBODY) {
     NBodyArgs a{};
     a.y = y_fixed;
@@ -431,10 +419,11 @@ hipError_t enqueue_rhs(const SolveBufs& b, const double* y_fixed, double* k,
     a.stage0 = stage0;
     a.eps2 = b.eps2;
     a.near2 = b.near2;
+    a.next = next;
     return launch_nbody_rhs(a, b.nbody_variant, s);
   }
   return launch_simple_rhs(b.rhs_kind, y_fixed, b.xb0, b.xb1, b.st, k, b.kfsal,
-                           stage0, b.n_var, s);
+                           stage0, next, b.n_var, s);
 }
 
 hipError_t enqueue_solve_init(const SolveBufs& b, const double* x_in,
@@ -476,24 +465,21 @@ hipError_t enqueue_initial_step(const SolveBufs& b, hipStream_t s) {
 hipError_t enqueue_attempt(const SolveBufs& b, hipStream_t s) {
   const Tableau& T = host_tableau(b.tableau);
   const size_t n = b.n_var;
-  hipError_t e = enqueue_rhs(b, nullptr, b.ks, 1, s);
-  if (e != hipSuccess) return e;
-  for (int stage = 1; stage < T.S; ++stage) {
-    double* temp = (stage & 1) ? b.ytmp1 : b.ytmp0;
-    hipLaunchKernelGGL(k_stage_dev, dim3(blocks_for(n)), dim3(kBlock), 0, s,
-                       b.st, b.tableau, stage, temp, b.ks, b.xb0, b.xb1, n);
-    if ((e = enqueue_rhs(b, temp, b.ks + stage * n, 0, s)) != hipSuccess) return e;
+  hipError_t e = hipSuccess;
+  const double* in = nullptr;  // the current state
+  for (int stage = 0; stage < T.S; ++stage) {
+    // two buffers in turn: a stage's input is read while the next one is written
+    double* y = stage + 1 < T.S ? ((stage & 1) ? b.ytmp0 : b.ytmp1) : nullptr;
+    e = enqueue_rhs(b, in, b.ks + stage * n, stage == 0 ? 1 : 0, s,
+                    NextStage{y, b.ks, stage, b.tableau});
+    if (e != hipSuccess) return e;
+    in = y;
   }
-  hipLaunchKernelGGL(k_final_dev, dim3(blocks_for(n)), dim3(kBlock), 0, s, b.st,
-                     b.tableau, b.ks, b.xb0, b.xb1, b.atol, b.rtol, b.partA,
-                     b.kfsal, n);
-  if (b.controller == ODEHIP_CONTROLLER_LEARNED) {
-    hipLaunchKernelGGL(k_controller_learned, dim3(1), dim3(64), 0, s, b.st, b.partA, n,
-                       b.times, b.trace, b.mlp, b.n_particles);
-  } else {
-    hipLaunchKernelGGL(k_controller, dim3(1), dim3(64), 0, s, b.st, b.partA, n, b.times,
-                       b.trace);
-  }
+  auto* final_pass = b.controller == ODEHIP_CONTROLLER_LEARNED ? k_final_dev<true>
+                                                               : k_final_dev<false>;
+  hipLaunchKernelGGL(final_pass, dim3(blocks_for(n)), dim3(kBlock), 0, s, b.st, b.tableau,
+                     b.ks, b.xb0, b.xb1, b.atol, b.rtol, b.partA,
+                     b.kfsal, n, b.times, b.trace, b.mlp, b.n_particles);
   if (b.states && b.states_cap > 0)
     hipLaunchKernelGGL(k_save_state, dim3(blocks_for(n)), dim3(kBlock), 0, s, b.st, b.xb0,
                        b.xb1, b.states, b.states_cap, n);

@@ -5,10 +5,9 @@
 #include <algorithm>
 
 #include "ensemble.hpp"
+#include "mlp.hpp"
 
 namespace odehip {
-
-struct MlpInfer;
 
 constexpr int kSoloWaves = 16;    // at most, per workgroup
 constexpr int kSoloTerms = 4;     // exact: partners per wave and block
@@ -45,15 +44,20 @@ struct SoloArgs {
   int lds_doubles;     // set by launch_solo
 };
 
-// LDS of a system of n bodies: state, stage input, S stage vectors, masses and
-// the partial sums of the waves.
-__host__ __device__ inline int solo_lds_doubles(int n, int S, int variant, int waves) {
-  const int sums = variant == ODEHIP_NBODY_EXACT ? 3 * 64 * kSoloTerms : 192;
-  return (S + 2) * 6 * n + ((n + 1) & ~1) + waves * sums;
+// LDS of a system of n bodies: state, stage input, S stage vectors, masses, the
+// partial sums of the waves and the learned controller's network.
+__host__ __device__ constexpr int solo_sums(int variant) {
+  return variant == ODEHIP_NBODY_EXACT ? 3 * 64 * kSoloTerms : 192;
+}
+__host__ __device__ inline int solo_lds_doubles(int n, int S, int variant, int waves,
+                                                bool learned) {
+  static_assert(sizeof(MlpInfer) % 8 == 0, "copied by doubles");
+  return (S + 2) * 6 * n + ((n + 1) & ~1) + waves * solo_sums(variant) +
+         (learned ? static_cast<int>(sizeof(MlpInfer) / 8) : 0);
 }
 
 // Waves of the workgroup for systems of up to n bodies, 0 if they do not fit.
-inline int solo_waves(int n, int S, int variant) {
+inline int solo_waves(int n, int S, int variant, bool learned) {
   if (n < 1 || n > kSoloMaxN) return 0;
   for (int w : {kSoloWaves, 8}) {
     // fast, mixed: a thread per target and coordinate; more waves than units
@@ -62,16 +66,16 @@ inline int solo_waves(int n, int S, int variant) {
       if (w == kSoloWaves && n <= 128) continue;
       if (192 * ((n + 63) / 64) > 64 * w) continue;
     }
-    if (solo_lds_doubles(n, S, variant, w) <= kSoloLdsDoubles) return w;
+    if (solo_lds_doubles(n, S, variant, w, learned) <= kSoloLdsDoubles) return w;
   }
   return 0;
 }
 
 // Bodies up to which a solve is one workgroup's.
-inline int solo_limit(int S, int variant) {
+inline int solo_limit(int S, int variant, bool learned) {
   const int want = variant == ODEHIP_NBODY_EXACT ? kSoloExactN : kSoloSumN;
   for (int n = want; n > 0; --n)
-    if (solo_waves(n, S, variant) > 0) return n;
+    if (solo_waves(n, S, variant, learned) > 0) return n;
   return 0;
 }
 

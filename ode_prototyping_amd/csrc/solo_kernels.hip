@@ -14,6 +14,8 @@
 // kernels (rk_kernels.hip, ensemble_kernels.hip), so which of them runs a solve
 // changes no result.  A launch makes at most `attempts` attempts per system and
 // keeps what the next one needs in the state's global buffers.
+#include <type_traits>
+
 #include "ens_chunks.hpp"
 #include "mlp.hpp"
 #include "rk_device.hpp"
@@ -31,6 +33,18 @@ typedef ODEHIP_LDS double* lds_ptr;
 typedef const ODEHIP_LDS double* lds_cptr;
 
 extern __shared__ __attribute__((aligned(16))) double solo_lds[];
+
+// f(std::integral_constant<int, J>) for J = count in [Lo, Hi]: sums over the
+// stages unrolled, so that their loads go out together.
+template <int Lo, int Hi, typename F>
+__device__ __forceinline__ void with_count(int count, F&& f) {
+  if constexpr (Lo <= Hi) {
+    if (count == Lo)
+      f(std::integral_constant<int, Lo>{});
+    else
+      with_count<Lo + 1, Hi>(count, f);
+  }
+}
 
 // exact: the terms of blocks of kSoloTerms partners per wave go to LDS, waves
 // 0, 1, 2 add the block's x, y, z terms in partner order.  A target's own index
@@ -107,8 +121,9 @@ __device__ __forceinline__ void solo_groups(lds_cptr in, lds_cptr mass, lds_ptr 
       const double xi[1] = {in[3 * ic[0]]}, yi[1] = {in[3 * ic[0] + 1]},
                    zi[1] = {in[3 * ic[0] + 2]};
       double px[1] = {0.0}, py[1] = {0.0}, pz[1] = {0.0};
-      if constexpr (kVariant == ODEHIP_NBODY_FAST)
-        fast_group<kMass, kGuard, 1>(in, mass, j0, j1, ic, xi, yi, zi, eps2, px, py, pz);
+      if constexpr (!kNear)
+        lds_group<kVariant, kMass, kGuard>(in + 3 * j0, mass + j0, j0, j1 - j0, ic[0], xi[0],
+                                           yi[0], zi[0], eps2, px[0], py[0], pz[0]);
       else
         mixed_chunk<kMass, kGuard, kNear, 1>(in, mass, j0, j1, ic, xi, yi, zi, eps2, near2, px,
                                              py, pz);
@@ -149,14 +164,14 @@ template <int kVariant, bool kMass, bool kSpecial, bool kNear>
 __global__ __launch_bounds__(64 * kSoloWaves) void k_solo(SoloArgs a) {
   __shared__ SolverState st;
   __shared__ double quad_[kSoloMaxQuads];
-  __shared__ float mlp_x[16], mlp_h[64];
+  __shared__ MlpRowLds mlp_lds;
   lds_ptr quad = (lds_ptr)quad_;
   const int slot = a.list ? a.list[blockIdx.x] : 0;
   SolverState* gst = a.st + slot;
   if (gst->done) return;
   const EnsSys sy = a.sys ? a.sys[slot] : a.one;
   const int n = sy.n, nv = 6 * n, threads = blockDim.x, tid = threadIdx.x;
-  if (n < 1 || solo_lds_doubles(n, s_tab[a.tableau].S, kVariant, threads / 64) > a.lds_doubles)
+  if (n < 1 || solo_lds_doubles(n, s_tab[a.tableau].S, kVariant, threads / 64, a.mlp) > a.lds_doubles)
     return;  // does not fit what the launch set aside (uniform)
   const int lane = tid & 63, waves = threads >> 6;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -194,6 +209,14 @@ __global__ __launch_bounds__(64 * kSoloWaves) void k_solo(SoloArgs a) {
   const float near2 = kNear ? mixed_near2(a.near_c, n) : 0.0f;
   double* trace = a.trace ? a.trace + static_cast<size_t>(slot) * a.trace_cap * 3 : nullptr;
   const int n_quads = 4 * sy.n_groups;
+  // the network beside the system, for the same reason
+  const bool learned = st.controller == ODEHIP_CONTROLLER_LEARNED;
+  const MlpInfer* net = (const MlpInfer*)(work + waves * solo_sums(kVariant));
+  if (learned) {
+    uint64_t* to = (uint64_t*)net;
+    for (int e = tid; e < static_cast<int>(sizeof(MlpInfer) / 8); e += threads)
+      to[e] = reinterpret_cast<const uint64_t*>(a.mlp)[e];
+  }
 
   for (int att = 0; att < a.attempts; ++att) {
     const double dt = st.dt;
@@ -209,14 +232,20 @@ __global__ __launch_bounds__(64 * kSoloWaves) void k_solo(SoloArgs a) {
         if (kVariant == ODEHIP_NBODY_EXACT && kSpecial)
           for (int e = tid; e < 3 * n; e += threads) ok = ok & coord_shared_ok(x0[e]);
       } else {
-        for (int e = tid; e < nv; e += threads) {
-          double tmp = 0.0;  // stage_value (rk_device.hpp)
-          for (int j = 0; j < stage; ++j) tmp += T.a[stage - 1][j] * ks[j * nv + e];
-          const double v = x0[e] + tmp * dt;
-          y[e] = v;
-          if (kVariant == ODEHIP_NBODY_EXACT && kSpecial)
-            ok = ok & ((e >= 3 * n) | coord_shared_ok(v));
-        }
+        with_count<1, kMaxStages - 1>(stage, [&](auto J) {
+          const double* row = T.a[J - 1];
+          for (int e = tid; e < nv; e += threads) {
+            double k[J], tmp = 0.0;  // stage_value (rk_device.hpp)
+#pragma unroll
+            for (int j = 0; j < J; ++j) k[j] = ks[j * nv + e];
+#pragma unroll
+            for (int j = 0; j < J; ++j) tmp += row[j] * k[j];
+            const double v = x0[e] + tmp * dt;
+            y[e] = v;
+            if (kVariant == ODEHIP_NBODY_EXACT && kSpecial)
+              ok = ok & ((e >= 3 * n) | coord_shared_ok(v));
+          }
+        });
       }
       bool shared = false;
       if (kVariant == ODEHIP_NBODY_EXACT && kSpecial)
@@ -241,15 +270,18 @@ __global__ __launch_bounds__(64 * kSoloWaves) void k_solo(SoloArgs a) {
     }
     // new state, embedded error, scaled squared error by quads (k_ens_final);
     // whole waves, so that a quad is one wave's pass
+    with_count<2, kMaxStages>(S, [&](auto J) {
     for (int e0 = 64 * wave; e0 < 64 * n_quads; e0 += threads) {
       const int e = e0 + lane;
       double term = 0.0;
       if (e < nv) {
-        double xs = 0.0, es = 0.0;
-        for (int j = 0; j < S; ++j) {
-          const double kj = ks[j * nv + e];
-          xs += T.b[j] * kj;
-          es += T.db[j] * kj;
+        double k[J], xs = 0.0, es = 0.0;
+#pragma unroll
+        for (int j = 0; j < J; ++j) k[j] = ks[j * nv + e];
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+          xs += T.b[j] * k[j];
+          es += T.db[j] * k[j];
         }
         const double xo = x0[e];
         const double xv = xo + xs * dt, ev = es * dt;
@@ -263,10 +295,14 @@ __global__ __launch_bounds__(64 * kSoloWaves) void k_solo(SoloArgs a) {
       for (int s = 32; s >= 1; s >>= 1) term = term + __shfl_xor(term, s, 64);
       if (lane == 0) quad[e0 / 64] = term;
     }
+    });
     __syncthreads();
     if (wave == 0) {
       const double sum = lane == 0 ? solo_fold(quad, sy.n_groups) : 0.0;
-      ctrl_attempt_wave(&st, T, sum, nv, a.times, trace, a.mlp, n, mlp_x, mlp_h);
+      if (learned)
+        ctrl_attempt_wave(&st, T, sum, nv, a.times, trace, net, n, &mlp_lds);
+      else if (lane == 0)
+        ctrl_attempt(&st, T, sum, nv, a.times, trace);
     }
     __syncthreads();
     if (st.just_accepted)
@@ -301,10 +337,10 @@ hipError_t launch_solo(const SoloArgs& args, int n_max, int variant, unsigned bl
                        hipStream_t s) {
   SoloArgs a = args;
   const int S = host_tableau(a.tableau).S;
-  const int waves = solo_waves(n_max, S, variant);
+  const int waves = solo_waves(n_max, S, variant, a.mlp);
   if (waves == 0) return hipErrorInvalidValue;
   if (blocks == 0) return hipSuccess;
-  a.lds_doubles = solo_lds_doubles(n_max, S, variant, waves);
+  a.lds_doubles = solo_lds_doubles(n_max, S, variant, waves, a.mlp);
   void* k = nullptr;
   if (variant == ODEHIP_NBODY_EXACT)
     k = solo_kernel<ODEHIP_NBODY_EXACT, false>(a.mass, a.eps2 >= 0x1p-200 && a.eps2 <= 0x1p100);
