@@ -77,13 +77,6 @@ ODEHIP_HD inline dd div(dd a, dd b) {
   dd q = quick_two_sum(q1, q2);
   return add(q, dd{q3, 0.0});
 }
-ODEHIP_HD inline dd from_ratio(double num, double den) {
-  // num/den to double-double precision (num, den exact small integers).
-  double hi = num / den;
-  double lo = std::fma(-hi, den, num) / den;
-  return quick_two_sum(hi, lo);
-}
-
 // Exact power-of-two scaling through the exponent field.
 ODEHIP_HD inline double scale2(double v, int k) {
   // k is small (|k| < 1000 here); split to stay in the normal range.
@@ -97,6 +90,47 @@ ODEHIP_HD inline double scale2(double v, int k) {
   }
   return v * from_bits(static_cast<uint64_t>(k + 1023) << 52);
 }
+
+// 1 / (2k + 1), k = 0 .. 21, and 1 / k!, k = 0 .. 11, to double-double: 66
+// divisions a call were half of its time on the controller's one lane.
+constexpr dd kOddInverse[22] = {
+    {0x1.0000000000000p+0, 0x0.0p+0},
+    {0x1.5555555555555p-2, 0x1.5555555555555p-56},
+    {0x1.999999999999ap-3, -0x1.999999999999ap-57},
+    {0x1.2492492492492p-3, 0x1.2492492492492p-57},
+    {0x1.c71c71c71c71cp-4, 0x1.c71c71c71c71cp-58},
+    {0x1.745d1745d1746p-4, -0x1.745d1745d1746p-59},
+    {0x1.3b13b13b13b14p-4, -0x1.3b13b13b13b14p-58},
+    {0x1.1111111111111p-4, 0x1.1111111111111p-60},
+    {0x1.e1e1e1e1e1e1ep-5, 0x1.e1e1e1e1e1e1ep-61},
+    {0x1.af286bca1af28p-5, 0x1.af286bca1af28p-59},
+    {0x1.8618618618618p-5, 0x1.8618618618618p-59},
+    {0x1.642c8590b2164p-5, 0x1.642c8590b2164p-60},
+    {0x1.47ae147ae147bp-5, -0x1.eb851eb851eb8p-61},
+    {0x1.2f684bda12f68p-5, 0x1.2f684bda12f68p-59},
+    {0x1.1a7b9611a7b96p-5, 0x1.1a7b9611a7b96p-61},
+    {0x1.0842108421084p-5, 0x1.0842108421084p-60},
+    {0x1.f07c1f07c1f08p-6, -0x1.f07c1f07c1f08p-61},
+    {0x1.d41d41d41d41dp-6, 0x1.0750750750750p-60},
+    {0x1.bacf914c1bad0p-6, -0x1.bacf914c1bad0p-60},
+    {0x1.a41a41a41a41ap-6, 0x1.0690690690690p-60},
+    {0x1.8f9c18f9c18fap-6, -0x1.f3831f3831f38p-61},
+    {0x1.7d05f417d05f4p-6, 0x1.7d05f417d05f4p-62},
+};
+constexpr dd kInverseFactorial[12] = {
+    {0x1.0000000000000p+0, 0x0.0p+0},
+    {0x1.0000000000000p+0, 0x0.0p+0},
+    {0x1.0000000000000p-1, 0x0.0p+0},
+    {0x1.5555555555555p-3, 0x1.5555555555555p-57},
+    {0x1.5555555555555p-5, 0x1.5555555555555p-59},
+    {0x1.1111111111111p-7, 0x1.1111111111111p-63},
+    {0x1.6c16c16c16c17p-10, -0x1.f49f49f49f49fp-65},
+    {0x1.a01a01a01a01ap-13, 0x1.a01a01a01a01ap-73},
+    {0x1.a01a01a01a01ap-16, 0x1.a01a01a01a01ap-76},
+    {0x1.71de3a556c734p-19, -0x1.c154f8ddc6c00p-73},
+    {0x1.27e4fb7789f5cp-22, 0x1.cbbc05b4fa99ap-76},
+    {0x1.ae64567f544e4p-26, -0x1.c062e06d1f209p-80},
+};
 
 // ln 2 to ~107 bits.
 constexpr double kLn2Hi = 6.93147180559945286227e-01;
@@ -118,9 +152,10 @@ ODEHIP_HD inline dd log_dd(double x) {
   dd u = div(num, den);
   dd w = mul(u, u);
   // sum_{k=0}^{21} w^k / (2k+1), Horner from the top.
-  dd s = from_ratio(1.0, 43.0);
+  dd s = kOddInverse[21];
+#pragma unroll
   for (int k = 20; k >= 0; --k) {
-    s = add(mul(s, w), from_ratio(1.0, 2.0 * k + 1.0));
+    s = add(mul(s, w), kOddInverse[k]);
   }
   dd lm = mul(mul_d(u, 2.0), s);
   dd le = add(two_prod(static_cast<double>(e), kLn2Hi),
@@ -137,12 +172,10 @@ ODEHIP_HD inline double exp_dd_round(dd z) {
   // r' = r / 256 (exact)
   dd rp{r.hi * 0.00390625, r.lo * 0.00390625};
   // s = exp(r') - 1 = r' + r'^2/2! + ... + r'^11/11!
-  dd s = from_ratio(1.0, 39916800.0);  // 1/11!
-  double fact[11] = {1.0,      2.0,       6.0,        24.0,        120.0,
-                     720.0,    5040.0,    40320.0,    362880.0,    3628800.0,
-                     39916800.0};
+  dd s = kInverseFactorial[11];
+#pragma unroll
   for (int n = 10; n >= 1; --n) {
-    s = add(mul(s, rp), from_ratio(1.0, fact[n - 1]));
+    s = add(mul(s, rp), kInverseFactorial[n]);
   }
   s = mul(s, rp);
   for (int i = 0; i < 8; ++i) {

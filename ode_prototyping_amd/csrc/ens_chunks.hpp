@@ -98,14 +98,15 @@ __device__ __forceinline__ void mixed_terms(const double (&c)[3 * U], const doub
 }
 
 // The sum over one group of `count` partners from j0 on, in LDS at p (3 doubles
-// each) with masses at m; p, m, j0 and count may differ between the lanes.
-template <int kVariant, bool kMass, bool kGuard>
+// each) with masses at m; p, m, j0 and count may differ between the lanes.  U
+// partners a step: more of them hide a lone wave's latencies, fewer leave room for
+// other waves.
+template <int kVariant, bool kMass, bool kGuard, int U>
 __device__ __forceinline__ void lds_group(const __attribute__((address_space(3))) double* p,
                                           const __attribute__((address_space(3))) double* m,
                                           int j0, int count, int i, double xi, double yi,
                                           double zi, double eps2, double& ax, double& ay,
                                           double& az) {
-  constexpr int U = 4;
   float fx = 0.0f, fy = 0.0f, fz = 0.0f;
   ax = ay = az = 0.0;
   const float eps2f = static_cast<float>(eps2);

@@ -649,10 +649,10 @@ __global__ __launch_bounds__(64 * kFineWaves) void k_ens_rhs_fine(EnsBufs b, con
       const int j0 = r0 + g * kEnsGroup;
       double sx, sy_, sz;
       if (kMass && per_term)
-        lds_group<kVariant, true, kSpecial>(pos + g * kFineStride, mass + g * (kEnsGroup + 1), j0,
+        lds_group<kVariant, true, kSpecial, 4>(pos + g * kFineStride, mass + g * (kEnsGroup + 1), j0,
                                             have, i, xi, yi, zi, b.eps2, sx, sy_, sz);
       else
-        lds_group<kVariant, false, kSpecial>(pos + g * kFineStride, mass, j0, have, i, xi, yi, zi,
+        lds_group<kVariant, false, kSpecial, 4>(pos + g * kFineStride, mass, j0, have, i, xi, yi, zi,
                                              b.eps2, sx, sy_, sz);
       part[g][t] = sx;
       part[g][T + t] = sy_;
@@ -743,7 +743,7 @@ __global__ __launch_bounds__(kBlock) void k_ens_final(EnsBufs b) {
     __shared__ MlpRowLds lds;
     ctrl_attempt_wave(&ls, T, sum, 6 * static_cast<size_t>(sy.n), nullptr, trace,
                       static_cast<const MlpInfer*>(b.mlp), sy.n, &lds);
-  } else if (threadIdx.x == 0) {
+  } else {
     ctrl_attempt(&ls, T, sum, 6 * static_cast<size_t>(sy.n), nullptr, trace);
   }
   wave_lds_fence();

@@ -50,13 +50,17 @@ struct SolverState {
 
 // What a right-hand-side launch of an attempt does with each element of the
 // stage vector k_n it writes: the next stage's input there,
-// x0 + dt (a_0 k_0 + ... + a_n k_n), with row n of the tableau's a.
+// x0 + dt (a_0 k_0 + ... + a_n k_n), with row n of the tableau's a.  A leapfrog
+// step's launch writes the next launch's state there instead (n < 0): the
+// velocities after this step, and the positions moved on with them.
 struct NextStage {
   double* y;             // that input, or null: none
-  const double* ks;      // the attempt's stage vectors
-  int n;                 // index of the one being written
+  const double* ks;      // the attempt's stage vectors; the last step's accelerations
+  int n;                 // index of the one being written, kLeapMove or kLeapStay
   int tab;
 };
+constexpr int kLeapMove = -1;  // positions of the next step
+constexpr int kLeapStay = -2;  // the last step: positions kept
 
 // Arguments of the N-body RHS kernels.  Exactly one of y / (xb0, xb1, st)
 // selects the input state: y if non-null, else the x0 buffer st->cur names.
@@ -74,7 +78,8 @@ struct NBodyArgs {
   double eps2;
   float near2;          // mixed variant: pairs with FP32 r^2 below this are
                         // computed in FP64 (0: none)
-  NextStage next;       // (solve only)
+  NextStage next;       // (solves and leapfrog only)
+  double leap_dt;       // leapfrog step
 };
 
 // Near-field threshold of the mixed RHS for a system of n bodies: pairs with

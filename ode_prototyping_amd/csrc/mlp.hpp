@@ -168,12 +168,6 @@ __device__ inline MlpRowWeights mlp_row_weights(const MlpInfer* M) {
   return w;
 }
 
-// Orders a wave's own LDS writes before its later reads.
-__device__ inline void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 __device__ inline float mlp_row_forward(const MlpRowWeights& w, const float* x, float* h) {
   const int lane = threadIdx.x & 63;
   const int r = lane & 15;
@@ -278,7 +272,7 @@ __device__ inline void ctrl_attempt_wave(SolverState* st, const Tableau& T, doub
   const float f = mlp_feature(M, lds->arg, lane < 16 ? lane : 15);
   if (lane < 16) lds->x[lane] = f;
   const float out = mlp_row_forward(w, lds->x, lds->h);
-  if (lane == 0 && judged) ctrl_step(st, accept, mlp_ratio(out));
+  ctrl_step_wave(st, judged, accept, mlp_ratio(out));
 }
 
 // The solve state from global memory to LDS and back, by one wave: the

@@ -66,9 +66,20 @@ __device__ inline NBodyArgs late_args() {
 template <int L>
 __device__ inline void put(const NBodyArgs& a, long e, double v) {
   a.k[e] = v;
-  if (a.next.y)
+  if (!a.next.y) return;
+  if (a.next.n >= 0) {
     next_stage<L>(a.next, n_tab[a.next.tab], 6 * static_cast<size_t>(a.n), e, v,
                   (a.st->cur ? a.xb1 : a.xb0)[e], a.st->dt);
+    return;
+  }
+  // update_velocity_kernel, then the next step's update_position_kernel
+  // (LeapfrogParallel.hpp:57-68)
+  const long p = e - 3L * a.n;
+  if (p < 0) return;
+  const double dt = a.leap_dt, x = a.y[p];
+  const double vel = a.y[e] + 0.5 * dt * (a.next.ks[p] + v);
+  a.next.y[e] = vel;
+  a.next.y[p] = a.next.n == kLeapMove ? x + dt * (vel + 0.5 * dt * v) : x;
 }
 
 // Returns true if the launch has nothing to compute (solve finished, or k1

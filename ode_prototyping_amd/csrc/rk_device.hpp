@@ -245,38 +245,44 @@ __device__ inline bool ctrl_judge(SolverState* st, const Tableau& T,
 // (err_prev/err)^(0.4/k), k = 1 + q -- the reference controller's steady
 // error 0.38 --, err_prev the error of the last accepted step (1e-4 before
 // the first one, floored at 1e-4), no growth right after a rejection.
-__device__ inline double pi_proposal(const SolverState* st, double err,
-                                     bool accept) {
+// The two powers, `which` = 0, 1: a wave's first two lanes take one each.
+__device__ inline double pi_power(const SolverState* st, double err, int which) {
   const double k_inv = st->inv_q1;
-  double fac = cr_pow(0.38 / err, 0.3 * k_inv) * cr_pow(st->err_prev / err, 0.4 * k_inv);
+  return cr_pow((which ? st->err_prev : 0.38) / err, (which ? 0.4 : 0.3) * k_inv);
+}
+__device__ inline double pi_proposal(const SolverState* st, double power0, double power1,
+                                     bool accept) {
+  double fac = power0 * power1;
   if (!accept && fac > 1.0) fac = 1.0;
   return st->dt * fac;
+}
+
+// Whether a judged attempt's step comes from the PI controller: always its own,
+// the learned one's before three attempts of history exist, after two rejections
+// in a row or when its ratio is not finite.
+__device__ inline bool pi_steps(const SolverState* st, double learned_ratio) {
+  if (st->controller == ODEHIP_CONTROLLER_PI) return true;
+  return st->controller == ODEHIP_CONTROLLER_LEARNED &&
+         !(std::isfinite(learned_ratio) && st->attempts >= 3 && st->rejects_in_row < 2);
 }
 
 // Second half (RKEmbeddedParallel.hpp:64-79): the new step size, its clamps
 // and the clip to tf, then the termination tests.  `learned_ratio` is the
 // learned controller's proposed dt_new / dt (ODEHIP_CONTROLLER_LEARNED only,
-// capped at 1 right after a rejection); the PI proposal replaces it when it
-// is not finite, before three attempts of history exist, or after two
-// rejections in a row.
-__device__ inline void ctrl_step(SolverState* st, bool accept,
-                                 double learned_ratio) {
+// capped at 1 right after a rejection); `power0` and `power1` (pi_power) are
+// read where pi_steps says so.
+__device__ inline void ctrl_step(SolverState* st, bool accept, double learned_ratio,
+                                 double power0, double power1) {
   const double scaled_error = st->err;
   double dt = st->dt;
   const double t = st->t;
   double dtnew;
-  if (st->controller == ODEHIP_CONTROLLER_PI) {
-    dtnew = pi_proposal(st, scaled_error, accept);
+  if (pi_steps(st, learned_ratio)) {
+    dtnew = pi_proposal(st, power0, power1, accept);
   } else if (st->controller == ODEHIP_CONTROLLER_LEARNED) {
-    const bool usable = std::isfinite(learned_ratio) && st->attempts >= 3 &&
-                        st->rejects_in_row < 2;
-    if (usable) {
-      // no growth right after a rejection
-      dtnew = dt * ((!accept && learned_ratio > 1.0) ? 1.0 : learned_ratio);
-      st->learned_steps += 1;
-    } else {
-      dtnew = pi_proposal(st, scaled_error, accept);
-    }
+    // no growth right after a rejection
+    dtnew = dt * ((!accept && learned_ratio > 1.0) ? 1.0 : learned_ratio);
+    st->learned_steps += 1;
   } else {
     dtnew = dt * st->safety / cr_root(scaled_error, st->inv_q1, st->root_k);
   }
@@ -307,13 +313,33 @@ __device__ inline void ctrl_step(SolverState* st, bool accept,
   }
 }
 
-// A whole attempt end with the reference or PI controller.
+// Orders a wave's own LDS writes before its later reads.
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// The step of a judged attempt by one wave (every lane calls; `judged` and
+// `learned_ratio` are lane 0's).  `st`, in LDS, is this wave's alone to change.
+__device__ inline void ctrl_step_wave(SolverState* st, bool judged, bool accept,
+                                      double learned_ratio) {
+  const int lane = threadIdx.x & 63;
+  double power = 1.0;
+  wave_lds_fence();
+  if (__any(lane == 0 && judged && pi_steps(st, learned_ratio)) && lane < 2)
+    power = pi_power(st, st->err, lane);
+  const double power1 = __shfl(power, 1, 64);
+  if (lane == 0 && judged) ctrl_step(st, accept, learned_ratio, power, power1);
+}
+
+// A whole attempt end with the reference or PI controller, by one wave (`sum` is
+// read in lane 0).
 __device__ inline void ctrl_attempt(SolverState* st, const Tableau& T,
                                     double sum, size_t n_var, double* times,
                                     double* trace) {
-  bool accept = false;
-  if (ctrl_judge(st, T, sum, n_var, times, trace, &accept))
-    ctrl_step(st, accept, NAN);
+  bool accept = false, judged = false;
+  if ((threadIdx.x & 63) == 0) judged = ctrl_judge(st, T, sum, n_var, times, trace, &accept);
+  ctrl_step_wave(st, judged, accept, NAN);
 }
 
 // ------------------------------------------------------- dense output ----

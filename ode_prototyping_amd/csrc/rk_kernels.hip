@@ -125,7 +125,7 @@ __global__ __launch_bounds__(kBlock) void k_final_dev(
   if constexpr (kLearned) {
     __shared__ MlpRowLds lds;
     ctrl_attempt_wave(&ls, T, sum, n_var, times, trace, M, n_particles, &lds);
-  } else if (threadIdx.x == 0) {
+  } else {
     ctrl_attempt(&ls, T, sum, n_var, times, trace);
   }
   wave_lds_fence();

@@ -80,12 +80,22 @@ __device__ __forceinline__ void solo_exact(lds_cptr in, lds_cptr mass, lds_ptr k
         const int cnt = min(B, (n - jb + kSoloTerms - 1) / kSoloTerms * kSoloTerms);
         lds_cptr t = term + wave * B * 64 + lane;
         int q = 0;
-        for (; q + 16 <= cnt; q += 16) {
-          double v[16];
+        if (cnt >= 16) {  // the next 16 terms come in while 16 are added
+          double v[2][16];
 #pragma unroll
-          for (int u = 0; u < 16; ++u) v[u] = t[(q + u) * 64];
+          for (int u = 0; u < 16; ++u) v[0][u] = t[u * 64];
+          for (; q + 32 <= cnt; q += 16) {
 #pragma unroll
-          for (int u = 0; u < 16; ++u) acc += v[u];
+            for (int u = 0; u < 16; ++u) v[1][u] = t[(q + 16 + u) * 64];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < 16; ++u) acc += v[0][u];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) v[0][u] = v[1][u];
+          }
+#pragma unroll
+          for (int u = 0; u < 16; ++u) acc += v[0][u];
+          q += 16;
         }
         for (; q < cnt; q += kSoloTerms) {
 #pragma unroll
@@ -122,7 +132,7 @@ __device__ __forceinline__ void solo_groups(lds_cptr in, lds_cptr mass, lds_ptr 
                    zi[1] = {in[3 * ic[0] + 2]};
       double px[1] = {0.0}, py[1] = {0.0}, pz[1] = {0.0};
       if constexpr (!kNear)
-        lds_group<kVariant, kMass, kGuard>(in + 3 * j0, mass + j0, j0, j1 - j0, ic[0], xi[0],
+        lds_group<kVariant, kMass, kGuard, kMass || kGuard ? 4 : 8>(in + 3 * j0, mass + j0, j0, j1 - j0, ic[0], xi[0],
                                            yi[0], zi[0], eps2, px[0], py[0], pz[0]);
       else
         mixed_chunk<kMass, kGuard, kNear, 1>(in, mass, j0, j1, ic, xi, yi, zi, eps2, near2, px,
@@ -164,6 +174,7 @@ template <int kVariant, bool kMass, bool kSpecial, bool kNear>
 __global__ __launch_bounds__(64 * kSoloWaves) void k_solo(SoloArgs a) {
   __shared__ SolverState st;
   __shared__ double quad_[kSoloMaxQuads];
+  __shared__ int wide[kMaxStages];  // exact: a coordinate of the stage fails coord_shared_ok
   __shared__ MlpRowLds mlp_lds;
   lds_ptr quad = (lds_ptr)quad_;
   const int slot = a.list ? a.list[blockIdx.x] : 0;
@@ -221,6 +232,11 @@ __global__ __launch_bounds__(64 * kSoloWaves) void k_solo(SoloArgs a) {
   for (int att = 0; att < a.attempts; ++att) {
     const double dt = st.dt;
     const int k1_valid = st.k1_valid;
+    if (kVariant == ODEHIP_NBODY_EXACT && kSpecial) {
+      // (read last before the final pass's barrier of the attempt before)
+      if (tid < kMaxStages) wide[tid] = 0;
+      __syncthreads();
+    }
     for (int stage = 0; stage < S; ++stage) {
       lds_cptr in = stage == 0 ? x0 : y;
       lds_ptr kout = ks + stage * nv;
@@ -247,14 +263,12 @@ __global__ __launch_bounds__(64 * kSoloWaves) void k_solo(SoloArgs a) {
           }
         });
       }
-      bool shared = false;
-      if (kVariant == ODEHIP_NBODY_EXACT && kSpecial)
-        shared = __syncthreads_and(ok) != 0;
-      else
-        __syncthreads();
+      if (kVariant == ODEHIP_NBODY_EXACT && kSpecial && !__all(ok) && lane == 0) wide[stage] = 1;
+      __syncthreads();
+      const bool shared = kVariant == ODEHIP_NBODY_EXACT && kSpecial && wide[stage] == 0;
       for (int e = tid; e < 3 * n; e += threads) kout[e] = in[3 * n + e];
       if constexpr (kVariant == ODEHIP_NBODY_EXACT) {
-        if (kSpecial && shared)
+        if (shared)
           solo_exact<kMass, true>(in, mass, kout, work, n, a.eps2, wave, waves, lane);
         else
           solo_exact<kMass, false>(in, mass, kout, work, n, a.eps2, wave, waves, lane);
@@ -301,7 +315,7 @@ __global__ __launch_bounds__(64 * kSoloWaves) void k_solo(SoloArgs a) {
       const double sum = lane == 0 ? solo_fold(quad, sy.n_groups) : 0.0;
       if (learned)
         ctrl_attempt_wave(&st, T, sum, nv, a.times, trace, net, n, &mlp_lds);
-      else if (lane == 0)
+      else
         ctrl_attempt(&st, T, sum, nv, a.times, trace);
     }
     __syncthreads();
