@@ -405,8 +405,8 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
                                 opt->max_attempts, opt->fsal ? 1 : 0, opt->controller, s));
   HIP_TRY(ctx, ens_enqueue_initial_step(b, s));
 
-  // The one-workgroup solves: launches of kSoloAttempts attempts, two ahead of
-  // the host, until their count of running systems has been seen at zero.
+  // The one-workgroup solves: launches of kSoloTicks, two ahead of the host,
+  // until their count of running systems has been seen at zero.
   SoloArgs sa{};
   long solo_pushed = 0, solo_seen = 0;
   bool solo_done = solo.empty();
@@ -459,7 +459,6 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
     sa.eps2 = b.eps2;
     sa.near_c = b.near_c;
     sa.tableau = tableau;
-    sa.attempts = kSoloAttempts;
     HIP_TRY(ctx, hipEventRecord(w->ev_fork, s));
     HIP_TRY(ctx, hipStreamWaitEvent(w->side, w->ev_fork, 0));
     if ((rc = poll_solo(false))) return rc;

@@ -611,34 +611,75 @@ __global__ __launch_bounds__(64 * kFineWaves) void k_ens_rhs_fine(EnsBufs b, con
   const int n = sy.n, i0 = tile.i0 + T * static_cast<int>(blockIdx.y);
   if (i0 >= n) return;
   const SolverState* st = b.st ? b.st + tile.sys : nullptr;
-  if (st && (stage0 == 2 ? st->dense_go == 0 : st->done)) return;
+  constexpr int kThreads = 64 * kFineWaves;
+  constexpr int kRound = kFineGroups * kEnsGroup;  // partners
+  constexpr int kStage = 3 * kRound / kThreads;    // coordinates per thread and round
+  // What the workgroup needs of memory goes out at once -- system state, partners
+  // and targets (of a stage; a k1's depend on which buffer is current), the
+  // stage vectors behind the next stage's input --: one after the other, these
+  // latencies were half of a small launch.
+  const int done = st ? (stage0 == 2 ? st->dense_go == 0 : st->done) : 0;
+  const int k1_valid = st ? st->k1_valid : 0;
+  const double* x0 = st && st->cur ? b.xb1 : b.xb0;
+  const double dt = st ? st->dt : 0.0;
+  const double* y = (y_in ? y_in : x0) + sy.eoff;
+  const int slot = lane / T, t = lane % T;
+  const int i = min(i0 + t, n - 1);
+  double first[kStage];
+#pragma unroll
+  for (int s = 0; s < kStage; ++s) {
+    const int e = threadIdx.x + s * kThreads;
+    first[s] = y[e < 3 * n ? e : 0];
+  }
+  const double xi = y[3 * i], yi = y[3 * i + 1], zi = y[3 * i + 2];
+  // a thread's element of the result: 0 .. 3T - 1 accelerations, 3T .. 6T - 1
+  // velocities
+  const int f = threadIdx.x;
+  const bool is_acc = f < 3 * T;
+  const int fi = is_acc ? i0 + f % T : i0 + (f - 3 * T) / 3;
+  const bool has = f < 6 * T && fi < n;
+  const long fe = is_acc ? 3L * n + 3L * fi + f / T : 3L * i0 + f - 3 * T;
+  const double vel = has && !is_acc ? y[3L * n + fe] : 0.0;
+  const size_t ge = static_cast<size_t>(sy.eoff + fe);
+  double tmp = 0.0, x0e = 0.0;
+  if (next.y && has) {
+    // (next_stage, its sum up to the vector this launch adds)
+    double v[kStageLoads];
+#pragma unroll
+    for (int s = 0; s < kStageLoads; ++s)
+      v[s] = s < next.n ? next.ks[static_cast<size_t>(s) * b.nv + ge] : 0.0;
+    x0e = x0[ge];
+#pragma unroll
+    for (int s = 0; s < kStageLoads; ++s)
+      if (s < next.n) tmp += e_tab[next.tab].a[next.n][s] * v[s];
+  }
+  if (done) return;
   const auto out = ens_sink<kStageLoads>(b, next, st, k_out, sy);
-  if (st && stage0 == 1 && st->k1_valid) {
+  if (st && stage0 == 1 && k1_valid) {
     if (wave == 0) tile_reuse_k1(b, st, out, n, i0, T);
     return;
   }
-  const double* y = (y_in ? y_in : (st->cur ? b.xb1 : b.xb0)) + sy.eoff;
+  auto put = [&](double v) {
+    out.k[fe] = v;
+    if (next.y) next.y[ge] = x0e + (tmp + e_tab[next.tab].a[next.n][next.n] * v) * dt;
+  };
   const double* m = kMass ? b.mass + sy.eoff / 6 : nullptr;
   // equal masses: unit-mass terms, each finished sum scaled once (as k_ens_rhs)
   const double m_uni = kMass ? system_uniform_mass(st, m, n) : 0.0;
   const bool per_term = kMass && m_uni == 0.0;
   const double scale = per_term || !kMass ? 1.0 : m_uni;
-  const int slot = lane / T, t = lane % T;
-  const int i = min(i0 + t, n - 1);
-  const double xi = y[3 * i], yi = y[3 * i + 1], zi = y[3 * i + 2];
-  // a thread's velocity element, written at the end
-  const int f = threadIdx.x;  // 0 .. 3T - 1: accelerations; 3T .. 6T - 1: velocities
-  const long ve = 3L * i0 + f - 3 * T;
-  const bool has_v = f >= 3 * T && f < 6 * T && ve < 3L * n;
-  const double vel = has_v ? y[3L * n + ve] : 0.0;
   auto* pos = (__attribute__((address_space(3))) double*)pos_;
   auto* mass = (__attribute__((address_space(3))) double*)mass_;
-  constexpr int kRound = kFineGroups * kEnsGroup;  // partners
   double acc = 0.0, chunk = 0.0;
   for (int r0 = 0; r0 < n; r0 += kRound) {
     const int cnt = min(kRound, n - r0);
-    for (int e = threadIdx.x; e < 3 * cnt; e += 64 * kFineWaves)
-      pos[e / (3 * kEnsGroup) * kFineStride + e % (3 * kEnsGroup)] = y[3 * r0 + e];
+#pragma unroll
+    for (int s = 0; s < kStage; ++s) {
+      const int e = threadIdx.x + s * kThreads;
+      if (e < 3 * cnt)
+        pos[e / (3 * kEnsGroup) * kFineStride + e % (3 * kEnsGroup)] =
+            r0 == 0 ? first[s] : y[3 * r0 + e];
+    }
     if (per_term)
       for (int e = threadIdx.x; e < cnt; e += 64 * kFineWaves)
         mass[e / kEnsGroup * (kEnsGroup + 1) + e % kEnsGroup] = m[r0 + e];
@@ -659,7 +700,7 @@ __global__ __launch_bounds__(64 * kFineWaves) void k_ens_rhs_fine(EnsBufs b, con
       part[g][2 * T + t] = sz;
     }
     __syncthreads();
-    if (f < 3 * T) {
+    if (is_acc) {
       const int groups = (cnt + kEnsGroup - 1) / kEnsGroup;
       constexpr int kPer = kEnsChunk / kEnsGroup;
       int q = 0;
@@ -677,11 +718,7 @@ __global__ __launch_bounds__(64 * kFineWaves) void k_ens_rhs_fine(EnsBufs b, con
     }
     if (r0 + kRound < n) __syncthreads();  // LDS is written again
   }
-  if (f < 3 * T) {
-    const long e = 3L * (i0 + f % T) + f / T;
-    if (i0 + f % T < n) out.put(3L * n + e, acc * scale);
-  }
-  if (has_v) out.put(ve, vel);
+  if (has) put(is_acc ? acc * scale : vel);
 }
 
 // ------------------------------------------------------ element kernels --
@@ -731,10 +768,9 @@ __global__ __launch_bounds__(kBlock) void k_ens_final(EnsBufs b) {
     if (st->fsal && T.fsal) b.kfsal[p.e] = b.ks[(T.S - 1) * b.nv + p.e];
   }
   const double g = group_reduce(term);
-  if (threadIdx.x == 0) b.partA[p.g] = g;
   const EnsSys sy = b.sys[p.sys];
-  if (!last_group(st, sy.n_groups)) return;
-  const double sum = fold_partials_block(b.partA + sy.gbase, sy.n_groups);
+  if (!last_group(st, sy.n_groups, b.partA + p.g, g)) return;
+  const double sum = fold_partials_block<true>(b.partA + sy.gbase, sy.n_groups);
   __shared__ SolverState ls;
   if (threadIdx.x >= 64) return;
   state_words(&ls, st);

@@ -710,7 +710,6 @@ int odehip_rk_solve(odehip_context* ctx, int tableau, const odehip_ode* ode,
                     states_cap == 0 && b.n_particles <= solo_limit(S, ode->nbody_variant, b.mlp != nullptr);
   SoloArgs sa{};
   if (solo) {
-    K = kSoloAttempts;
     sa.one = EnsSys{0, b.n_particles, 0, n_groups_for(n), 0};
     sa.st = b.st;
     sa.xb0 = b.xb0;
@@ -726,7 +725,6 @@ int odehip_rk_solve(odehip_context* ctx, int tableau, const odehip_ode* ode,
     sa.mlp = b.mlp;
     sa.eps2 = b.eps2;
     sa.tableau = tableau;
-    sa.attempts = K;
   }
   if (K > 0 && !solo) {
     GraphKey key;
@@ -786,7 +784,6 @@ int odehip_rk_solve(odehip_context* ctx, int tableau, const odehip_ode* ode,
   for (;;) {
     if (solo) {
       HIP_TRY(ctx, launch_solo(sa, b.n_particles, ode->nbody_variant, 1, s));
-      launched += K;
     } else if (K > 0) {
       HIP_TRY(ctx, hipGraphLaunch(ctx->exec, s));
       launched += K;

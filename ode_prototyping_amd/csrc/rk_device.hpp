@@ -45,14 +45,19 @@ __device__ inline double fold_partials(const double* p, int n_groups) {
 // The same fold, called by every thread of a block: the partials are first
 // staged through LDS (coalesced), kFoldLds at a time, then thread 0 adds them in
 // order from LDS.  Returns the sum in thread 0.
+// kCoherent: of partials that other workgroups of this launch have written
+// (last_group).
 constexpr int kFoldLds = 512;
+template <bool kCoherent = false>
 __device__ inline double fold_partials_block(const double* p, int n_groups) {
   __shared__ double buf[kFoldLds];
   double r = 0.0;
   for (int g0 = 0; g0 < n_groups; g0 += kFoldLds) {
     const int cnt = min(kFoldLds, n_groups - g0);
     if (g0 > 0) __syncthreads();
-    for (int g = threadIdx.x; g < cnt; g += blockDim.x) buf[g] = p[g0 + g];
+    for (int g = threadIdx.x; g < cnt; g += blockDim.x)
+      buf[g] = kCoherent ? __hip_atomic_load(p + g0 + g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                         : p[g0 + g];
     __syncthreads();
     if (threadIdx.x == 0) {
 #pragma unroll 8
@@ -111,21 +116,24 @@ __device__ inline void update_values(const Tableau& T, double dt,
   err = es * dt;
 }
 
-// Called by every thread of a workgroup of an attempt's final pass once thread 0
-// has written the workgroup's partial: true in the last of the n_groups
-// workgroups, which then sees every partial and may change the solve's state.
-// (The fences make the partials visible between the XCDs' L2s.)
-__device__ inline bool last_group(SolverState* st, int n_groups) {
+// Called by every thread of a workgroup of an attempt's final pass, `partial` (its
+// group's sum, in thread 0) going to *slot: true in the last of the n_groups
+// workgroups, which then may fold every partial (fold_partials_block<true>) and
+// change the solve's state.  The partials alone pass between workgroups here, so
+// they are written and read past the XCDs' L2s, each store complete before its
+// group is counted; a fence would write the whole L2 back, which 1000 groups made
+// 50 us of.
+__device__ inline bool last_group(SolverState* st, int n_groups, double* slot, double partial) {
   __shared__ int last;
   if (threadIdx.x == 0) {
-    __threadfence();
-    last = atomicAdd(&st->arrived, 1) == n_groups - 1;
+    __hip_atomic_store(slot, partial, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    last = __hip_atomic_fetch_add(&st->arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+           n_groups - 1;
     if (last) st->arrived = 0;
   }
   __syncthreads();
-  if (!last) return false;
-  __threadfence();
-  return true;
+  return last != 0;
 }
 
 // ---------------------------------------------------------- controller ----

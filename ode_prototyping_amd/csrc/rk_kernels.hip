@@ -116,9 +116,8 @@ __global__ __launch_bounds__(kBlock) void k_final_dev(
     if (st->fsal && T.fsal) kfsal[i] = ks[(T.S - 1) * n_var + i];
   }
   const double g = group_reduce(term);
-  if (threadIdx.x == 0) partials[blockIdx.x] = g;
-  if (!last_group(st, gridDim.x)) return;
-  const double sum = fold_partials_block(partials, gridDim.x);
+  if (!last_group(st, gridDim.x, partials + blockIdx.x, g)) return;
+  const double sum = fold_partials_block<true>(partials, gridDim.x);
   __shared__ SolverState ls;
   if (threadIdx.x >= 64) return;
   state_words(&ls, st);

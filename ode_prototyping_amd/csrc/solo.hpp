@@ -14,7 +14,7 @@ constexpr int kSoloTerms = 4;     // exact: partners per wave and block
 constexpr int kSoloMaxN = 320;    // fast, mixed: 192 threads per 64 targets
 constexpr int kSoloExactN = 128;  // sizes up to which it is the faster form
 constexpr int kSoloSumN = 256;
-constexpr int kSoloAttempts = 64; // per launch
+constexpr uint64_t kSoloTicks = 200000;  // of the 100 MHz clock: 2 ms a launch
 constexpr int kSoloMaxQuads = 4 * ((6 * kSoloMaxN + ODEHIP_REDUCE_GROUP - 1) / ODEHIP_REDUCE_GROUP);
 // LDS of a CU less the kernel's static use and some to spare.
 constexpr int kSoloLdsDoubles = (160 * 1024 - 2048) / 8;
@@ -40,7 +40,6 @@ struct SoloArgs {
   double eps2;
   double near_c;
   int tableau;
-  int attempts;        // of this launch, per system
   int lds_doubles;     // set by launch_solo
 };
 

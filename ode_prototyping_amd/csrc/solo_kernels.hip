@@ -12,8 +12,9 @@
 //
 // Every number is computed by the functions and in the order of the lockstep
 // kernels (rk_kernels.hip, ensemble_kernels.hip), so which of them runs a solve
-// changes no result.  A launch makes at most `attempts` attempts per system and
-// keeps what the next one needs in the state's global buffers.
+// changes no result.  A workgroup starts no attempt once kSoloTicks have passed
+// and keeps what the next launch needs in the state's global buffers: launches
+// of bounded time, whose systems need not wait for one another's attempts.
 #include <type_traits>
 
 #include "ens_chunks.hpp"
@@ -176,6 +177,7 @@ __global__ __launch_bounds__(64 * kSoloWaves) void k_solo(SoloArgs a) {
   __shared__ double quad_[kSoloMaxQuads];
   __shared__ int wide[kMaxStages];  // exact: a coordinate of the stage fails coord_shared_ok
   __shared__ MlpRowLds mlp_lds;
+  __shared__ int stop;  // no further attempt in this launch
   lds_ptr quad = (lds_ptr)quad_;
   const int slot = a.list ? a.list[blockIdx.x] : 0;
   SolverState* gst = a.st + slot;
@@ -229,7 +231,8 @@ __global__ __launch_bounds__(64 * kSoloWaves) void k_solo(SoloArgs a) {
       to[e] = reinterpret_cast<const uint64_t*>(a.mlp)[e];
   }
 
-  for (int att = 0; att < a.attempts; ++att) {
+  const uint64_t start = __builtin_amdgcn_s_memrealtime();
+  for (;;) {
     const double dt = st.dt;
     const int k1_valid = st.k1_valid;
     if (kVariant == ODEHIP_NBODY_EXACT && kSpecial) {
@@ -317,11 +320,12 @@ __global__ __launch_bounds__(64 * kSoloWaves) void k_solo(SoloArgs a) {
         ctrl_attempt_wave(&st, T, sum, nv, a.times, trace, net, n, &mlp_lds);
       else
         ctrl_attempt(&st, T, sum, nv, a.times, trace);
+      if (lane == 0) stop = st.done || __builtin_amdgcn_s_memrealtime() - start >= kSoloTicks;
     }
     __syncthreads();
     if (st.just_accepted)
       for (int e = tid; e < nv; e += threads) x0[e] = y[e];
-    if (st.done) break;
+    if (stop) break;
   }
   // the next launch's (or the caller's) state
   double* g = (st.cur ? a.xb1 : a.xb0) + sy.eoff;
