@@ -474,7 +474,7 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
     int k = opt->rounds_per_launch;
     if (k <= 0) {
       const double work = static_cast<double>(S) * sum_n2;
-      k = work > 1.0e10 ? 2 : (work > 1.0e9 ? 4 : (work > 1.0e8 ? 8 : 32));
+      k = work > 1.0e10 ? 2 : (work > 1.0e9 ? 4 : 8);  // (a recapture costs by its launches)
     }
     return k;
   };

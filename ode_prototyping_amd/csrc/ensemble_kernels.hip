@@ -782,6 +782,8 @@ __global__ __launch_bounds__(kBlock) void k_ens_final(EnsBufs b) {
   } else {
     ctrl_attempt(&ls, T, sum, 6 * static_cast<size_t>(sy.n), nullptr, trace);
   }
+  if (b.n_dense > 0 && threadIdx.x == 0)
+    dense_gate(&ls, b.dense_t, b.n_dense, b.tableau == ODEHIP_TABLEAU_DOPRI5 ? 0 : 4);
   wave_lds_fence();
   state_words(st, &ls);
   if (threadIdx.x == 0 && ls.done) atomicSub(b.n_active, 1);
@@ -794,12 +796,6 @@ __global__ __launch_bounds__(kBlock) void k_ens_final(EnsBufs b) {
 // stages, evaluated for those systems only; then the rows, one workgroup per
 // reduction group.  A system that finished in this round still writes its
 // last step's rows.
-__global__ void k_ens_dense_begin(EnsBufs b, int extra_rhs) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= b.n_sys) return;
-  dense_gate(b.st + s, b.dense_t, b.n_dense, extra_rhs);
-}
-
 __global__ __launch_bounds__(kBlock) void k_ens_dense_stage8(EnsBufs b, int x) {
   const GroupPos p = group_pos(b);
   const SolverState* st = b.st + p.sys;
@@ -1055,10 +1051,8 @@ hipError_t ens_enqueue_round(const EnsBufs& b, hipStream_t s) {
   else
     hipLaunchKernelGGL(k_ens_final<false>, dim3(groups_grid(b)), dim3(kBlock), 0, s, b);
   if (b.n_dense > 0 && b.tableau == ODEHIP_TABLEAU_DOPRI5) {
-    hipLaunchKernelGGL(k_ens_dense_begin, dim3(sys_grid(b)), dim3(64), 0, s, b, 0);
     hipLaunchKernelGGL(k_ens_dense_out5, dim3(groups_grid(b)), dim3(kBlock), 0, s, b);
   } else if (b.n_dense > 0) {
-    hipLaunchKernelGGL(k_ens_dense_begin, dim3(sys_grid(b)), dim3(64), 0, s, b, 4);
     if ((e = ens_launch_rhs(b, nullptr, b.kfsal, 2, s)) != hipSuccess) return e;
     for (int x = 0; x < 3; ++x) {
       hipLaunchKernelGGL(k_ens_dense_stage8, dim3(groups_grid(b)), dim3(kBlock), 0, s, b, x);

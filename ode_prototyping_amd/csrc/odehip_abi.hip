@@ -686,13 +686,16 @@ int odehip_rk_solve(odehip_context* ctx, int tableau, const odehip_ode* ode,
   const int S = host_tableau(tableau).S;
   const size_t n = ode->n_var;
 
-  // attempts per replay: aim for several ms of work per replay
+  // attempts per replay: enough that a replay (0.3 ms and more) covers its own
+  // launch and the copy of the done flag, and no more, since the solve's last
+  // replay and the one behind it run empty attempts (1000 bodies, 289 attempts: 63
+  // empty ones with 32 a replay)
   int K = opt->attempts_per_launch;
   if (K == 0) {
-    const double work = ode->rhs_kind == ODEHIP_RHS_NBODY
-                            ? static_cast<double>(S) * (n / 6.0) * (n / 6.0)
-                            : static_cast<double>(S) * n;
-    K = work > 4.0e9 ? 2 : (work > 1.0e8 ? 8 : 32);
+    const bool nbody = ode->rhs_kind == ODEHIP_RHS_NBODY;
+    const double work = nbody ? static_cast<double>(S) * (n / 6.0) * (n / 6.0)
+                              : static_cast<double>(S) * n;
+    K = work > 1.0e8 ? 2 : (nbody ? 8 : 32);
   }
 
   hipStream_t s = begin_work(ctx);

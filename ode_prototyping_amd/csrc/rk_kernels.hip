@@ -92,12 +92,14 @@ __global__ void k_target(double* sc, const double* atol, const double* rtol,
 // scaled squared error folded into this group's partial -- one coalesced pass
 // over ks (RKEmbeddedParallel.hpp:47-55, 103-137) --, then, in the last group
 // to get there, accept/reject and step-size control (:57-79) with the
-// termination tests and counters.  kLearned: with the network.
+// termination tests and counters, and the gate of the dense-output pass.
+// kLearned: with the network.
 template <bool kLearned>
 __global__ __launch_bounds__(kBlock) void k_final_dev(
     SolverState* st, int tab, const double* ks, double* xb0, double* xb1,
     const double* atol, const double* rtol, double* partials, double* kfsal,
-    size_t n_var, double* times, double* trace, const MlpInfer* M, int n_particles) {
+    size_t n_var, double* times, double* trace, const MlpInfer* M, int n_particles,
+    const double* dense_t, long n_dense, int dense_rhs) {
   if (st->done) return;
   const Tableau& T = c_tab[tab];
   const int cur = st->cur;
@@ -127,6 +129,7 @@ __global__ __launch_bounds__(kBlock) void k_final_dev(
   } else {
     ctrl_attempt(&ls, T, sum, n_var, times, trace);
   }
+  if (n_dense > 0 && threadIdx.x == 0) dense_gate(&ls, dense_t, n_dense, dense_rhs);
   wave_lds_fence();
   state_words(st, &ls);
 }
@@ -235,13 +238,6 @@ __global__ void k_save_state(const SolverState* st, const double* xb0,
 // controller has already swapped the ping-pong buffers: the step went from
 // the buffer st->cur does not name to the one it names, over st->dt_acc,
 // ending at st->t.
-
-// The gate of the dense pass (one thread).
-__global__ void k_dense_begin(SolverState* st, const double* times, long n_dense,
-                              int extra_rhs) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  dense_gate(st, times, n_dense, extra_rhs);
-}
 
 // The input of extra stage 13 + x (StepperDopr853.hpp:239-262).
 __global__ void k_dense_stage(const SolverState* st, int x, double* ytmp,
@@ -478,16 +474,15 @@ hipError_t enqueue_attempt(const SolveBufs& b, hipStream_t s) {
                                                                : k_final_dev<false>;
   hipLaunchKernelGGL(final_pass, dim3(blocks_for(n)), dim3(kBlock), 0, s, b.st, b.tableau,
                      b.ks, b.xb0, b.xb1, b.atol, b.rtol, b.partA,
-                     b.kfsal, n, b.times, b.trace, b.mlp, b.n_particles);
+                     b.kfsal, n, b.times, b.trace, b.mlp, b.n_particles, b.dense_t,
+                     b.n_dense, b.tableau == ODEHIP_TABLEAU_DOPRI5 ? 0 : 4);
   if (b.states && b.states_cap > 0)
     hipLaunchKernelGGL(k_save_state, dim3(blocks_for(n)), dim3(kBlock), 0, s, b.st, b.xb0,
                        b.xb1, b.states, b.states_cap, n);
   if (b.n_dense > 0 && b.tableau == ODEHIP_TABLEAU_DOPRI5) {
-    hipLaunchKernelGGL(k_dense_begin, dim3(1), dim3(64), 0, s, b.st, b.dense_t, b.n_dense, 0);
     hipLaunchKernelGGL(k_dense_out5, dim3(blocks_for(n)), dim3(kBlock), 0, s, b.st, b.ks,
                        b.xb0, b.xb1, b.dense_t, b.dense_out, n);
   } else if (b.n_dense > 0) {
-    hipLaunchKernelGGL(k_dense_begin, dim3(1), dim3(64), 0, s, b.st, b.dense_t, b.n_dense, 4);
     if ((e = enqueue_rhs(b, nullptr, b.kfsal, 2, s)) != hipSuccess) return e;
     for (int x = 0; x < 3; ++x) {
       double* temp = (x & 1) ? b.ytmp1 : b.ytmp0;
