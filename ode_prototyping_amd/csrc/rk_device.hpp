@@ -83,7 +83,7 @@ __device__ inline double stage_value(const Tableau& T, int stage, double dt,
 // All of them for kernels whose launch is a chain of latencies; few for those
 // that fill the chip, whose occupancy the loads' registers would take.
 constexpr int kStageLoads = kMaxStages - 1;
-constexpr int kStageLoadsLean = 6;
+constexpr int kStageLoadsLean = 2;
 template <int L>
 __device__ inline void next_stage(const NextStage& N, const Tableau& T, size_t n_var, size_t e,
                                   double k, double x0, double dt) {
