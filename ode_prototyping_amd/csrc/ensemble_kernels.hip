@@ -752,7 +752,10 @@ template <bool kLearned>
 __global__ __launch_bounds__(kBlock) void k_ens_final(EnsBufs b) {
   const GroupPos p = group_pos(b);
   SolverState* st = b.st + p.sys;
-  if (st->done) return;  // uniform over the workgroup
+  if (st->done) {  // uniform over the workgroup
+    if (b.n_dense > 0 && p.g == b.sys[p.sys].gbase && threadIdx.x == 0) dense_over(st);
+    return;
+  }
   const Tableau& T = e_tab[b.tableau];
   const int cur = st->cur;
   const double* x0 = cur ? b.xb1 : b.xb0;

@@ -379,6 +379,11 @@ __device__ inline void dense_gate(SolverState* st, const double* times, long n_d
   st->dense_go = go;
 }
 
+// By one thread of the final pass of an attempt enqueued behind a solve's last one,
+// whose own dense pass has run: the passes from here on find the gate shut (left
+// open, each of them would evaluate and write the last step's rows again).
+__device__ inline void dense_over(SolverState* st) { st->dense_go = 0; }
+
 // DOP853's stage vector j of a dense pass: 0..11 the accepted attempt's
 // stages (nv apart in ks), 12 = f at the step's end (k13), 13..15 the extra
 // stages, kept in the slots of stages 1..3, which the extension never reads.

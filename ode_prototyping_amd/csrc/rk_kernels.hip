@@ -100,7 +100,10 @@ __global__ __launch_bounds__(kBlock) void k_final_dev(
     const double* atol, const double* rtol, double* partials, double* kfsal,
     size_t n_var, double* times, double* trace, const MlpInfer* M, int n_particles,
     const double* dense_t, long n_dense, int dense_rhs) {
-  if (st->done) return;
+  if (st->done) {
+    if (n_dense > 0 && blockIdx.x == 0 && threadIdx.x == 0) dense_over(st);
+    return;
+  }
   const Tableau& T = c_tab[tab];
   const int cur = st->cur;
   const double* x0 = cur ? xb1 : xb0;
