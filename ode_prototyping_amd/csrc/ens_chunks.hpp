@@ -17,16 +17,16 @@ namespace odehip {
 constexpr int kEnsGroup = 32;
 static_assert(kEnsChunk % kEnsGroup == 0, "chunks are whole groups");
 
-// U partners of one lane, coordinates c and masses m already loaded: the terms of
-// fast_term (nbody_terms.hpp) step by step for all of them, so that a wave that
-// has its SIMD to itself does not wait out each partner's chain of a dozen
-// instructions (one partner after the other took 200 cycles each), then their sums
-// in increasing j.
-template <bool kMass, bool kGuard, int U>
-__device__ __forceinline__ void fast_terms(const double (&c)[3 * U], const double (&m)[U], int j,
-                                           int i, double xi, double yi, double zi, double eps2,
-                                           double& ax, double& ay, double& az) {
-  double dx[U], dy[U], dz[U], r2[U], y0[U], y2[U], e[U], w[U];
+// U partners of one lane, coordinates c and masses m already loaded: displacements
+// and m r^-3 of fast_term (nbody_terms.hpp) step by step for all of them, so that a
+// wave that has its SIMD to itself does not wait out each partner's chain of a dozen
+// instructions (one partner after the other took 200 cycles each).
+template <bool kMass, int U>
+__device__ __forceinline__ void fast_weights(const double (&c)[3 * U], const double (&m)[U],
+                                             double xi, double yi, double zi, double eps2,
+                                             double (&dx)[U], double (&dy)[U], double (&dz)[U],
+                                             double (&w)[U]) {
+  double r2[U], y0[U], y2[U], e[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     dx[u] = c[3 * u] - xi;
@@ -51,9 +51,19 @@ __device__ __forceinline__ void fast_terms(const double (&c)[3 * U], const doubl
 #pragma unroll
   for (int u = 0; u < U; ++u) e[u] = e[u] * __builtin_fma(e[u], 1.25, 1.0);
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    w[u] = __builtin_fma(y0[u] * e[u], 1.5, y0[u]);
-    if (kGuard) w[u] = j + u == i ? 0.0 : w[u];
+  for (int u = 0; u < U; ++u) w[u] = __builtin_fma(y0[u] * e[u], 1.5, y0[u]);
+}
+
+// Their terms summed in increasing j.
+template <bool kMass, bool kGuard, int U>
+__device__ __forceinline__ void fast_terms(const double (&c)[3 * U], const double (&m)[U], int j,
+                                           int i, double xi, double yi, double zi, double eps2,
+                                           double& ax, double& ay, double& az) {
+  double dx[U], dy[U], dz[U], w[U];
+  fast_weights<kMass, U>(c, m, xi, yi, zi, eps2, dx, dy, dz, w);
+  if (kGuard) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) w[u] = j + u == i ? 0.0 : w[u];
   }
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll

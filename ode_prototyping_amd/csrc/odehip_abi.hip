@@ -709,8 +709,8 @@ int odehip_rk_solve(odehip_context* ctx, int tableau, const odehip_ode* ode,
   // Small systems: whole attempts by one workgroup (solo.hpp), unless the
   // caller says how the attempts are launched or every state is kept.
   const bool solo = ode->rhs_kind == ODEHIP_RHS_NBODY && opt->attempts_per_launch == 0 &&
-                    ode->nbody_variant != ODEHIP_NBODY_MIXED && n_dense == 0 &&
-                    states_cap == 0 && b.n_particles <= solo_limit(S, ode->nbody_variant, b.mlp != nullptr);
+                    n_dense == 0 && states_cap == 0 &&
+                    b.n_particles <= solo_one_limit(S, ode->nbody_variant, b.mlp != nullptr);
   SoloArgs sa{};
   if (solo) {
     sa.one = EnsSys{0, b.n_particles, 0, n_groups_for(n), 0};

@@ -14,6 +14,11 @@ constexpr int kSoloTerms = 4;     // exact: partners per wave and block
 constexpr int kSoloMaxN = 320;    // fast, mixed: 192 threads per 64 targets
 constexpr int kSoloExactN = 128;  // sizes up to which it is the faster form
 constexpr int kSoloSumN = 256;
+// fast, a solve of its own: two tiles of targets by 16 waves (DOPRI5 / DOP853,
+// launched attempts against one workgroup: 64 bodies 22.3 / 25.2 against 8.6 /
+// 10.3 ms, 128 bodies 10.2 / 11.9 against 8.6 / 11.4; with three tiles on, 180 bodies,
+// 7.2 / 9.1 against 17.4 / 25.4)
+constexpr int kSoloOneFastN = 128;
 constexpr uint64_t kSoloTicks = 200000;  // of the 100 MHz clock: 2 ms a launch
 constexpr int kSoloMaxQuads = 4 * ((6 * kSoloMaxN + ODEHIP_REDUCE_GROUP - 1) / ODEHIP_REDUCE_GROUP);
 // LDS of a CU less the kernel's static use and some to spare.
@@ -76,6 +81,16 @@ inline int solo_limit(int S, int variant, bool learned) {
   for (int n = want; n > 0; --n)
     if (solo_waves(n, S, variant, learned) > 0) return n;
   return 0;
+}
+
+// The same for a solve of its own (odehip_rk_solve).
+inline int solo_one_limit(int S, int variant, bool learned) {
+  const int all = solo_limit(S, variant, learned);
+  switch (variant) {
+    case ODEHIP_NBODY_EXACT: return all;
+    case ODEHIP_NBODY_FAST: return std::min(all, kSoloOneFastN);
+    default: return 0;  // mixed: the launched kernels' sums have another order
+  }
 }
 
 // One launch: `blocks` systems of at most n_max bodies.

@@ -10,9 +10,12 @@
 // is that chain: barriers, LDS reads and the dependent arithmetic of one
 // wave's partners, not throughput (a CU holds one or two such workgroups).
 //
-// Every number is computed by the functions and in the order of the lockstep
-// kernels (rk_kernels.hip, ensemble_kernels.hip), so which of them runs a solve
-// changes no result.  A workgroup starts no attempt once kSoloTicks have passed
+// Every number is computed by the functions and in the order of the kernels that
+// run the same solve by launches -- for a solve of its own those of rk_kernels.hip and
+// nbody_kernels.hip, for an ensemble's system the lockstep ones of
+// ensemble_kernels.hip, whose fast sums have another order --, so which form runs a
+// solve changes no bit of its result (tests/test_gpu_solve_forms.py,
+// tests/test_gpu_solo.py).  A workgroup starts no attempt once kSoloTicks have passed
 // and keeps what the next launch needs in the state's global buffers: launches
 // of bounded time, whose systems need not wait for one another's attempts.
 #include <type_traits>
@@ -162,6 +165,110 @@ __device__ __forceinline__ void solo_groups(lds_cptr in, lds_cptr mass, lds_ptr 
   if (ft < tiles && i < n) kout[3 * n + 3 * i + fc / 64] = acc * scale;
 }
 
+// fast, one system: the order of k_nbody_fast_rows (nbody_kernels.hip), which
+// evaluates such systems wherever attempts are launched (dense output, kept states,
+// attempts_per_launch), so that a solve's bits do not depend on these.  Up to four
+// sets of 64 partners each has a wave of its own there, a lane per partner, which
+// folds lanes l with l + 32, then + 16, 8, 4, 2 and 1: the sum of the lanes
+// l = c mod B is, level by level, the same whoever computes it.  Lanes past the last
+// partner add +0 there, which changes at most the sign of a zero, and the fold over
+// the sets starts at +0; so they are left out here where that is a whole level.
+static_assert(kSoloOneFastN <= 2 * 64, "a share of 8 or 16 lanes per wave");
+
+// Lanes c, c + 8, ... of a set, the first kLive of them, j the first one's partner.
+// (Unclamped loads in sets that are whole spill, and take 10 % longer.)
+template <bool kMass, bool kGuard, int kLive>
+__device__ __forceinline__ void row_lanes(lds_cptr in, lds_cptr mass, int j, int n, int i,
+                                          double xi, double yi, double zi, double eps2,
+                                          double (&s)[3]) {
+  double c[3 * kLive], m[kLive], dx[kLive], dy[kLive], dz[kLive], w[kLive];
+#pragma unroll
+  for (int u = 0; u < kLive; ++u) {
+    const int q = min(j + 8 * u, n - 1);
+    c[3 * u] = in[3 * q];
+    c[3 * u + 1] = in[3 * q + 1];
+    c[3 * u + 2] = in[3 * q + 2];
+    m[u] = kMass ? mass[q] : 1.0;
+  }
+  fast_weights<kMass, kLive>(c, m, xi, yi, zi, eps2, dx, dy, dz, w);
+#pragma unroll
+  for (int u = 0; u < kLive; ++u) {
+    const bool out = (j + 8 * u >= n) | (kGuard & (j + 8 * u == i));
+    w[u] = out ? 0.0 : w[u];
+    dx[u] = __builtin_fma(dx[u], w[u], 0.0);  // (a lane's sum starts at +0)
+    dy[u] = __builtin_fma(dy[u], w[u], 0.0);
+    dz[u] = __builtin_fma(dz[u], w[u], 0.0);
+  }
+#pragma unroll
+  for (int h = kLive / 2; h >= 1; h /= 2) {
+#pragma unroll
+    for (int u = 0; u < h; ++u) {
+      dx[u] += dx[u + h];
+      dy[u] += dy[u + h];
+      dz[u] += dz[u + h];
+    }
+  }
+  s[0] = dx[0];
+  s[1] = dy[0];
+  s[2] = dz[0];
+}
+
+// kTiles tiles of 64 targets and sets of 64 partners (n / 64, rounded up), one wave for
+// the lanes l = c mod P of a set and a tile: eight waves and P = 8 at up to 64
+// bodies, sixteen and P = 4 at up to 128.  Thread (tile, coordinate, target) folds the
+// shares of a set, then adds the sets.
+template <bool kMass, bool kGuard, int kTiles>
+__device__ __forceinline__ void solo_rows(lds_cptr in, lds_cptr mass, lds_ptr kout, lds_ptr part,
+                                          int n, double eps2, int wave, int lane) {
+  static_assert(kTiles == 1 || kTiles == 2, "shares of 8 or 16 lanes");
+  constexpr int P = kTiles == 1 ? 8 : 4;
+  {
+    const int i = min(64 * (wave / P % kTiles) + lane, n - 1);
+    const int j = 64 * (wave / P / kTiles) + wave % P;
+    const double xi = in[3 * i], yi = in[3 * i + 1], zi = in[3 * i + 2];
+    double s[3], t[3];
+    if constexpr (kTiles == 1) {
+      if (n > 32)
+        row_lanes<kMass, kGuard, 8>(in, mass, j, n, i, xi, yi, zi, eps2, s);
+      else if (n > 16)
+        row_lanes<kMass, kGuard, 4>(in, mass, j, n, i, xi, yi, zi, eps2, s);
+      else
+        row_lanes<kMass, kGuard, 2>(in, mass, j, n, i, xi, yi, zi, eps2, s);
+    } else {
+#pragma unroll 1  // (the loads of both halves together would spill)
+      for (int h = 0; h < 2; ++h) {
+        row_lanes<kMass, kGuard, 8>(in, mass, j + 4 * h, n, i, xi, yi, zi, eps2, s);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          if (h == 0)
+            t[k] = s[k];
+          else
+            s[k] += t[k];
+        }
+      }
+    }
+    lds_ptr o = part + wave * 192 + lane;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) o[64 * k] = s[k];
+  }
+  __syncthreads();
+  const int ft = threadIdx.x / 192, fc = threadIdx.x % 192, i = 64 * ft + fc % 64;
+  if (ft >= kTiles || i >= n) return;
+  double acc = 0.0;
+#pragma unroll
+  for (int set = 0; set < kTiles; ++set) {
+    double v[P];
+#pragma unroll
+    for (int c = 0; c < P; ++c) v[c] = part[(P * (kTiles * set + ft) + c) * 192 + fc];
+#pragma unroll
+    for (int h = P / 2; h >= 1; h /= 2)
+#pragma unroll
+      for (int c = 0; c < h; ++c) v[c] += v[c + h];
+    acc += v[0];
+  }
+  kout[3 * n + 3 * i + fc / 64] = acc;
+}
+
 // Sum over the workgroup's elements of 64-element quads and groups in the
 // canonical order (rk_device.hpp): quad[] holds the quads' sums.
 __device__ __forceinline__ double solo_fold(lds_cptr quad, int n_groups) {
@@ -171,7 +278,9 @@ __device__ __forceinline__ double solo_fold(lds_cptr quad, int n_groups) {
   return r;
 }
 
-template <int kVariant, bool kMass, bool kSpecial, bool kNear>
+// kRows: fast, one system (solo_rows); an ensemble's systems have the lockstep
+// kernels' order (solo_groups).
+template <int kVariant, bool kMass, bool kSpecial, bool kNear, bool kRows>
 __global__ __launch_bounds__(64 * kSoloWaves) void k_solo(SoloArgs a) {
   __shared__ SolverState st;
   __shared__ double quad_[kSoloMaxQuads];
@@ -208,14 +317,7 @@ __global__ __launch_bounds__(64 * kSoloWaves) void k_solo(SoloArgs a) {
   if (kMass) {
     const double* m = a.mass + sy.eoff / 6;
     for (int e = tid; e < n; e += threads) mass[e] = m[e];
-    if (kVariant != ODEHIP_NBODY_EXACT) {
-      if (a.sys)
-        m_uni = st.mass_uniform;
-      else
-        m_uni = __syncthreads_and(lane_masses_uniform<kScanLoadsLean>(m, n, tid, threads)) != 0
-                    ? m[0]
-                    : 0.0;
-    }
+    if (kVariant != ODEHIP_NBODY_EXACT && !kRows) m_uni = st.mass_uniform;
   }
   const bool per_term = kMass && m_uni == 0.0;
   const double scale = per_term || !kMass ? 1.0 : m_uni;
@@ -275,6 +377,11 @@ __global__ __launch_bounds__(64 * kSoloWaves) void k_solo(SoloArgs a) {
           solo_exact<kMass, true>(in, mass, kout, work, n, a.eps2, wave, waves, lane);
         else
           solo_exact<kMass, false>(in, mass, kout, work, n, a.eps2, wave, waves, lane);
+      } else if constexpr (kRows) {
+        if (n <= 64)
+          solo_rows<kMass, kSpecial, 1>(in, mass, kout, work, n, a.eps2, wave, lane);
+        else
+          solo_rows<kMass, kSpecial, 2>(in, mass, kout, work, n, a.eps2, wave, lane);
       } else {
         if (kMass && per_term)
           solo_groups<kVariant, true, kSpecial, kNear>(in, mass, kout, work, n, a.eps2, near2,
@@ -341,12 +448,12 @@ __global__ __launch_bounds__(64 * kSoloWaves) void k_solo(SoloArgs a) {
   if (tid == 0 && st.done && a.n_active) atomicSub(a.n_active, 1);
 }
 
-template <int kVariant, bool kNear>
+template <int kVariant, bool kNear, bool kRows = false>
 void* solo_kernel(bool mass, bool special) {
-  return mass ? (special ? (void*)k_solo<kVariant, true, true, kNear>
-                         : (void*)k_solo<kVariant, true, false, kNear>)
-              : (special ? (void*)k_solo<kVariant, false, true, kNear>
-                         : (void*)k_solo<kVariant, false, false, kNear>);
+  return mass ? (special ? (void*)k_solo<kVariant, true, true, kNear, kRows>
+                         : (void*)k_solo<kVariant, true, false, kNear, kRows>)
+              : (special ? (void*)k_solo<kVariant, false, true, kNear, kRows>
+                         : (void*)k_solo<kVariant, false, false, kNear, kRows>);
 }
 
 }  // namespace
@@ -355,13 +462,18 @@ hipError_t launch_solo(const SoloArgs& args, int n_max, int variant, unsigned bl
                        hipStream_t s) {
   SoloArgs a = args;
   const int S = host_tableau(a.tableau).S;
-  const int waves = solo_waves(n_max, S, variant, a.mlp);
-  if (waves == 0) return hipErrorInvalidValue;
+  const bool rows = variant == ODEHIP_NBODY_FAST && !a.sys;
+  int waves = solo_waves(n_max, S, variant, a.mlp);
+  if (rows) waves = n_max > kSoloOneFastN ? 0 : n_max > 64 ? kSoloWaves : 8;
+  if (waves == 0 || (variant == ODEHIP_NBODY_MIXED && !a.sys)) return hipErrorInvalidValue;
   if (blocks == 0) return hipSuccess;
   a.lds_doubles = solo_lds_doubles(n_max, S, variant, waves, a.mlp);
+  if (a.lds_doubles > kSoloLdsDoubles) return hipErrorInvalidValue;
   void* k = nullptr;
   if (variant == ODEHIP_NBODY_EXACT)
     k = solo_kernel<ODEHIP_NBODY_EXACT, false>(a.mass, a.eps2 >= 0x1p-200 && a.eps2 <= 0x1p100);
+  else if (rows)
+    k = solo_kernel<ODEHIP_NBODY_FAST, false, true>(a.mass, !(a.eps2 >= 1e-150));
   else if (variant == ODEHIP_NBODY_FAST)
     k = solo_kernel<ODEHIP_NBODY_FAST, false>(a.mass, !(a.eps2 >= 1e-150));
   else if (a.near_c > 0.0)
