@@ -168,6 +168,15 @@ void set_tile_cfg(EnsBufs* b, int cfg, int n_tiles) {
   b->n_tiles = n_tiles;
 }
 
+// Waits for a stream when a call that put work on it returns early, so that the next
+// call may set up the same buffers.
+struct DrainOnReturn {
+  hipStream_t stream = nullptr;  // null: nothing to wait for
+  ~DrainOnReturn() {
+    if (stream) (void)hipStreamSynchronize(stream);
+  }
+};
+
 bool tune_cache_hit(const EnsembleWorkspace* w, const Layout& L, int variant,
                     bool mass, double eps2, double near_c) {
   return w->tuned_cfg >= 0 && w->tuned_variant == variant && w->tuned_mass == mass &&
@@ -410,6 +419,7 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
   SoloArgs sa{};
   long solo_pushed = 0, solo_seen = 0;
   bool solo_done = solo.empty();
+  DrainOnReturn drain;
   auto push_solo = [&]() -> int {
     const int at = static_cast<int>(solo_pushed & 1);
     HIP_TRY(ctx, launch_solo(sa, solo_max, nbody_variant, static_cast<unsigned>(solo.size()),
@@ -461,6 +471,7 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
     sa.tableau = tableau;
     HIP_TRY(ctx, hipEventRecord(w->ev_fork, s));
     HIP_TRY(ctx, hipStreamWaitEvent(w->side, w->ev_fork, 0));
+    drain.stream = w->side;
     if ((rc = poll_solo(false))) return rc;
   }
 
@@ -582,6 +593,7 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
     if ((rc = poll_solo(true))) return rc;
     HIP_TRY(ctx, hipEventRecord(w->ev_join, w->side));
     HIP_TRY(ctx, hipStreamWaitEvent(s, w->ev_join, 0));
+    drain.stream = nullptr;  // `s` goes on behind it
   }
   HIP_TRY(ctx, ens_enqueue_copy_out(b, x_out, s));
   std::vector<SolverState> hs(L.sys.size());
