@@ -84,16 +84,24 @@ int make_layout(odehip_context* ctx, int n_systems, const int* n_particles,
 
 int workspace(odehip_context* ctx, size_t bytes, EnsembleWorkspace** out) {
   if (!ctx->ens) {
-    auto* w = new (std::nothrow) EnsembleWorkspace();
-    if (!w) return fail(ctx, ODEHIP_ERR_NOMEM, "ensemble workspace");
-    ctx->ens = w;
-    HIP_TRY(ctx, hipHostMalloc(reinterpret_cast<void**>(&w->h_active), 4 * sizeof(int)));
-    HIP_TRY(ctx, hipStreamCreateWithFlags(&w->side, hipStreamNonBlocking));
-    for (hipEvent_t* e : {&w->ev[0], &w->ev[1], &w->ev_side[0], &w->ev_side[1], &w->ev_fork,
-                          &w->ev_join})
-      HIP_TRY(ctx, hipEventCreateWithFlags(e, hipEventDisableTiming));
-    HIP_TRY(ctx, hipEventCreate(&w->t0));
-    HIP_TRY(ctx, hipEventCreate(&w->t1));
+    auto* made = new (std::nothrow) EnsembleWorkspace();
+    if (!made) return fail(ctx, ODEHIP_ERR_NOMEM, "ensemble workspace");
+    // the context holds it once all of it is there
+    const int rc = [&]() -> int {
+      HIP_TRY(ctx, hipHostMalloc(reinterpret_cast<void**>(&made->h_active), 4 * sizeof(int)));
+      HIP_TRY(ctx, hipStreamCreateWithFlags(&made->side, hipStreamNonBlocking));
+      for (hipEvent_t* e : {&made->ev[0], &made->ev[1], &made->ev_side[0], &made->ev_side[1],
+                            &made->ev_fork, &made->ev_join})
+        HIP_TRY(ctx, hipEventCreateWithFlags(e, hipEventDisableTiming));
+      HIP_TRY(ctx, hipEventCreate(&made->t0));
+      HIP_TRY(ctx, hipEventCreate(&made->t1));
+      return ODEHIP_OK;
+    }();
+    if (rc != ODEHIP_OK) {
+      destroy_ensemble_workspace(made);
+      return rc;
+    }
+    ctx->ens = made;
   }
   EnsembleWorkspace* w = ctx->ens;
   if (w->cap < bytes) {

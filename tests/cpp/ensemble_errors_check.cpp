@@ -211,7 +211,13 @@ int main() {
           ++bad;
         }
       }
+      // (after the arena's allocation has failed, too, the next call finds what it needs)
       fail_at = -1;
+      calls = 0;
+      if (hit && solve() != ODEHIP_OK) {
+        std::printf("call %ld (%s) failed: so does the next solve\n", k, failed);
+        ++bad;
+      }
       odehip_destroy(ctx);
       std::free(x);
       if (!hit) break;
