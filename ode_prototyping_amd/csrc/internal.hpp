@@ -90,6 +90,9 @@ __host__ __device__ inline float mixed_near2(double coefficient, int n) {
 }
 
 // ---- launchers (nbody_kernels.hip) ----
+// Whether a launch should form the next stage's input itself (NBodyArgs::next): if
+// not, a launch behind it does.
+bool nbody_rhs_forms_next(int n, int variant, float near2, bool masses);
 hipError_t launch_nbody_rhs(const NBodyArgs& a, int variant, hipStream_t s);
 hipError_t launch_probe_fp64(double* out, long long* clk, int blocks, int iters,
                              hipStream_t s);

@@ -4,8 +4,9 @@
 // (NBodyODE::acc, NBodyODE.hpp:41-46).  Per step: one RHS launch, which also
 // updates the velocities and moves the positions of its bodies on (three launches
 // a step, position kernel, RHS, velocity kernel, took 1000 bodies 14.5 us a step);
-// where every state is kept, those three.  The two acceleration buffers swap
-// roles instead of the reference's copy acc0 = acc1.  The step times are computed
+// where every state is kept, or the launch should not form the next state
+// (nbody_rhs_forms_next), those three.  The two acceleration buffers swap roles
+// instead of the reference's copy acc0 = acc1.  The step times are computed
 // on the host with the reference's own t += dt loop (no clip of the last
 // step), so the number of steps and every saved time match it exactly.
 #include <algorithm>
@@ -91,7 +92,9 @@ extern "C" int odehip_leapfrog(odehip_context* ctx, const odehip_ode* ode,
     return hipSuccess;
   };
   if ((e = save(0)) == hipSuccess) e = rhs(k0);
-  if (!states && n_steps > 0 && e == hipSuccess) {
+  const bool fused = !states && nbody_rhs_forms_next(a.n, ode->nbody_variant, a.near2,
+                                                     a.mass != nullptr);
+  if (fused && n_steps > 0 && e == hipSuccess) {
     // one launch per step: the step's right-hand side leaves the state with which
     // the next one starts
     double* cur = x;
@@ -110,7 +113,7 @@ extern "C" int odehip_leapfrog(odehip_context* ctx, const odehip_ode* ode,
     if (e == hipSuccess && cur != x)
       e = hipMemcpyAsync(x, cur, n_var * sizeof(double), hipMemcpyDeviceToDevice, s);
   }
-  for (long step = 0; states && step < n_steps && e == hipSuccess; ++step) {
+  for (long step = 0; !fused && step < n_steps && e == hipSuccess; ++step) {
     hipLaunchKernelGGL(k_lf_position, dim3(blocks), dim3(kBlock), 0, s, x, k0 + n_dof, dt,
                        n_dof);
     if ((e = rhs(k1)) != hipSuccess) break;

@@ -69,6 +69,16 @@ __global__ void k_stage_host_dt(int tab, int stage, double dt, double* temp,
   if (i < n_var) temp[i] = stage_value(c_tab[tab], stage, dt, ks, x0, i, n_var);
 }
 
+// The input of a stage whose predecessor's launch has not formed it.
+__global__ void k_stage_dev(const SolverState* st, int tab, int stage, double* y,
+                            const double* ks, const double* xb0, const double* xb1,
+                            size_t n_var) {
+  if (st->done) return;
+  const size_t i = gid();
+  const double* x0 = st->cur ? xb1 : xb0;
+  if (i < n_var) y[i] = stage_value(c_tab[tab], stage, st->dt, ks, x0, i, n_var);
+}
+
 __global__ void k_update_host_dt(int tab, double dt, double* x, double* err,
                                  const double* ks, const double* x0,
                                  size_t n_var) {
@@ -465,12 +475,18 @@ hipError_t enqueue_attempt(const SolveBufs& b, hipStream_t s) {
   const size_t n = b.n_var;
   hipError_t e = hipSuccess;
   const double* in = nullptr;  // the current state
+  const bool fused = b.rhs_kind != ODEHIP_RHS_NBODY ||
+                     nbody_rhs_forms_next(b.n_particles, b.nbody_variant, b.near2,
+                                          b.mass != nullptr);
   for (int stage = 0; stage < T.S; ++stage) {
     // two buffers in turn: a stage's input is read while the next one is written
     double* y = stage + 1 < T.S ? ((stage & 1) ? b.ytmp0 : b.ytmp1) : nullptr;
     e = enqueue_rhs(b, in, b.ks + stage * n, stage == 0 ? 1 : 0, s,
-                    NextStage{y, b.ks, stage, b.tableau});
+                    fused ? NextStage{y, b.ks, stage, b.tableau} : NextStage{});
     if (e != hipSuccess) return e;
+    if (!fused && y)
+      hipLaunchKernelGGL(k_stage_dev, dim3(blocks_for(n)), dim3(kBlock), 0, s, b.st, b.tableau,
+                         stage + 1, y, b.ks, b.xb0, b.xb1, n);
     in = y;
   }
   auto* final_pass = b.controller == ODEHIP_CONTROLLER_LEARNED ? k_final_dev<true>
