@@ -12,8 +12,13 @@ namespace odehip {
 constexpr int kSoloWaves = 16;    // at most, per workgroup
 constexpr int kSoloTerms = 4;     // exact: partners per wave and block
 constexpr int kSoloMaxN = 320;    // fast, mixed: 192 threads per 64 targets
-constexpr int kSoloExactN = 128;  // sizes up to which it is the faster form
+constexpr int kSoloExactN = 128;  // an ensemble's systems: sizes up to which it takes them
 constexpr int kSoloSumN = 256;
+// exact, a solve of its own: one tile of targets (DOPRI5 / DOP853, launched attempts
+// against one workgroup: 64 bodies 21.6 / 24.4 against 12.8 / 16.1 ms; with a second
+// tile, 80 bodies 21.5 / 25.2 against 23.4 / 30.7, 128 bodies 11.7 / 14.2 against 17.3 /
+// 27.9)
+constexpr int kSoloOneExactN = 64;
 // fast, a solve of its own: two tiles of targets by 16 waves (DOPRI5 / DOP853,
 // launched attempts against one workgroup: 64 bodies 22.3 / 25.2 against 8.6 /
 // 10.3 ms, 128 bodies 10.2 / 11.9 against 8.6 / 11.4; with three tiles on, 180 bodies,
@@ -87,7 +92,7 @@ inline int solo_limit(int S, int variant, bool learned) {
 inline int solo_one_limit(int S, int variant, bool learned) {
   const int all = solo_limit(S, variant, learned);
   switch (variant) {
-    case ODEHIP_NBODY_EXACT: return all;
+    case ODEHIP_NBODY_EXACT: return std::min(all, kSoloOneExactN);
     case ODEHIP_NBODY_FAST: return std::min(all, kSoloOneFastN);
     default: return 0;  // mixed: the launched kernels' sums have another order
   }
