@@ -488,7 +488,14 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
   // running systems has fallen to 7/8 of the last list's, so the long tail of
   // a few slow systems does not launch workgroups for all the finished ones
   // (on 2048 systems 3/4 measured 1-1.5 % faster than 1/2, and 7/8 another
-  // 0-1 %; same results).
+  // 0-1 %; same results), but where launches bound a round (kEnsListWork pairs or
+  // less), no sooner than kEnsListRounds rounds after the last time: new lists gain
+  // little there, and their graph costs as much as a dozen rounds.  (64 systems of 64
+  // bodies in rounds, DOPRI5 fast 5.5 -> 4.2 ms; 128 of up to 1024, DOP853 exact 44.9 ->
+  // 33.9; with 1e8 pairs 141 of up to 233, DOP853 exact, take 108 ms instead of 105,
+  // with 1e7 the second example stays at 44.)
+  constexpr long kEnsListRounds = 64;
+  constexpr double kEnsListWork = 3.0e7;
   auto rounds_per_replay = [&](double sum_n2) {
     int k = opt->rounds_per_launch;
     if (k <= 0) {
@@ -524,6 +531,7 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
   };
   EnsBufs rb = b;  // run_cfg: the tile shape of the running systems
   int K = 0, n_live = n_rounds;
+  double work = S * L.work;  // of a round of the present lists
   // Lists and graph for the systems `live` marks (the stream is idle).
   auto set_running = [&]() -> int {
     std::vector<int2> act;
@@ -548,6 +556,7 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
     rb.n_groups = static_cast<int>(act.size());
     set_tile_cfg(&rb, run_cfg, static_cast<int>(tiles.size()));
     K = rounds_per_replay(sum_n2);
+    work = S * sum_n2;
     return capture(rb, K);
   };
   if (n_rounds == n_systems) {
@@ -563,6 +572,8 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
   int slot = 0;
   bool have_prev = false;
   int compact_below = n_rounds * 7 / 8;
+  auto next_lists = [&] { return launched + (work > kEnsListWork ? 0 : kEnsListRounds); };
+  long compact_from = next_lists();
   std::vector<SolverState> hst;
   while (n_rounds > 0) {
     HIP_TRY(ctx, hipGraphLaunch(w->exec, s));
@@ -576,7 +587,7 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
       HIP_TRY(ctx, hipEventSynchronize(w->ev[slot ^ 1]));
       const int running = w->h_active[slot ^ 1];
       if (running == 0) break;
-      if (running <= compact_below) {
+      if (running <= compact_below && launched >= compact_from) {
         HIP_TRY(ctx, hipStreamSynchronize(s));
         hst.resize(L.sys.size());
         HIP_TRY(ctx, hipMemcpy(hst.data(), b.st, hst.size() * sizeof(SolverState),
@@ -589,6 +600,7 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
         if (n_live == 0) break;
         if ((rc = set_running())) return rc;
         compact_below = n_live * 7 / 8;
+        compact_from = next_lists();
         have_prev = false;
         slot = 0;
         continue;
