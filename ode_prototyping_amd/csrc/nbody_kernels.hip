@@ -520,8 +520,7 @@ __device__ __forceinline__ void mixed_partners(uniform_ptr yu, uniform_ptr mass,
 // kNext: a.next is set; without its code in the epilogue the partner loop is
 // scheduled 3 % faster (65536 bodies 1485 -> 1430 us).
 template <bool kMass, bool kGuard, bool kNear, bool kNext>
-__global__ __launch_bounds__(64 * kMixedWaves) ODEHIP_EIGHT_WAVES_SGPRS
-void k_nbody_mixed(NBodyArgs a) {
+__device__ __forceinline__ void mixed_body(const NBodyArgs& a) {
   if (prologue_skip(a)) return;
   __shared__ double red[kMixedWaves][3][64];
   const double* __restrict__ y = select_input(a);
@@ -573,6 +572,20 @@ void k_nbody_mixed(NBodyArgs a) {
     const long e = 3L * i0 + threadIdx.x, lim = 3L * n;
     if (threadIdx.x < 192 && e < lim) a.k[e] = y[lim + e];
   }
+}
+
+// Held to eighty SGPRs, the loop over unequal masses spills (16384 bodies with near
+// field 157 instead of 151 us), and only launches that form the next stage's input
+// in more than one workgroup a CU need the limit: those without masses, the others
+// leave it to a launch of its own there (nbody_rhs_forms_next).
+template <bool kMass, bool kGuard, bool kNear, bool kNext>
+__global__ __launch_bounds__(64 * kMixedWaves) void k_nbody_mixed(NBodyArgs a) {
+  mixed_body<kMass, kGuard, kNear, kNext>(a);
+}
+template <bool kGuard, bool kNear>
+__global__ __launch_bounds__(64 * kMixedWaves) ODEHIP_EIGHT_WAVES_SGPRS
+void k_nbody_mixed_unit_next(NBodyArgs a) {
+  mixed_body<false, kGuard, kNear, true>(a);
 }
 
 // ----------------------------------------------------------------- energy --
@@ -782,29 +795,30 @@ void launch_fast_rows(const NBodyArgs& a, bool guard, hipStream_t s) {
 }  // namespace
 
 namespace {
-template <bool kNext>
-auto* mixed_kernel(bool mass, bool guard, bool near) {
-  return mass ? (guard ? (near ? k_nbody_mixed<true, true, true, kNext>
-                               : k_nbody_mixed<true, true, false, kNext>)
-                       : (near ? k_nbody_mixed<true, false, true, kNext>
-                               : k_nbody_mixed<true, false, false, kNext>))
-              : (guard ? (near ? k_nbody_mixed<false, true, true, kNext>
-                               : k_nbody_mixed<false, true, false, kNext>)
-                       : (near ? k_nbody_mixed<false, false, true, kNext>
-                               : k_nbody_mixed<false, false, false, kNext>));
+template <bool kMass, bool kNext>
+auto* mixed_kernel(bool guard, bool near) {
+  return guard ? (near ? k_nbody_mixed<kMass, true, true, kNext>
+                       : k_nbody_mixed<kMass, true, false, kNext>)
+               : (near ? k_nbody_mixed<kMass, false, true, kNext>
+                       : k_nbody_mixed<kMass, false, false, kNext>);
+}
+auto* mixed_unit_next(bool guard, bool near) {
+  return guard ? (near ? k_nbody_mixed_unit_next<true, true> : k_nbody_mixed_unit_next<true, false>)
+               : (near ? k_nbody_mixed_unit_next<false, true>
+                       : k_nbody_mixed_unit_next<false, false>);
 }
 }  // namespace
 
-// The mixed kernel's partner loop without near field is slower beside that code, by 3 %
-// with equal masses and 6 % with unequal ones; the launch it saves makes up for that
-// in small grids only.  A DOP853 solve of 10 steps, formed here / by a launch behind, with
-// equal masses: 4096 bodies 6.57 / 6.74 ms, 8192 11.12 / 11.12, 16384 21.0 / 20.6, 65536
-// 235 / 229; unequal: 1000 2.83 / 3.10, 4096 6.96 / 6.79, 8192 12.76 / 12.05, 65536
-// 276 / 265.  Whether masses are equal is found on the device, so any that are given
-// count as unequal.
+// With masses, the mixed kernel's partner loop is slower beside that code; the launch
+// it saves makes up for that up to one workgroup a CU with near field and half as
+// many without.  A DOP853 solve of 10 steps, formed here / by a launch behind: unequal
+// masses 2000 bodies 4.16 / 4.47 ms, 8192 12.19 / 12.06, 16384 23.2 / 22.6 (with near
+// field 28.6 / 28.4), 65536 276 / 265 (292 / 289); equal ones 8192 11.13 / 11.14, 16384
+// 21.0 / 20.7 (24.1 / 24.3), 65536 235 / 230 (261 / 261).  Without masses 16384 26.7 /
+// 27.2, 65536 367 / 373.
 bool nbody_rhs_forms_next(int n, int variant, float near2, bool masses) {
-  if (variant != ODEHIP_NBODY_MIXED || near2 > 0.0f) return true;
-  return (n + 63L) / 64 <= device_cus() / (masses ? 4 : 2);
+  if (variant != ODEHIP_NBODY_MIXED || !masses) return true;
+  return (n + 63L) / 64 <= device_cus() / (near2 > 0.0f ? 1 : 2);
 }
 
 hipError_t launch_nbody_rhs(const NBodyArgs& a, int variant, hipStream_t s) {
@@ -841,8 +855,10 @@ hipError_t launch_nbody_rhs(const NBodyArgs& a, int variant, hipStream_t s) {
       const bool guardf = !(static_cast<float>(a.eps2) >= 1e-12f);
       const bool near = a.near2 > 0.0f;
       const dim3 g(blocks), th(64 * kMixedWaves);
-      auto* kern = a.next.y ? mixed_kernel<true>(mass, guardf, near)
-                            : mixed_kernel<false>(mass, guardf, near);
+      auto* kern = a.next.y ? (mass ? mixed_kernel<true, true>(guardf, near)
+                                    : mixed_unit_next(guardf, near))
+                            : (mass ? mixed_kernel<true, false>(guardf, near)
+                                    : mixed_kernel<false, false>(guardf, near));
       hipLaunchKernelGGL(kern, g, th, 0, s, a);
       break;
     }

@@ -19,19 +19,20 @@ def system(n, masses):
     return x, None if masses == "unit" else m
 
 
-# on 256 CUs the change comes at 4096 bodies with masses, at 8192 without
-@pytest.mark.parametrize("n,masses", [(4096, "equal"), (4096, "spread"), (4097, "equal"),
-                                      (4161, "spread"), (8192, "unit"), (8193, "unit"),
-                                      (8257, "equal")])
-@pytest.mark.parametrize("tableau,fsal", [("DOPRI5", True), ("DOP853", False)])
-def test_mixed_attempts(exe, n, masses, tableau, fsal):
+# on 256 CUs the change comes at 8192 bodies with masses
+@pytest.mark.parametrize("n,masses", [(4096, "equal"), (8192, "spread"), (8192, "equal"),
+                                      (8193, "equal"), (8193, "spread"), (8193, "unit"),
+                                      (16500, "spread")])
+@pytest.mark.parametrize("tableau,fsal,near", [("DOPRI5", True, 0.0), ("DOP853", False, 0.0),
+                                               ("DOPRI5", False, 20.0)])
+def test_mixed_attempts(exe, n, masses, tableau, fsal, near):
     import ode_prototyping_amd as oh
     from ode_prototyping_amd.core import _Sub, tableau_shape
     x0, m = system(n, masses)
     ode = oh.NBodyODE(1e-2, m, "mixed")
-    near = exe.near_field
+    keep = exe.near_field
     try:
-        exe.near_field = 0.0
+        exe.near_field = near
         res = oh.integrate(tableau, x0, 0.0, 10.0, 1e-10, 1e-10, ode, exe=exe, fsal=fsal,
                            max_accepted=3, trace_cap=32)
         x = oh.HipState(exe, data=x0)
@@ -51,20 +52,21 @@ def test_mixed_attempts(exe, n, masses, tableau, fsal):
         assert res.accepted == 3
         assert np.array_equal(bits(res.x_final), bits(x.to_numpy()))
     finally:
-        exe.near_field = near
+        exe.near_field = keep
 
 
-@pytest.mark.parametrize("n,masses", [(4096, "spread"), (4097, "equal"), (8192, "unit"),
-                                      (8193, "unit")])
+@pytest.mark.parametrize("n,masses,near", [(8192, "spread", 0.0), (8193, "equal", 0.0),
+                                           (8193, "unit", 0.0), (16384, "spread", 20.0),
+                                           (16385, "equal", 20.0), (16385, "unit", 20.0)])
 @pytest.mark.parametrize("steps", [1, 2, 5])
-def test_mixed_leapfrog(exe, n, masses, steps):
+def test_mixed_leapfrog(exe, n, masses, near, steps):
     """Without output (one launch a step where the rule says so) and with it (three)."""
     import ode_prototyping_amd as oh
     x0, m = system(n, masses)
     ode = oh.NBodyODE(1e-2, m, "mixed")
-    near = exe.near_field
+    keep = exe.near_field
     try:
-        exe.near_field = 0.0
+        exe.near_field = near
         tf = (steps - 0.5) * 1e-3
         out = oh.RawOutput()
         a, st = oh.leapfrog(x0, 0.0, tf, 1e-3, ode, exe=exe)
@@ -72,4 +74,4 @@ def test_mixed_leapfrog(exe, n, masses, steps):
         assert st["steps"] == steps
         assert np.array_equal(bits(a), bits(b))
     finally:
-        exe.near_field = near
+        exe.near_field = keep
