@@ -58,6 +58,7 @@ struct EnsBufs {
   int wpb;         // waves per RHS workgroup
   int tpl2_min_n;  // systems with n >= this use 128-target tiles
   int split;       // > 1: waves sharing one tile's partners
+  int fine;        // ... in 16-target workgroups (fast and mixed without near field)
   double eps2;
   double near_c;  // mixed variant: pairs with FP32 r^2 < near_c / n in FP64
   const double* dense_t;  // DOPRI5 dense output: n_dense times, or null
@@ -90,9 +91,23 @@ constexpr int kEnsChunk = 128;
 // SIMDs of the device (256 CUs x 4): the waves one launch needs to give
 // each SIMD one.
 constexpr long kEnsSimds = 1024;
-// 64-target tiles up to which a shared tile of the fast and mixed sums is split
-// into 16-target workgroups.
+// 64-target tiles up to which a shared tile of the fast and mixed sums is split into
+// 16-target workgroups (k_ens_rhs_fine).  In a solve, where few of a list's systems
+// may still run, the largest sets a launch's time and the next stage's input is
+// formed behind the sums, that is the faster form up to 512 tiles.
 constexpr int kEnsFineTiles = 512;
+// A plain evaluation of every system takes it up to two workgroups a CU and one round
+// of partners (systems of 512 bodies, 128 tiles 11.5 us against 13.6 by eight waves a
+// tile, 160 tiles 14.8 against 14.0, 512 tiles 28.9 against 19.5; 512 tiles of 64
+// bodies 23.9 against 9.5; 64 tiles of 16 bodies 7.2 against 6.2, of 1024 16.0 against
+// 19.2, of 2000 44.9 against 33.9), and in place of two waves a tile wherever these
+// walk three chunks or more (256 tiles of 1000 bodies 24.6 against 34.8).
+constexpr int kEnsFinePlainTiles = 128;
+constexpr int kEnsFinePlainN = 1024;
+constexpr bool plain_fine(long tiles, long longest, int split) {
+  return (tiles <= kEnsFinePlainTiles && longest >= 64 && longest <= kEnsFinePlainN) ||
+         (tiles <= kEnsFineTiles && split == 2 && longest > 2 * kEnsChunk);
+}
 // Waves that give each of the 1024 SIMDs (256 CUs x 4) four, the depth that
 // hides the RHS arithmetic's latency.
 constexpr long kEnsFillWaves = 4096;

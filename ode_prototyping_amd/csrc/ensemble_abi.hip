@@ -169,7 +169,10 @@ EnsBufs make_bufs(EnsembleWorkspace* w, const Plan& p, const Layout& L,
   return b;
 }
 
-void set_tile_cfg(EnsBufs* b, int cfg, int n_tiles) {
+// `solve`: of a solve, or timed for one.
+void set_tile_cfg(EnsBufs* b, int cfg, int n_tiles, const Layout& L, bool solve) {
+  b->fine = solve ? n_tiles <= kEnsFineTiles
+                  : plain_fine(n_tiles, tail_shape(L, nullptr).longest, kEnsTileConfigs[cfg].split);
   b->wpb = kEnsTileConfigs[cfg].wpb;
   b->tpl2_min_n = kEnsTileConfigs[cfg].tpl2_min_n;
   b->split = kEnsTileConfigs[cfg].split;
@@ -207,7 +210,7 @@ int autotune(odehip_context* ctx, EnsembleWorkspace* w, const Plan& p,
     int n_tiles = 0;
     int rc = upload_tables(ctx, w, p, L, tiles_cap, c, &n_tiles, s);
     if (rc) return rc;
-    set_tile_cfg(&b, c, n_tiles);
+    set_tile_cfg(&b, c, n_tiles, L, true);
     HIP_TRY(ctx, ens_launch_rhs(b, y, k, 0, s));
     double ms_best = 1e300;
     for (int r = 0; r < 2; ++r) {
@@ -283,7 +286,7 @@ int odehip_ensemble_rhs(odehip_context* ctx, int n_systems,
   b.variant = nbody_variant;
   b.eps2 = eps2;
   b.near_c = near_c;
-  set_tile_cfg(&b, cfg, n_tiles);
+  set_tile_cfg(&b, cfg, n_tiles, L, false);
   HIP_TRY(ctx, hipEventRecord(w->t0, s));
   HIP_TRY(ctx, ens_launch_rhs(b, x, dxdt, 0, s));
   HIP_TRY(ctx, hipEventRecord(w->t1, s));
@@ -416,7 +419,7 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
   int run_cfg = tail_config(L, nullptr, cfg, exact);
   int n_tiles = 0;
   if ((rc = upload_tables(ctx, w, p, L, tcap, run_cfg, &n_tiles, s))) return rc;
-  set_tile_cfg(&b, run_cfg, n_tiles);
+  set_tile_cfg(&b, run_cfg, n_tiles, L, true);
 
   HIP_TRY(ctx, ens_enqueue_init(b, x0, opt->t0, opt->tf, opt->max_accepted,
                                 opt->max_attempts, opt->fsal ? 1 : 0, opt->controller, s));
@@ -554,7 +557,7 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
     w->tables.invalidate();  // the tile region now holds the running systems' tiles
     rb.groups = reinterpret_cast<const int2*>(w->dev + p.groups_act);
     rb.n_groups = static_cast<int>(act.size());
-    set_tile_cfg(&rb, run_cfg, static_cast<int>(tiles.size()));
+    set_tile_cfg(&rb, run_cfg, static_cast<int>(tiles.size()), L, true);
     K = rounds_per_replay(sum_n2);
     work = S * sum_n2;
     return capture(rb, K);

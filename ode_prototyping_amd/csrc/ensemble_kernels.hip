@@ -580,7 +580,7 @@ __global__ __launch_bounds__(64 * C) void k_ens_rhs_split(EnsBufs b,
 }
 
 // The reorderable variants when the running systems' 64-target tiles would not
-// fill the chip: a workgroup takes 16 of a tile's targets (blockIdx.y: which), a
+// fill the chip (EnsBufs::fine): a workgroup takes 16 of a tile's targets (blockIdx.y: which), a
 // lane one target and one of kFineSlots groups of partners at a time, so a
 // launch spreads over four times the CUs and a system's longest walk is a
 // quarter.  Partners go through LDS (the lanes of a wave read kFineSlots different
@@ -590,6 +590,7 @@ constexpr int kFineTargets = 16;
 constexpr int kFineSlots = 64 / kFineTargets;
 constexpr int kFineWaves = 8;
 constexpr int kFineGroups = kFineWaves * kFineSlots;     // groups per round
+static_assert(kEnsFinePlainN == kFineGroups * kEnsGroup, "one round of partners");
 constexpr int kFineStride = 3 * kEnsGroup + 2;           // doubles per group
 
 template <int kVariant, bool kMass, bool kSpecial>
@@ -929,7 +930,7 @@ hipError_t launch_rhs_v(const EnsBufs& b, const double* y, double* k,
       return hipGetLastError();
     } else {
       if constexpr (!kNear) {
-        if (b.n_tiles <= kEnsFineTiles) {
+        if (b.fine) {
           hipLaunchKernelGGL((k_ens_rhs_fine<kVariant, kMass, kSpecial>),
                              dim3(blocks, 64 / kFineTargets), dim3(64 * kFineWaves), 0, s, b, y, k,
                              stage0, next);
