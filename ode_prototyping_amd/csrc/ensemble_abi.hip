@@ -577,6 +577,7 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
   int compact_below = n_rounds * 7 / 8;
   auto next_lists = [&] { return launched + (work > kEnsListWork ? 0 : kEnsListRounds); };
   long compact_from = next_lists();
+  int seen = n_rounds;  // systems running at the last look
   std::vector<SolverState> hst;
   while (n_rounds > 0) {
     HIP_TRY(ctx, hipGraphLaunch(w->exec, s));
@@ -590,6 +591,13 @@ int odehip_ensemble_solve(odehip_context* ctx, int tableau, int n_systems,
       HIP_TRY(ctx, hipEventSynchronize(w->ev[slot ^ 1]));
       const int running = w->h_active[slot ^ 1];
       if (running == 0) break;
+      if (running <= compact_below && launched < compact_from && running < seen) {
+        // systems are ending: whether the last has is seen before another replay is
+        // launched, whose empty rounds would cost more than the wait
+        HIP_TRY(ctx, hipEventSynchronize(w->ev[slot]));
+        if (w->h_active[slot] == 0) break;
+      }
+      seen = running;
       if (running <= compact_below && launched >= compact_from) {
         HIP_TRY(ctx, hipStreamSynchronize(s));
         hst.resize(L.sys.size());
