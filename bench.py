@@ -43,14 +43,23 @@ sys.path.insert(0, ROOT)
 FP64_PEAK_TFLOPS = 78.6  # MI355X FP64 vector (and matrix) peak
 FLOP_PER_INTERACTION = 20
 # FP64 VALU wave-instructions per 64 directed interactions of the FP64 RHS
-# kernels (SQ_INSTS_VALU x 64 / N^2 at N=16384 with masses 1/N = 2^-14, which both kernels
-# take as unit-mass terms and one scale per sum;
-# profiles/nbody_rhs_n16384_valu_counters.txt) and how many of them are quarter-rate
-# transcendentals (v_rsq_f64, v_rcp_f64).  The exact entry is the count of the
-# kernel that profile was taken of; the present one needs 37 or so, one of them
-# quarter-rate, so the bound it gives is an upper one.
-VALU_PER_64_INTERACTIONS = {"exact": (38.38, 2), "fast": (17.18, 1)}
+# kernels with masses 1/N = 2^-14 (unit-mass terms and one scale per sum) and how
+# many of them are quarter-rate transcendentals (v_rsq_f64, v_rcp_f64).
+# k_exact_relay: its partner loop's instructions (30 of the term, the rsqrt, 3 adds);
+# the counters of profiles/nbody_rhs_n16384_valu_counters.txt (39.79) also hold the
+# waves' polls for their turn.  fast: SQ_INSTS_VALU x 64 / N^2 of the same profile at
+# N=16384.  exact: the counters of the tile kernel that k_exact_relay replaced, which no
+# result here uses.
+VALU_PER_64_INTERACTIONS = {"k_exact_relay": (34, 1), "fast": (17.18, 1), "exact": (38.38, 2)}
 SIMDS = 1024  # 256 CUs x 4 SIMDs
+
+
+def rhs_kernel(variant, n):
+    """The RHS kernel a launch of n bodies with masses takes on 256 CUs, where this file
+    knows it (the exact variant has a shape per size range)."""
+    if variant == "exact":
+        return "k_exact_relay" if 8192 < n <= 16384 else None
+    return f"k_nbody_{variant}"
 
 
 def instruction_bound(variant, n, clock_mhz, kernel_ms):
@@ -65,8 +74,9 @@ def instruction_bound(variant, n, clock_mhz, kernel_ms):
     return {"valu_per_64_interactions": total, "quarter_rate": quarter,
             "cycles_per_64_interactions": cycles, "bound_ms": bound_ms,
             "frac": bound_ms / kernel_ms,
-            "source": "SQ_INSTS_VALU per interaction from the committed counter profile; "
-                      "4 cycles per FP64 wave64 instruction, 16 for v_rsq_f64 / v_rcp_f64"}
+            "source": "FP64 instructions of the partner loop (k_exact_relay) or SQ_INSTS_VALU "
+                      "per interaction from the committed counter profile; 4 cycles per FP64 "
+                      "wave64 instruction, 16 for v_rsq_f64 / v_rcp_f64"}
 
 
 def log(msg):
@@ -795,6 +805,7 @@ def main():
     sus_tflops, sus_mhz = exe.probe_fp64()
     log(f"sustained FP64 FMA: {sus_tflops:.1f} TFLOP/s at {sus_mhz:.0f} MHz")
     traffic = None
+    kernel = rhs_kernel(args.variant, n)
     tfile = os.path.join(ROOT, "profiles", f"nbody_rhs_n{n}_traffic.json")
     if os.path.exists(tfile):
         tk = json.load(open(tfile))["kernels"].get(args.variant)
@@ -824,7 +835,7 @@ def main():
         "rejected": r.rejected,
         "ms_per_step_events": ev_ms / steps,
         "roofline": {"bound": "valu", "pipe": "FP64 vector ALU (no dense contraction)",
-                     "kernel": "k_exact_relay" if args.variant == "exact" else f"k_nbody_{args.variant}",
+                     "kernel": kernel or f"{args.variant} RHS",
                      "achieved": achieved,
                      "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / FP64_PEAK_TFLOPS, "traffic": traffic,
@@ -834,7 +845,8 @@ def main():
                      "kernel_ms_isolated": iso_ms,
                      "sustained_fp64_tflops": sus_tflops, "clock_mhz": sus_mhz,
                      "frac_of_sustained": achieved / sus_tflops,
-                     "instruction_bound": instruction_bound(args.variant, n, sus_mhz, rhs_ms),
+                     "instruction_bound": instruction_bound(
+                         kernel if args.variant == "exact" else args.variant, n, sus_mhz, rhs_ms),
                      "algorithmic": f"{FLOP_PER_INTERACTION} FLOP x N(N-1) = "
                                     f"{FLOP_PER_INTERACTION * interactions:.4g} FLOP/launch"},
     }
