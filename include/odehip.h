@@ -49,7 +49,10 @@ extern "C" {
 #define ODEHIP_NBODY_EXACT 0 /* the reference's FP64 expression, correctly
                                 rounded sqrt and divisions, partners summed
                                 in increasing index: bit-identical to
-                                NBodyODE with SingleThreadedExecutor */
+                                NBodyODE with SingleThreadedExecutor (but
+                                for fewer than 2^11 of the 2^104 pairs of
+                                significands, whose quotient may round to the
+                                other neighbour) */
 #define ODEHIP_NBODY_FAST 1  /* FP64 with a refined hardware rsqrt and
                                 parallel partial sums (~1 ulp per term) */
 #define ODEHIP_NBODY_MIXED 2 /* displacement rounded to FP32, pair force in
@@ -418,14 +421,18 @@ int odehip_mlp_infer(odehip_context* ctx, const odehip_mlp* mlp,
  * RKEmbeddedParallel.hpp:13-81; this is that call for every system at once).
  * States are packed: system k occupies 6 n_k doubles [pos | vel] starting at
  * 6 * (n_0 + ... + n_{k-1}); masses (optional) are packed the same way with
- * n_k entries per system.  Each system's result is bit-identical to
- * odehip_rk_solve on that system alone with the same options (same right-hand
- * side variant, FSAL setting and controller).
+ * n_k entries per system.  Each system's result is bit-identical to a solve
+ * of that system alone by this call, whatever other systems are in it, and with
+ * the exact variant to odehip_rk_solve with the same options (same FSAL setting
+ * and controller); the fast and mixed variants add their terms in another order
+ * there.
  *
  * The attempt of every active system advances in lockstep rounds: one
- * launch per stage covers all systems, a round ends with a controller pass
- * (one thread per system), and K rounds are captured in a HIP graph that is
- * replayed until every system has finished.  The right-hand side runs one
+ * launch per stage covers all systems, a round ends with a pass whose last
+ * workgroup of each system runs its controller, and K rounds are captured in a
+ * HIP graph that is replayed until every system has finished; small systems are
+ * solved by one workgroup each beside the rounds, with the same bits.  The
+ * right-hand side runs one
  * wavefront per tile of 64 (or 128) target particles; which systems use
  * 128-target tiles, the waves per workgroup and the XCD placement of tiles
  * are chosen by an autotuner that times the candidates on the ensemble and,

@@ -259,7 +259,8 @@ class NBodyODE:
 
     ``masses``: None for unit masses (the reference), else a length-N array
     (held on the device).  ``variant``: "exact" (bit-identical to the
-    reference's single-threaded evaluation), "fast" (FP64, refined rsqrt) or
+    reference's single-threaded evaluation, but for fewer than 2^11 of the 2^104
+    pairs of significands a quotient can have), "fast" (FP64, refined rsqrt) or
     "mixed" (FP32 pair force, FP64 accumulation; near pairs in FP64 when the
     executor's ``near_field`` is set).
     """

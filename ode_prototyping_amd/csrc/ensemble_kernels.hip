@@ -795,9 +795,9 @@ __global__ __launch_bounds__(kBlock) void k_ens_final(EnsBufs b) {
 
 // Dense output of every system whose attempt of this round was accepted and
 // covered an output time (StepperDopr5 / StepperDopr853 prepare_dense,
-// dense_out and DenseOutput::save, as the single-system pass): the gate, one
-// thread per system; for DOP853 f at the new state and the three extra
-// stages, evaluated for those systems only; then the rows, one workgroup per
+// dense_out and DenseOutput::save, as the single-system pass; the gate is the
+// final pass's): for DOP853 f at the new state and the three extra stages,
+// evaluated for those systems only; then the rows, one workgroup per
 // reduction group.  A system that finished in this round still writes its
 // last step's rows.
 __global__ __launch_bounds__(kBlock) void k_ens_dense_stage8(EnsBufs b, int x) {

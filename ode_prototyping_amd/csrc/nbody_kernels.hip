@@ -15,7 +15,8 @@
 //            rounded divisions) and, per target, the partners summed in
 //            increasing j -- the order the single-threaded pair loop adds into
 //            acc[i] (nbody_exact.hpp).  Result: bit-identical to NBodyODE with
-//            SingleThreadedExecutor.  Must be compiled with -ffp-contract=off.
+//            SingleThreadedExecutor, but for the few quotients that
+//            nbody_terms.hpp names.  Must be compiled with -ffp-contract=off.
 //  * fast:   FP64, r^-3 from the hardware reciprocal square root with a
 //            third-order correction (a few ulp), FMA accumulation, the j range
 //            split over 16 waves per workgroup and the partial sums combined
@@ -152,7 +153,7 @@ constexpr int kFastWaves = 16;
 // Two 16-wave workgroups share a CU only while a wave's SGPRs fit eighty: the
 // SIMD's 800 hold eight waves of 80 and the 16 the trap handler keeps per wave.
 // (With 88, which the compiler counts as eight waves too, 65536 bodies took 2584
-// instead of 2391 us, and the mixed kernel 1789 instead of 1430.)
+// instead of 2391 us.)
 #define ODEHIP_EIGHT_WAVES_SGPRS __attribute__((amdgpu_num_sgpr(80)))
 
 // kFastSet partners' coordinates (and masses), wave-uniform in SGPRs.
@@ -575,9 +576,10 @@ __device__ __forceinline__ void mixed_body(const NBodyArgs& a) {
 }
 
 // Held to eighty SGPRs, the loop over unequal masses spills (16384 bodies with near
-// field 157 instead of 151 us), and only launches that form the next stage's input
-// in more than one workgroup a CU need the limit: those without masses, the others
-// leave it to a launch of its own there (nbody_rhs_forms_next).
+// field 157 instead of 151 us).  Only launches that form the next stage's input in
+// more than one workgroup a CU gain by the limit; with masses they leave that to a
+// launch of its own (nbody_rhs_forms_next), without them they keep it (leapfrog, 20
+// steps at 65536 bodies, 37.6 instead of 38.3 ms).
 template <bool kMass, bool kGuard, bool kNear, bool kNext>
 __global__ __launch_bounds__(64 * kMixedWaves) void k_nbody_mixed(NBodyArgs a) {
   mixed_body<kMass, kGuard, kNear, kNext>(a);

@@ -54,7 +54,7 @@ __device__ inline void exact_term_ieee(double dx, double dy, double dz,
 //    error, far below the rounding of r.  Three instructions in the place of
 //    v_rcp_f64 (four times the cost of one) and a Newton step: 33 full-rate
 //    instructions and one transcendental per term instead of 32 and two,
-//    about 7 % of the arithmetic, with the same bits.
+//    about 7 % of the arithmetic, with the same bits but for those pairs.
 template <bool kMass>
 __device__ inline void exact_term_shared_rcp(double dx, double dy, double dz,
                                              double mj, double softening_sq,

@@ -3,13 +3,15 @@
 // the device-resident solve driver.
 //
 // The solve driver replaces the host loop of RKEmbeddedParallel::integrate
-// (RKEmbeddedParallel.hpp:35-80).  The attempt's kernels (S right-hand sides,
-// S-1 stage combinations, the fused final/error/norm pass and the controller)
-// are captured once into a HIP graph holding K attempts; the graph is
-// replayed until the device-side controller raises `done`.  Every kernel of a
-// finished solve returns at once, so over-enqueueing is harmless.  The host
-// only polls the done flag of the previous replay (one replay in flight), so
-// the device never waits on the host between attempts.
+// (RKEmbeddedParallel.hpp:35-80).  The attempt's kernels (S right-hand sides, each
+// of which forms the next stage's input, and the fused final/error/norm pass,
+// whose last workgroup runs the controller) are captured once into a HIP graph
+// holding K attempts; the graph is replayed until the device-side controller
+// raises `done`.  Every kernel of a finished solve returns at once, the dense
+// output's too, so over-enqueueing costs launches only.  The host only polls the
+// done flag of the previous replay (one replay in flight), so the device never
+// waits on the host between attempts.  Small N-body systems whose attempts
+// nothing names or looks into run whole in one workgroup (solo_kernels.hip).
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -707,7 +709,7 @@ int odehip_rk_solve(odehip_context* ctx, int tableau, const odehip_ode* ode,
   HIP_TRY(ctx, enqueue_initial_step(b, s));
 
   // Small systems: whole attempts by one workgroup (solo.hpp), unless the
-  // caller says how the attempts are launched or every state is kept.
+  // caller says how the attempts are launched or asks for states or dense output.
   const bool solo = ode->rhs_kind == ODEHIP_RHS_NBODY && opt->attempts_per_launch == 0 &&
                     n_dense == 0 && states_cap == 0 &&
                     b.n_particles <= solo_one_limit(S, ode->nbody_variant, b.mlp != nullptr);

@@ -231,7 +231,7 @@ __global__ void k_init_step_b(SolverState* st, const double* pa, size_t n_var) {
 
 // RawOutput::save_state of an accepted step (RawOutput.hpp:15-19): the new
 // x0 into slot `accepted` of the device state list.  Runs after every
-// controller launch; once a solve is done it rewrites the same slot with the
+// final pass; once a solve is done it rewrites the same slot with the
 // same state (harmless).
 __global__ void k_save_state(const SolverState* st, const double* xb0,
                              const double* xb1, double* states, long cap,

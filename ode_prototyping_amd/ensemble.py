@@ -5,8 +5,9 @@ call (``src/integrator/RKEmbeddedParallel/RKEmbeddedParallel.hpp:13-81``) with
 ``NBodyODE`` (``src/ode/NBodyODE.hpp``).  :func:`solve_ensemble` makes that
 call for many systems of different sizes at once: every system keeps its own
 step size, accept/reject sequence, counters and end condition, and its result
-is bit-identical to :func:`ode_prototyping_amd.integrate` on that system alone
-with the same options.
+does not depend on the other systems by a bit; with the exact variant it is
+bit-identical to :func:`ode_prototyping_amd.integrate` on that system with the
+same options (fast and mixed add their terms in another order there).
 
 States are packed: system k occupies ``6 n_k`` doubles ``[pos | vel]``
 starting at ``6 (n_0 + ... + n_{k-1})``; masses (optional) likewise with
